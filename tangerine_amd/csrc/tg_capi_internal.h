@@ -45,6 +45,7 @@ struct PruneState
 {
 	bool pending = false;        // a pass was issued; its counters are not read yet
 	bool level_parallel = false;
+	bool words = false;          // one word per entry (PruneArgs::words)
 	uint64_t ncells = 0, waves = 0, capacity = 0;
 	uint32_t cells_per_wave = 0;
 	float decide_radius = 0.0f;
@@ -86,14 +87,20 @@ struct CellPrograms
 	}
 };
 
+// With `words` the cells' programs are one word per entry; the result is only
+// valid where the level-parallel passes apply.
 int prune_cells(hipStream_t stream, const tg_program* p, const float origin[3], const float cell[3], float radius,
 	const uint32_t counts[3], bool fast, CellPrograms& out);
+
+// Whether `p` can be pruned over ncells cells by the level-parallel passes.
+bool level_prunable(const tg_program* p, uint64_t ncells);
 
 // A cell grid to prune a program over.
 struct CellGrid
 {
 	float origin[3], cell[3], radius;
 	uint32_t counts[3];
+	bool words = false;
 };
 
 // Job tables of prune_cells_many (kept between calls: the upload reads `host`).
@@ -114,7 +121,7 @@ int prune_cells_many(hipStream_t stream, const tg_program* const* progs, const C
 // fills the counts (same arguments).  Between them the caller may issue other
 // work (other trees' pruning on other streams).
 int prune_cells_start(hipStream_t stream, const tg_program* p, const float origin[3], const float cell[3],
-	float radius, const uint32_t counts[3], bool fast, CellPrograms& out);
+	float radius, const uint32_t counts[3], bool fast, CellPrograms& out, bool words = false);
 int prune_cells_finish(hipStream_t stream, const tg_program* p, const float origin[3], const float cell[3],
 	const uint32_t counts[3], bool fast, CellPrograms& out);
 }

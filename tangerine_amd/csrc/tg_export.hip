@@ -62,6 +62,9 @@ struct tg_mesher
 	// near-surface tiles run deeper programs, which want more spill room per
 	// wave than the plain export's tuning may leave
 	int culled_points_per_lane = 4, culled_waves = 4, culled_workgroups_per_cu = 6;
+	// tg_mesher_set_tuning / set_emission were called: exports then evaluate by
+	// blocks, whatever the grid (see tile_programs)
+	bool by_blocks = false;
 	int cus = 0;                  // compute units of the device
 	DevBuf persist_args, persist_head, persist_tables;  // the persistent launch's argument copy, queue head, tables
 	DevBuf order_keys, order_values, order, order_tmp;   // its queue: blocks by program cost
@@ -427,6 +430,65 @@ int prune_blocks(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t f
 	return prune_blocks_finish(m, p, g, flags);
 }
 
+// Grids whose tiles x program entries stay below this are pruned per 8^3
+// tile in grid-wide passes and evaluated a wave per tile, without blocks.  The
+// passes evaluate every entry at every tile's centre, so their cost grows with
+// this product; the block evaluators' per-block prologue, run by one wave,
+// costs a latency that few blocks cannot hide.
+constexpr uint64_t kTileEntryCells = 150ull << 20;
+
+bool tile_programs(const tg_program* p, const MeshArgs& ma)
+{
+	const uint64_t tiles = uint64_t(ma.tx) * ma.ty * ma.tz;
+	return tiles * p->decoded.entries.size() <= kTileEntryCells && level_prunable(p, tiles);
+}
+
+// The 8^3-sample tiles as cells (samples lie within 3.5 |d| of a tile's centre).
+BlockGrid tile_grid(const tg_mesher* m, const tg_grid* g)
+{
+	const MeshArgs& ma = m->args;
+	BlockGrid b{};
+	b.counts[0] = ma.tx; b.counts[1] = ma.ty; b.counts[2] = ma.tz;
+	b.origin[0] = g->x - 0.5f * g->dx; b.origin[1] = g->y - 0.5f * g->dy; b.origin[2] = g->z - 0.5f * g->dz;
+	b.cell[0] = float(kTile) * g->dx; b.cell[1] = float(kTile) * g->dy; b.cell[2] = float(kTile) * g->dz;
+	b.radius = 0.5f * float(kTile - 1) * std::sqrt(g->dx * g->dx + g->dy * g->dy + g->dz * g->dz);
+	return b;
+}
+
+// Points per lane of the tile evaluation: fewer, and so more waves to a tile,
+// while the waves do not fill the GPU and each wave's time is its program's
+// latency (64^3 cells, 497 primitives: 0.49 ms at 4 points, 0.15 ms at one).
+uint32_t tile_points(uint64_t tiles)
+{
+	uint32_t pts = 4;
+	while (pts > 1 && tiles * (kTile / pts) < 8192) pts >>= 1;
+	return pts;
+}
+
+// Tile-program evaluation of one grid (m->blocks pruned per tile).
+TileEvalArgs tile_args(tg_mesher* m, const tg_program* p, const tg_grid* g, unsigned long long* work)
+{
+	const MeshArgs& ma = m->args;
+	TileEvalArgs ta{};
+	ta.prog = static_cast<const Instr*>(p->device.ptr);
+	ta.words = m->blocks.pool.as<const uint32_t>();
+	ta.desc = m->blocks.desc.as<const BlockDesc>();
+	ta.whole = p->entries.as<const Entry>();
+	ta.n_whole = uint32_t(p->decoded.entries.size());
+	ta.gx = g->x; ta.gy = g->y; ta.gz = g->z;
+	ta.dx = g->dx; ta.dy = g->dy; ta.dz = g->dz;
+	ta.nx = ma.nx; ta.ny = ma.ny; ta.nz = ma.nz;
+	ta.tx = ma.tx; ta.ty = ma.ty; ta.tz = ma.tz;
+	ta.ntiles = uint32_t(m->blocks.ncells);
+	ta.out_pool = m->pool.as<float>();
+	ta.signs = m->signs.as<uint8_t>();
+	ta.points = tile_points(ta.ntiles);
+	// 5 KiB a wave: 32 waves fill a CU's LDS, the most it holds
+	ta.slots = block_spill_slots(std::max<uint32_t>(1, p->decoded.max_stack), int(ta.points), 5120);
+	ta.work = work;
+	return ta;
+}
+
 // Largest |p| over the grid's samples (the corners of its box).
 float grid_reach(const tg_grid* g)
 {
@@ -597,6 +659,30 @@ int eval_blocks(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t fl
 	hipError_t e = (flags & TG_FLAG_FAST) ? fast::launch_eval_blocks(ba, pts, m->stream)
 	                                      : exact::launch_eval_blocks(ba, pts, m->stream);
 	if (e != hipSuccess) return hip_fail(e, "block evaluation launch");
+	TG_CHECK_HIP(hipEventRecord(m->ev[5], m->stream), "event");
+	TG_CHECK_HIP(hipMemcpyAsync(work_readback(m), work, 16, hipMemcpyDeviceToHost, m->stream), "work read");
+	return TG_OK;
+}
+
+// Evaluation of every tile from its own program (m->blocks pruned per tile).
+// Asynchronous, read as eval_blocks is.
+int eval_tile_programs(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t flags)
+{
+	int rc = m->counters.ensure(64);
+	if (rc) return rc;
+	unsigned long long* work = m->counters.as<unsigned long long>();
+	TG_CHECK_HIP(hipMemsetAsync(m->counters.ptr, 0, 64, m->stream), "counter reset");
+	const TileEvalArgs ta = tile_args(m, p, g, work);
+	m->last_points_per_lane = int(ta.points);
+	m->last_waves = int(kTileEvalWaves);
+	m->last_workgroups = 0;
+	m->last_max_len = m->blocks.max_len;
+	m->last_max_binary = m->blocks.max_binary;
+	m->last_lds = uint32_t(spill_bytes_per_wave(ta.slots, int(ta.points)) * kTileEvalWaves);
+	TG_CHECK_HIP(hipEventRecord(m->ev[4], m->stream), "event");
+	const hipError_t e = (flags & TG_FLAG_FAST) ? fast::launch_eval_tile_programs(ta, m->stream)
+	                                            : exact::launch_eval_tile_programs(ta, m->stream);
+	if (e != hipSuccess) return hip_fail(e, "tile evaluation launch");
 	TG_CHECK_HIP(hipEventRecord(m->ev[5], m->stream), "event");
 	TG_CHECK_HIP(hipMemcpyAsync(work_readback(m), work, 16, hipMemcpyDeviceToHost, m->stream), "work read");
 	return TG_OK;
@@ -814,7 +900,17 @@ int run_export(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t fla
 	TG_CHECK_HIP(hipEventRecord(m->ev[0], m->stream), "event");
 	m->blocks.valid = false;
 	bool sorted = false;
-	if (!(flags & TG_FLAG_NO_PRUNE) && p->decoded.prunable())
+	const bool by_tiles = !culled && !m->by_blocks && !(flags & TG_FLAG_NO_PRUNE) && tile_programs(p, ma);
+	if (by_tiles)
+	{
+		const BlockGrid t = tile_grid(m, g);
+		rc = prune_cells_start(m->stream, p, t.origin, t.cell, t.radius, t.counts, (flags & TG_FLAG_FAST) != 0, m->blocks,
+			true);
+		if (!rc)
+			rc = prune_cells_finish(m->stream, p, t.origin, t.cell, t.counts, (flags & TG_FLAG_FAST) != 0, m->blocks);
+		if (rc) return rc;
+	}
+	else if (!(flags & TG_FLAG_NO_PRUNE) && p->decoded.prunable())
 	{
 		rc = prune_blocks_start(m, p, g, flags);
 		if (rc) return rc;
@@ -841,7 +937,12 @@ int run_export(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t fla
 	TG_CHECK_HIP(hipEventRecord(m->ev[3], m->stream), "event");
 	uint64_t evals = 0;
 	double flops = 0.0;
-	if (blocks)
+	if (by_tiles)
+	{
+		rc = eval_tile_programs(m, p, g, flags);
+		if (rc) return rc;
+	}
+	else if (blocks)
 	{
 		rc = culled ? eval_blocks(m, p, g, flags, m->tile_mask.as<const uint64_t>(), m->block_list.as<const uint32_t>(),
 		                          sel.listed)
@@ -871,6 +972,7 @@ int run_export(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t fla
 	{
 		rc = eval_blocks_read(m, &evals, &flops);
 		if (rc) return rc;
+		if (by_tiles) evals = uint64_t(ga.ntiles) * kTileSamples;
 	}
 	float t_pre = 0, t_eval = 0, t_mesh = 0, t_all = 0;
 	TG_CHECK_HIP(hipEventElapsedTime(&t_pre, m->ev[0], m->ev[3]), "timing");
@@ -968,6 +1070,7 @@ extern "C" int tg_mesher_set_tuning(tg_mesher* m, uint32_t points_per_lane, uint
 	m->waves = int(waves);
 	m->workgroups_per_cu = int(workgroups_per_cu);
 	m->min_prune_len = min_prune_len;
+	m->by_blocks = true;
 	return TG_OK;
 }
 
@@ -977,6 +1080,7 @@ extern "C" int tg_mesher_set_emission(tg_mesher* m, uint32_t mode)
 	if (mode > 2) return fail(TG_ERR_INVALID, "tg_mesher_set_emission: mode 0 (automatic), 1 (walk) or 2 (per block)");
 	if (int rc = refuse_batch_owned(m, "tg_mesher_set_emission")) return rc;
 	m->blocks.emission = int(mode);
+	m->by_blocks = true;
 	return TG_OK;
 }
 
@@ -1775,6 +1879,13 @@ struct tg_batch
 	std::vector<tg_grid> grids;
 	DevBuf trees, items, head, work;
 	DevBuf tables;                // per-workgroup decision tables and tile pools
+	// trees evaluated from tile programs (tile_programs): one launch beside the
+	// queue's, its jobs and their first workgroups
+	std::vector<uint8_t> by_tiles;
+	DevBuf tile_jobs;
+	uint32_t tile_njobs = 0, tile_blocks = 0;
+	size_t tile_lds = 0;          // per wave
+	bool by_blocks = false;       // tg_batch_set_tuning was called: every tree by blocks
 	PruneLaunches prune;          // every tree's level pruning and emission as shared launches
 	DevBuf queue_sort;            // the queue's keys, values, tree offsets and sort storage
 	hipGraph_t graph = nullptr;
@@ -1838,6 +1949,14 @@ int capture_batch(tg_batch* b)
 		                                 uint32_t(b->last_workgroups), b->stream)
 		            : exact::launch_batch(b->args, b->last_points_per_lane, uint32_t(b->last_waves),
 		                                  uint32_t(b->last_workgroups), b->stream);
+	if (e == hipSuccess && b->tile_njobs)
+	{
+		const TileEvalArgs* jobs = b->tile_jobs.as<const TileEvalArgs>();
+		const uint32_t* base = reinterpret_cast<const uint32_t*>(jobs + b->tile_njobs);
+		e = b->fast
+			? fast::launch_eval_tile_programs_multi(jobs, base, b->tile_njobs, b->tile_blocks, b->tile_lds, b->stream)
+			: exact::launch_eval_tile_programs_multi(jobs, base, b->tile_njobs, b->tile_blocks, b->tile_lds, b->stream);
+	}
 	hipGraph_t g = nullptr;
 	const hipError_t ee = hipStreamEndCapture(b->stream, &g);
 	if (e != hipSuccess)
@@ -1889,7 +2008,7 @@ extern "C" void tg_batch_destroy(tg_batch* b)
 	if (b->stream) (void)hipStreamSynchronize(b->stream);
 	drop_graph(b);
 	for (tg_mesher* m : b->meshers) destroy_mesher(m);
-	for (DevBuf* d : { &b->trees, &b->items, &b->head, &b->work, &b->tables, &b->prune.dev, &b->queue_sort })
+	for (DevBuf* d : { &b->trees, &b->items, &b->head, &b->work, &b->tables, &b->prune.dev, &b->queue_sort, &b->tile_jobs })
 		d->release();
 	for (hipEvent_t e : b->ev)
 		if (e) (void)hipEventDestroy(e);
@@ -1905,6 +2024,7 @@ extern "C" int tg_batch_set_tuning(tg_batch* b, uint32_t points_per_lane, uint32
 	b->points_per_lane = int(points_per_lane);
 	b->waves = int(waves);
 	b->workgroups_per_cu = int(workgroups_per_cu);
+	b->by_blocks = true;
 	if (b->exec) return capture_batch(b);
 	return TG_OK;
 }
@@ -1941,6 +2061,7 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 	}
 	b->programs.assign(programs, programs + count);
 	b->grids.assign(grids, grids + count);
+	b->by_tiles.assign(count, 0);
 	auto t0 = std::chrono::steady_clock::now();
 	int rc = b->work.ensure(size_t(count) * 16);
 	if (!rc) rc = b->head.ensure(256);
@@ -1962,8 +2083,10 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 		m->nbricks = 0;
 		rc = layout(m, &grids[i]);
 		if (rc) return rc;
-		const BlockGrid bg = block_grid(m, &grids[i]);
+		b->by_tiles[i] = !b->by_blocks && tile_programs(programs[i], m->args) ? 1 : 0;
+		const BlockGrid bg = b->by_tiles[i] ? tile_grid(m, &grids[i]) : block_grid(m, &grids[i]);
 		CellGrid& cg = cgs[i];
+		cg.words = b->by_tiles[i] != 0;
 		for (int k = 0; k < 3; ++k)
 		{
 			cg.origin[k] = bg.origin[k];
@@ -1973,6 +2096,11 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 		cg.radius = bg.radius;
 		outs[i] = &m->blocks;
 	}
+	std::vector<TileEvalArgs> tile_jobs;
+	std::vector<uint32_t> tile_base;
+	uint64_t tiles = 0;
+	b->tile_njobs = b->tile_blocks = 0;
+	b->tile_lds = 0;
 	rc = prune_cells_many(b->stream, programs, cgs.data(), count, fast, outs.data(), b->prune);
 	if (rc) return rc;
 	for (uint32_t i = 0; i < count; ++i)
@@ -1981,11 +2109,42 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 		rc = prune_cells_finish(b->stream, programs[i], cgs[i].origin, cgs[i].cell, cgs[i].counts, fast, m->blocks);
 		if (rc) return rc;
 		if (!m->blocks.valid) return fail(TG_ERR_LIMIT, "tg_batch_export: a tree could not be pruned");
-		args[i] = block_args(m, programs[i], &grids[i], nullptr, nullptr, 0, b->work.as<unsigned long long>() + 2 * i);
+		samples += uint64_t(m->args.nx) * m->args.ny * m->args.nz;
+		unsigned long long* work = b->work.as<unsigned long long>() + 2 * i;
+		if (b->by_tiles[i])
+		{
+			args[i].nblocks = 0;  // no queue items
+			const TileEvalArgs ta = tile_args(m, programs[i], &grids[i], work);
+			tile_jobs.push_back(ta);
+			b->tile_lds = std::max(b->tile_lds, spill_bytes_per_wave(ta.slots, int(ta.points)));
+			tiles += ta.ntiles;
+			continue;
+		}
+		args[i] = block_args(m, programs[i], &grids[i], nullptr, nullptr, 0, work);
 		ba.max_depth = std::max(ba.max_depth, args[i].max_depth);
 		ba.max_binary = std::max(ba.max_binary, args[i].max_binary);
 		ba.max_len = std::max(ba.max_len, args[i].max_len);
-		samples += uint64_t(m->args.nx) * m->args.ny * m->args.nz;
+	}
+	b->tile_njobs = uint32_t(tile_jobs.size());
+	if (b->tile_njobs)
+	{
+		// the jobs with the longest programs first (a wave's time is its
+		// program's length), then their first workgroups
+		std::stable_sort(tile_jobs.begin(), tile_jobs.end(), [](const TileEvalArgs& x, const TileEvalArgs& y) {
+			return x.points != y.points ? x.points < y.points : uint64_t(x.n_whole) * y.ntiles > uint64_t(y.n_whole) * x.ntiles;
+		});
+		for (const TileEvalArgs& ta : tile_jobs)
+		{
+			tile_base.push_back(b->tile_blocks);
+			b->tile_blocks += tile_eval_blocks(ta);
+		}
+		const size_t jb = tile_jobs.size() * sizeof(TileEvalArgs);
+		std::vector<uint8_t> blob(jb + tile_base.size() * 4);
+		std::memcpy(blob.data(), tile_jobs.data(), jb);
+		std::memcpy(blob.data() + jb, tile_base.data(), tile_base.size() * 4);
+		rc = b->tile_jobs.ensure(blob.size());
+		if (rc) return rc;
+		TG_CHECK_HIP(hipMemcpy(b->tile_jobs.ptr, blob.data(), blob.size(), hipMemcpyHostToDevice), "tile job upload");
 	}
 	// 2. the queue, sorted on the device: every tree's blocks, the most
 	// expensive block program first
@@ -2031,6 +2190,8 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 	if (rc) return rc;
 	std::vector<unsigned long long> wk(2 * size_t(count));
 	TG_CHECK_HIP(hipMemcpy(wk.data(), b->work.ptr, wk.size() * 8, hipMemcpyDeviceToHost), "work read");
+	for (uint32_t i = 0; i < count; ++i)
+		if (b->by_tiles[i]) wk[2 * i] = uint64_t(b->meshers[i]->blocks.ncells) * kTileSamples;
 	auto t2 = std::chrono::steady_clock::now();
 	double mesh_ms = 0;
 	uint64_t evals = 0;
@@ -2097,7 +2258,7 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 	st.mesh_ms = mesh_ms;
 	st.total_ms = std::chrono::duration<double, std::milli>(t3 - t0).count();
 	st.trees = count;
-	st.blocks = b->args.total;
+	st.blocks = b->args.total + tiles;
 	st.samples = samples;
 	st.exact_evals = evals;
 	st.flops = flops;

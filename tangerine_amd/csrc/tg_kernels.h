@@ -101,7 +101,11 @@ struct PruneArgs
 	const uint32_t* counts;   // with masks_ready: program length per lane, [group][64]
 	uint32_t splits;          // with masks_ready: waves per cell group (1, 2 or 4), each emitting 64 / splits columns
 	int columns;              // with masks_ready: a wave per cell, a lane per entry (k_prune_columns)
+	int words;                // with columns: one word per entry (its `rec`), `pool` then holds uint32_t
+	uint32_t emit_waves;      // with columns: waves per workgroup (at most kEmitWaves)
+	uint32_t emit_cells;      // with columns: cells one wave emits (emit_waves * emit_cells <= 64)
 };
+constexpr uint32_t kEmitWaves = 16;
 
 // Level-parallel decision pass: one launch per entry height (leaves 0, a
 // parent one above its highest child); wave = (entry of the level, cell
@@ -156,6 +160,27 @@ struct BlockEvalArgs
 	int waves;                   // waves per workgroup
 	float slack;                 // rounding slack of the per-tile pruning decisions (rounding_slack)
 };
+
+// Evaluation from one program per 8^3-sample tile (PruneArgs::words), no
+// pruning left to do: 8 / points waves per tile, each `points` z-slices.
+struct TileEvalArgs
+{
+	const Instr* prog;
+	const uint32_t* words;       // the tiles' programs, one word per entry
+	const BlockDesc* desc;       // one per tile
+	const Entry* whole;          // whole program, for tiles left with it
+	uint32_t n_whole;
+	float gx, gy, gz, dx, dy, dz;
+	uint32_t nx, ny, nz;
+	uint32_t tx, ty, tz;
+	uint32_t ntiles;
+	uint32_t points;             // points per lane: 1, 2 or 4
+	float* out_pool;
+	uint8_t* signs;              // 64 bytes per tile id (see GridArgs)
+	uint32_t slots;              // LDS spill slots per wave, each P floats per lane
+	unsigned long long* work;    // [1] cost units over the grid's samples
+};
+constexpr uint32_t kTileEvalWaves = 4;  // waves per workgroup
 
 // Persistent batched evaluation of many trees' blocks (one queue item = one
 // block of one tree).
@@ -335,9 +360,14 @@ hipError_t launch_prune_level_multi(const LevelArgs* jobs, const uint32_t* wave_
 // many programs' emissions in one launch: job k owns blocks [block_base[k], ...) of `blocks`
 hipError_t launch_prune_cells_multi(const PruneArgs* jobs, const uint32_t* block_base, uint32_t njobs, uint32_t blocks,
 	uint32_t max_slots, hipStream_t s);
-// the same a wave per cell (PruneArgs::columns): job k owns cells [cell_base[k], ...) of `cells`
-hipError_t launch_prune_columns_multi(const PruneArgs* jobs, const uint32_t* cell_base, uint32_t njobs, uint32_t cells,
-	uint32_t max_entries, hipStream_t s);
+// the same a wave per cell (PruneArgs::columns): job k owns workgroups [block_base[k], ...) of `blocks`
+// (prune_column_blocks of each); max_entries: over the jobs that emit whole entries
+hipError_t launch_prune_columns_multi(const PruneArgs* jobs, const uint32_t* block_base, uint32_t njobs, uint32_t blocks,
+	uint32_t max_waves, uint32_t max_entries, hipStream_t s);
+hipError_t launch_eval_tile_programs(const TileEvalArgs& a, hipStream_t s);
+// many grids in one launch: job k owns workgroups [block_base[k], ...) of `blocks` (tile_eval_blocks of each)
+hipError_t launch_eval_tile_programs_multi(const TileEvalArgs* jobs, const uint32_t* block_base, uint32_t njobs,
+	uint32_t blocks, size_t lds_per_wave, hipStream_t s);
 hipError_t launch_vox(const VoxArgs& a, int stage, hipStream_t s);  // 0 select, 1 list
 hipError_t launch_pivot(const PivotArgs& a, hipStream_t s);
 hipError_t launch_cloud(const CloudArgs& a, int stage, hipStream_t s);  // 0 select, 1 points, 2 refine
@@ -364,9 +394,14 @@ hipError_t launch_prune_level_multi(const LevelArgs* jobs, const uint32_t* wave_
 // many programs' emissions in one launch: job k owns blocks [block_base[k], ...) of `blocks`
 hipError_t launch_prune_cells_multi(const PruneArgs* jobs, const uint32_t* block_base, uint32_t njobs, uint32_t blocks,
 	uint32_t max_slots, hipStream_t s);
-// the same a wave per cell (PruneArgs::columns): job k owns cells [cell_base[k], ...) of `cells`
-hipError_t launch_prune_columns_multi(const PruneArgs* jobs, const uint32_t* cell_base, uint32_t njobs, uint32_t cells,
-	uint32_t max_entries, hipStream_t s);
+// the same a wave per cell (PruneArgs::columns): job k owns workgroups [block_base[k], ...) of `blocks`
+// (prune_column_blocks of each); max_entries: over the jobs that emit whole entries
+hipError_t launch_prune_columns_multi(const PruneArgs* jobs, const uint32_t* block_base, uint32_t njobs, uint32_t blocks,
+	uint32_t max_waves, uint32_t max_entries, hipStream_t s);
+hipError_t launch_eval_tile_programs(const TileEvalArgs& a, hipStream_t s);
+// many grids in one launch: job k owns workgroups [block_base[k], ...) of `blocks` (tile_eval_blocks of each)
+hipError_t launch_eval_tile_programs_multi(const TileEvalArgs* jobs, const uint32_t* block_base, uint32_t njobs,
+	uint32_t blocks, size_t lds_per_wave, hipStream_t s);
 hipError_t launch_vox(const VoxArgs& a, int stage, hipStream_t s);  // 0 select, 1 list
 hipError_t launch_pivot(const PivotArgs& a, hipStream_t s);
 hipError_t launch_cloud(const CloudArgs& a, int stage, hipStream_t s);  // 0 select, 1 points, 2 refine
@@ -437,6 +472,16 @@ __host__ __device__ inline uint64_t block_global_words(uint32_t max_binary, uint
 __host__ __device__ inline size_t block_lds_bytes_global(uint32_t slots, int p, int waves)
 {
 	return kTileInfoBytes + size_t(waves) * spill_bytes_per_wave(slots, p);
+}
+// Workgroups of the column emission and of the tile-program evaluation.
+inline uint32_t prune_column_blocks(const PruneArgs& a)
+{
+	const uint32_t per = a.emit_waves * a.emit_cells;
+	return (a.nx * a.ny * a.nz + per - 1) / per;
+}
+inline uint32_t tile_eval_blocks(const TileEvalArgs& a)
+{
+	return uint32_t((uint64_t(a.ntiles) * (uint32_t(kTile) / a.points) + kTileEvalWaves - 1) / kTileEvalWaves);
 }
 // Cell pruning: per-lane position stacks and the spill region (the decision
 // masks and liveness live in global scratch, prune_scratch_words per wave).

@@ -66,6 +66,9 @@ namespace {
 // One emission pass (and, on the first, the level-parallel decision passes)
 // with the pool capacity out.state.capacity; the five counters are copied to
 // out.host (pinned) on `stream`.
+// Bytes of a pool entry.
+size_t entry_bytes(const PruneState& ps) { return ps.words ? sizeof(uint32_t) : sizeof(Entry); }
+
 // Emission arguments of a prepared pruning (pool capacity: state.capacity).
 PruneArgs prune_args(const tg_program* p, const float origin[3], const float cell[3], const uint32_t counts[3],
 	const CellPrograms& out)
@@ -100,7 +103,14 @@ PruneArgs prune_args(const tg_program* p, const float origin[3], const float cel
 	// time is the longest walk), and loses on many cells with short programs
 	// (1024^3 blocks: 32,768 cells, 2.3 ms against the walk's 1.0 ms).
 	const bool few = ps.ncells <= kColumnCells || (ps.ncells <= 2 * kColumnCells && d.entries.size() >= 1024);
-	pa.columns = (ps.level_parallel && (out.emission == 2 || (out.emission == 0 && few))) ? 1 : 0;
+	pa.columns = (ps.level_parallel && (ps.words || out.emission == 2 || (out.emission == 0 && few))) ? 1 : 0;
+	pa.words = ps.words ? 1 : 0;
+	// One pool reservation (a device-wide atomic) for each workgroup's cells:
+	// large workgroups, and several cells to a wave once the waves fill the GPU
+	// anyway (30k tiles of a 31-entry program: 537 us with 4 cells to a
+	// workgroup).  Whole entries keep 4 waves: each has a position table in LDS.
+	pa.emit_waves = pa.words ? kEmitWaves : 4u;
+	pa.emit_cells = ps.ncells >= 4 * 8192 ? 4u : ps.ncells >= 8192 ? 2u : 1u;
 	return pa;
 }
 
@@ -157,7 +167,7 @@ int prune_pass(hipStream_t stream, const tg_program* p, const float origin[3], c
 	const uint32_t counts[3], bool fast, CellPrograms& out, bool first)
 {
 	PruneState& ps = out.state;
-	int rc = out.pool.ensure(ps.capacity * sizeof(Entry));
+	int rc = out.pool.ensure(ps.capacity * entry_bytes(ps));
 	if (rc) return rc;
 	hipError_t e = hipMemsetAsync(out.counters.ptr, 0, 64, stream);
 	if (e != hipSuccess) return hip_fail(e, "prune counters");
@@ -190,7 +200,7 @@ namespace {
 // upload of the entries by height.  *ready is false when the program is not
 // pruned here.
 int prune_prepare(hipStream_t stream, const tg_program* p, const float origin[3], const float cell[3],
-	float radius, const uint32_t counts[3], CellPrograms& out, bool* ready)
+	float radius, const uint32_t counts[3], CellPrograms& out, bool words, bool* ready)
 {
 	const DecodedProgram& d = p->decoded;
 	*ready = false;
@@ -210,6 +220,7 @@ int prune_prepare(hipStream_t stream, const tg_program* p, const float origin[3]
 		}
 	}
 	PruneState& ps = out.state;
+	ps.words = words;
 	ps.ncells = ncells;
 	// decision radius: the cell radius with the Lipschitz tolerance and the
 	// rounding slack for points of the cells' box
@@ -223,7 +234,7 @@ int prune_prepare(hipStream_t stream, const tg_program* p, const float origin[3]
 	// Fewer cells per wave only when there are very few cells (every wave
 	// gathers the whole program, so smaller groups cost L2 traffic).
 	uint32_t cpw = 64;
-	while (cpw > 16 && (ncells + cpw - 1) / cpw < 256) cpw >>= 1;
+	while (!words && cpw > 16 && (ncells + cpw - 1) / cpw < 256) cpw >>= 1;
 	ps.cells_per_wave = cpw;
 	ps.waves = (ncells + cpw - 1) / cpw;
 	int rc = out.desc.ensure(ncells * sizeof(BlockDesc));
@@ -235,6 +246,7 @@ int prune_prepare(hipStream_t stream, const tg_program* p, const float origin[3]
 	std::vector<uint32_t>& level_order = ps.level_order;
 	ps.level_parallel = entry_levels(d, level_order, ps.level_first) &&
 	                    uint64_t(d.entries.size()) * ps.waves * 64 * 4 <= kMaxValueBytes;
+	if (words && !ps.level_parallel) return TG_OK;
 	if (ps.level_parallel)
 	{
 		ps.heights = ps.level_first.size() - 1;
@@ -255,19 +267,30 @@ int prune_prepare(hipStream_t stream, const tg_program* p, const float origin[3]
 	}
 	// First guess: a quarter of the whole program per cell, at most 1 GiB; grown
 	// to the exact total and rerun if any cell did not fit (prune_cells_finish).
-	ps.capacity = std::max<uint64_t>(out.pool.bytes / sizeof(Entry),
-		std::min<uint64_t>(ncells * std::max<size_t>(d.entries.size() / 4, 16), (1ull << 30) / sizeof(Entry)));
+	// (tile programs are short: at most 64 entries each at first)
+	size_t per_cell = std::max<size_t>(d.entries.size() / 4, 16);
+	if (words) per_cell = std::min<size_t>(per_cell, 64);
+	ps.capacity = std::max<uint64_t>(out.pool.bytes / entry_bytes(ps),
+		std::min<uint64_t>(ncells * per_cell, (1ull << 30) / entry_bytes(ps)));
 	*ready = true;
 	return TG_OK;
 }
 
 }  // namespace
 
+bool level_prunable(const tg_program* p, uint64_t ncells)
+{
+	const DecodedProgram& d = p->decoded;
+	if (!d.prunable() || d.entries.empty() || d.entries.size() >= 65535 || ncells == 0 || ncells >= (1ull << 31)) return false;
+	std::vector<uint32_t> order, first;
+	return uint64_t(d.entries.size()) * ((ncells + 63) / 64) * 256 <= kMaxValueBytes && entry_levels(d, order, first);
+}
+
 int prune_cells_start(hipStream_t stream, const tg_program* p, const float origin[3], const float cell[3],
-	float radius, const uint32_t counts[3], bool fast, CellPrograms& out)
+	float radius, const uint32_t counts[3], bool fast, CellPrograms& out, bool words)
 {
 	bool ready = false;
-	int rc = prune_prepare(stream, p, origin, cell, radius, counts, out, &ready);
+	int rc = prune_prepare(stream, p, origin, cell, radius, counts, out, words, &ready);
 	if (rc || !ready) return rc;
 	rc = prune_pass(stream, p, origin, cell, counts, fast, out, true);
 	if (rc) return rc;
@@ -285,12 +308,13 @@ int prune_cells_many(hipStream_t stream, const tg_program* const* progs, const C
 	{
 		bool r = false;
 		int rc = prune_prepare(stream, progs[i], grids[i].origin, grids[i].cell, grids[i].radius, grids[i].counts,
-			*outs[i], &r);
+			*outs[i], grids[i].words, &r);
 		if (rc) return rc;
+		if (!r && grids[i].words) return fail(TG_ERR_LIMIT, "tile programs need the level-parallel pruning");
 		if (!r) continue;
 		CellPrograms& out = *outs[i];
 		ready[i] = 1;
-		rc = out.pool.ensure(out.state.capacity * sizeof(Entry));
+		rc = out.pool.ensure(out.state.capacity * entry_bytes(out.state));
 		if (rc) return rc;
 		TG_CHECK_HIP(hipMemsetAsync(out.counters.ptr, 0, 64, stream), "prune counters");
 		if (out.state.level_parallel)
@@ -338,10 +362,11 @@ int prune_cells_many(hipStream_t stream, const tg_program* const* progs, const C
 		level_launches.push_back(Launch{ j, b, uint32_t(jobs.size()), waves });
 	}
 	// emission jobs: the sequential walk's (a wave per group part) and the
-	// column emission's (a wave per cell), one launch each
+	// column emission's (a wave per cell), one launch each; `cells`: the
+	// latter's workgroups
 	std::vector<PruneArgs> ejobs, cjobs;
 	std::vector<uint32_t> ebase, cbase;
-	uint32_t blocks = 0, max_slots = 1, cells = 0, max_entries = 1;
+	uint32_t blocks = 0, max_slots = 1, cells = 0, max_entries = 0, max_waves = 1;
 	for (uint32_t i = 0; i < n; ++i)
 	{
 		if (!ready[i]) continue;
@@ -350,8 +375,9 @@ int prune_cells_many(hipStream_t stream, const tg_program* const* progs, const C
 		if (pa.masks_ready && pa.columns)
 		{
 			cbase.push_back(cells);
-			cells += ncells;
-			max_entries = std::max(max_entries, pa.n_entries);
+			cells += prune_column_blocks(pa);
+			max_waves = std::max(max_waves, pa.emit_waves);
+			if (!pa.words) max_entries = std::max(max_entries, pa.n_entries);
 			cjobs.push_back(pa);
 			continue;
 		}
@@ -361,7 +387,6 @@ int prune_cells_many(hipStream_t stream, const tg_program* const* progs, const C
 		max_slots = std::max(max_slots, pa.slots);
 		ejobs.push_back(pa);
 	}
-	cbase.push_back(cells);
 	size_t ej = 0, eb = 0, cj = 0, cb = 0;
 	if (!ejobs.empty())
 	{
@@ -403,8 +428,8 @@ int prune_cells_many(hipStream_t stream, const tg_program* const* progs, const C
 		const PruneArgs* jobs = reinterpret_cast<const PruneArgs*>(dev + cj);
 		const uint32_t* base = reinterpret_cast<const uint32_t*>(dev + cb);
 		const hipError_t e =
-			fast ? fast::launch_prune_columns_multi(jobs, base, uint32_t(cjobs.size()), cells, max_entries, stream)
-			     : exact::launch_prune_columns_multi(jobs, base, uint32_t(cjobs.size()), cells, max_entries, stream);
+			fast ? fast::launch_prune_columns_multi(jobs, base, uint32_t(cjobs.size()), cells, max_waves, max_entries, stream)
+			     : exact::launch_prune_columns_multi(jobs, base, uint32_t(cjobs.size()), cells, max_waves, max_entries, stream);
 		if (e != hipSuccess) return hip_fail(e, "cell pruning launch");
 	}
 	for (uint32_t i = 0; i < n; ++i)
@@ -428,7 +453,7 @@ int prune_cells_finish(hipStream_t stream, const tg_program* p, const float orig
 	hipError_t e = hipStreamSynchronize(stream);
 	if (e != hipSuccess) return hip_fail(e, "cell pruning");
 	const unsigned long long* c = out.host;
-	if (c[0] > ps.capacity && c[0] * sizeof(Entry) <= (size_t(8) << 30))
+	if (c[0] > ps.capacity && c[0] * entry_bytes(ps) <= (size_t(8) << 30))
 	{
 		// some cells did not fit: rerun the emission with the exact total
 		out.reran = true;
@@ -451,7 +476,7 @@ int prune_cells_finish(hipStream_t stream, const tg_program* p, const float orig
 int prune_cells(hipStream_t stream, const tg_program* p, const float origin[3], const float cell[3], float radius,
 	const uint32_t counts[3], bool fast, CellPrograms& out)
 {
-	int rc = prune_cells_start(stream, p, origin, cell, radius, counts, fast, out);
+	int rc = prune_cells_start(stream, p, origin, cell, radius, counts, fast, out, false);
 	if (rc) return rc;
 	return prune_cells_finish(stream, p, origin, cell, counts, fast, out);
 }
