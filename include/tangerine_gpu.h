@@ -410,11 +410,13 @@ int tg_mesher_set_culled_tuning(tg_mesher* mesher, uint32_t points_per_lane, uin
                                 uint32_t workgroups_per_cu);
 /* How the mesher's block pruning emits each block's program once its
  * decision and liveness passes ran: 0 automatic (the default: a wave per
- * block, with a lane per program entry, on grids of at most 2048 blocks, or
- * 4096 for programs of 1024 entries or more; otherwise the walk), 1 one wave
+ * block, with a lane per program entry, on grids of at most 8192 blocks, or
+ * 16384 for programs of 1024 entries or more; otherwise the walk), 1 one wave
  * walking the entries of 16 blocks at a time, 2 a wave per block.  Every
  * setting emits the same programs, so exports give the same samples and
- * mesh. */
+ * mesh.  A mesher whose emission or tuning was set (to any value) evaluates
+ * every grid by blocks; one left alone evaluates grids of few tiles and short
+ * programs a wave per 8^3-sample tile, with the same samples. */
 int tg_mesher_set_emission(tg_mesher* mesher, uint32_t mode);
 
 /* ---- batched export (no reference counterpart; closest: one Sodapop

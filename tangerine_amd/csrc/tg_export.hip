@@ -51,7 +51,7 @@ struct tg_mesher
 	// surface-net stages run without waiting for their counts
 	uint64_t spec_verts = 0, spec_quads = 0;
 	uint32_t* tail = nullptr;     // pinned: vertex and quad totals read back by surface nets, then
-	                              // (from word 4) the block evaluation's two work counters
+	                              // (from word 4) the evaluation's work counters
 	uint32_t* tail_dev = nullptr; // the same words as the kernels address them
 	bool have_grid = false;
 	tg_export_stats stats{};
@@ -316,7 +316,7 @@ constexpr size_t kMaxLds = 160 * 1024 - 256;
 // [8b, 8b + 8]) reads sample tiles b and b + 1 on each axis, so tile i is
 // needed when one of the bricks i - 1 and i (per axis) is kept: one ballot is
 // the block's mask, stored whole (no atomics).  The lane whose tile index is
-// a brick index counts that brick when it is kept (counter[0]).
+// a brick index counts that brick when it is kept (counter slots, 0).
 __global__ void __launch_bounds__(256) k_tiles_from_bricks(const uint8_t* flags, uint32_t cbx, uint32_t cby,
 	uint32_t cbz, uint32_t tx, uint32_t ty, uint32_t tz, uint32_t bx, uint32_t by, uint32_t bz,
 	unsigned long long* mask, unsigned long long* counter)
@@ -343,7 +343,7 @@ __global__ void __launch_bounds__(256) k_tiles_from_bricks(const uint8_t* flags,
 	if (lane == 0)
 	{
 		mask[w] = m;
-		if (o) atomicAdd(counter, (unsigned long long)__popcll(o));
+		if (o) atomicAdd(&counter[size_t(blockIdx.x % kWorkSlots) * kWorkStride], (unsigned long long)__popcll(o));
 	}
 }
 
@@ -540,8 +540,8 @@ BlockEvalArgs block_args(tg_mesher* m, const tg_program* p, const tg_grid* g, co
 	return ba;
 }
 
-// The block evaluation's work counters, copied back into the pinned words 4..7
-// of m->tail.
+// The block evaluation's work counters, copied back into pinned memory behind
+// the first four words of m->tail.
 unsigned long long* work_readback(tg_mesher* m) { return reinterpret_cast<unsigned long long*>(m->tail + 4); }
 
 // The persistent launch's queue: the n blocks (all, or those of `list`) by
@@ -569,10 +569,10 @@ int block_order(tg_mesher* m, const BlockDesc* desc, const uint32_t* list, uint3
 int eval_blocks(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t flags, const uint64_t* tile_mask,
 	const uint32_t* block_list, uint32_t n_listed, bool sorted = false)
 {
-	int rc = m->counters.ensure(64);
+	int rc = m->counters.ensure(kWorkBytes);
 	if (rc) return rc;
 	unsigned long long* work = m->counters.as<unsigned long long>();
-	TG_CHECK_HIP(hipMemsetAsync(m->counters.ptr, 0, 64, m->stream), "counter reset");
+	TG_CHECK_HIP(hipMemsetAsync(m->counters.ptr, 0, kWorkBytes, m->stream), "counter reset");
 	BlockEvalArgs ba = block_args(m, p, g, tile_mask, block_list, n_listed, work);
 	// culled exports (a block list) have their own launch shape
 	const bool culled = block_list != nullptr;
@@ -633,7 +633,7 @@ int eval_blocks(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t fl
 		         : exact::launch_batch(q, pts, uint32_t(waves), wgs, m->stream);
 		if (e != hipSuccess) return hip_fail(e, "block evaluation launch");
 		TG_CHECK_HIP(hipEventRecord(m->ev[5], m->stream), "event");
-		TG_CHECK_HIP(hipMemcpyAsync(work_readback(m), work, 16, hipMemcpyDeviceToHost, m->stream), "work read");
+		TG_CHECK_HIP(hipMemcpyAsync(work_readback(m), work, kWorkBytes, hipMemcpyDeviceToHost, m->stream), "work read");
 		return TG_OK;
 	}
 	// Fit the LDS: fewer points per lane first, then fewer waves.
@@ -660,7 +660,7 @@ int eval_blocks(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t fl
 	                                      : exact::launch_eval_blocks(ba, pts, m->stream);
 	if (e != hipSuccess) return hip_fail(e, "block evaluation launch");
 	TG_CHECK_HIP(hipEventRecord(m->ev[5], m->stream), "event");
-	TG_CHECK_HIP(hipMemcpyAsync(work_readback(m), work, 16, hipMemcpyDeviceToHost, m->stream), "work read");
+	TG_CHECK_HIP(hipMemcpyAsync(work_readback(m), work, kWorkBytes, hipMemcpyDeviceToHost, m->stream), "work read");
 	return TG_OK;
 }
 
@@ -668,10 +668,10 @@ int eval_blocks(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t fl
 // Asynchronous, read as eval_blocks is.
 int eval_tile_programs(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t flags)
 {
-	int rc = m->counters.ensure(64);
+	int rc = m->counters.ensure(kWorkBytes);
 	if (rc) return rc;
 	unsigned long long* work = m->counters.as<unsigned long long>();
-	TG_CHECK_HIP(hipMemsetAsync(m->counters.ptr, 0, 64, m->stream), "counter reset");
+	TG_CHECK_HIP(hipMemsetAsync(m->counters.ptr, 0, kWorkBytes, m->stream), "counter reset");
 	const TileEvalArgs ta = tile_args(m, p, g, work);
 	m->last_points_per_lane = int(ta.points);
 	m->last_waves = int(kTileEvalWaves);
@@ -684,7 +684,7 @@ int eval_tile_programs(tg_mesher* m, const tg_program* p, const tg_grid* g, uint
 	                                            : exact::launch_eval_tile_programs(ta, m->stream);
 	if (e != hipSuccess) return hip_fail(e, "tile evaluation launch");
 	TG_CHECK_HIP(hipEventRecord(m->ev[5], m->stream), "event");
-	TG_CHECK_HIP(hipMemcpyAsync(work_readback(m), work, 16, hipMemcpyDeviceToHost, m->stream), "work read");
+	TG_CHECK_HIP(hipMemcpyAsync(work_readback(m), work, kWorkBytes, hipMemcpyDeviceToHost, m->stream), "work read");
 	return TG_OK;
 }
 
@@ -694,8 +694,8 @@ int eval_blocks_read(tg_mesher* m, uint64_t* evals, double* flops)
 	float kms = 0;
 	TG_CHECK_HIP(hipEventElapsedTime(&kms, m->ev[4], m->ev[5]), "timing");
 	m->last_block_ms = kms;
-	*evals = work_readback(m)[0];
-	*flops = double(work_readback(m)[1]);
+	*evals = work_sum(work_readback(m), 0);
+	*flops = double(work_sum(work_readback(m), 1));
 	return TG_OK;
 }
 
@@ -714,7 +714,7 @@ extern "C" int tg_mesher_create(tg_mesher** out)
 	if (e == hipSuccess) e = hipDeviceGetAttribute(&m->cus, hipDeviceAttributeMultiprocessorCount, dev);
 	if (e == hipSuccess) e = hipStreamCreate(&m->stream);
 	for (int i = 0; e == hipSuccess && i < 6; ++i) e = hipEventCreate(&m->ev[i]);
-	if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&m->tail), 32, hipHostMallocDefault);
+	if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&m->tail), 16 + kWorkBytes, hipHostMallocDefault);
 	if (e == hipSuccess) e = hipHostGetDevicePointer(reinterpret_cast<void**>(&m->tail_dev), m->tail, 0);
 	if (e != hipSuccess)
 	{
@@ -789,10 +789,10 @@ int select_tiles(tg_mesher* m, const tg_program* p, const tg_grid* g, const tg_s
 	int rc = m->brick_flags.ensure(nbricks);
 	if (!rc) rc = m->tile_mask.ensure(nblocks * 8);
 	if (!rc) rc = tiles ? m->tile_list.ensure(ntiles * 4) : m->block_list.ensure(nblocks * 4);
-	if (!rc) rc = m->counters.ensure(64);
+	if (!rc) rc = m->counters.ensure(kWorkBytes);
 	if (rc) return rc;
 	unsigned long long* ctr = m->counters.as<unsigned long long>();
-	TG_CHECK_HIP(hipMemsetAsync(m->counters.ptr, 0, 64, m->stream), "counter reset");
+	TG_CHECK_HIP(hipMemsetAsync(m->counters.ptr, 0, kWorkBytes, m->stream), "counter reset");
 	TG_CHECK_HIP(hipMemsetAsync(m->tile_mask.ptr, 0, nblocks * 8, m->stream), "mask reset");
 	const float radius = 4.0f * std::sqrt(g->dx * g->dx + g->dy * g->dy + g->dz * g->dz);
 	sel.threshold = 0.0f;
@@ -836,7 +836,7 @@ int select_tiles(tg_mesher* m, const tg_program* p, const tg_grid* g, const tg_s
 		ca.cbx = ma.cbx; ca.cby = ma.cby; ca.cbz = ma.cbz;
 		ca.radius = radius * (1.0f + 1.0e-5f) + rounding_slack(p->decoded, grid_reach(g));
 		ca.flags = m->brick_flags.as<uint8_t>();
-		ca.counters = ctr + 2;
+		ca.counters = ctr;
 		ca.slots = std::max<uint32_t>(1, std::max(blocks ? m->blocks.max_stack : 0u, p->decoded.max_stack) - 1);
 		hipError_t e = (flags & TG_FLAG_FAST) ? fast::launch_certify(ca, m->stream) : exact::launch_certify(ca, m->stream);
 		if (e != hipSuccess) return hip_fail(e, "brick certificate launch");
@@ -852,13 +852,15 @@ int select_tiles(tg_mesher* m, const tg_program* p, const tg_grid* g, const tg_s
 		hipLaunchKernelGGL(k_list_blocks, dim3(grid_for(nblocks)), dim3(256), 0, m->stream,
 			m->tile_mask.as<const unsigned long long>(), uint32_t(nblocks), m->block_list.as<uint32_t>(), ctr + 1);
 	TG_CHECK_HIP(hipGetLastError(), "list launch");
-	unsigned long long c[4] = { 0, 0, 0, 0 };
-	TG_CHECK_HIP(hipMemcpyAsync(c, ctr, sizeof(c), hipMemcpyDeviceToHost, m->stream), "count read");
+	// counters: 0 kept bricks, 1 (slot 0 only) listed blocks or tiles, 2 bricks
+	// the certificate added, 3 its cost
+	unsigned long long* c = work_readback(m);
+	TG_CHECK_HIP(hipMemcpyAsync(c, ctr, kWorkBytes, hipMemcpyDeviceToHost, m->stream), "count read");
 	TG_CHECK_HIP(hipStreamSynchronize(m->stream), "tile selection");
-	sel.flagged = c[0];
-	sel.listed = uint32_t(c[1]);
-	sel.certified = c[2];
-	sel.cert_flops = double(c[3]);
+	sel.flagged = work_sum(c, 0);
+	sel.listed = uint32_t(work_sum(c, 1));
+	sel.certified = work_sum(c, 2);
+	sel.cert_flops = double(work_sum(c, 3));
 	m->nbricks = nbricks;
 	ma.brick_flags = m->brick_flags.as<const uint8_t>();
 	return TG_OK;
@@ -1940,7 +1942,7 @@ int capture_batch(tg_batch* b)
 	drop_graph(b);
 	int rc = shape_batch(b, b->points_per_lane, b->waves, b->workgroups_per_cu);
 	if (rc) return rc;
-	const uint32_t nwork = uint32_t(2 * b->meshers.size());
+	const uint32_t nwork = uint32_t(b->meshers.size() * (kWorkBytes / 8));
 	TG_CHECK_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal), "capture begin");
 	hipError_t e = b->fast ? fast::launch_batch_reset(b->args.head, b->work.as<unsigned long long>(), nwork, b->stream)
 	                       : exact::launch_batch_reset(b->args.head, b->work.as<unsigned long long>(), nwork, b->stream);
@@ -2063,7 +2065,7 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 	b->grids.assign(grids, grids + count);
 	b->by_tiles.assign(count, 0);
 	auto t0 = std::chrono::steady_clock::now();
-	int rc = b->work.ensure(size_t(count) * 16);
+	int rc = b->work.ensure(size_t(count) * kWorkBytes);
 	if (!rc) rc = b->head.ensure(256);
 	if (!rc) rc = b->trees.ensure(size_t(count) * sizeof(BlockEvalArgs));
 	if (rc) return rc;
@@ -2110,7 +2112,7 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 		if (rc) return rc;
 		if (!m->blocks.valid) return fail(TG_ERR_LIMIT, "tg_batch_export: a tree could not be pruned");
 		samples += uint64_t(m->args.nx) * m->args.ny * m->args.nz;
-		unsigned long long* work = b->work.as<unsigned long long>() + 2 * i;
+		unsigned long long* work = b->work.as<unsigned long long>() + size_t(i) * (kWorkBytes / 8);
 		if (b->by_tiles[i])
 		{
 			args[i].nblocks = 0;  // no queue items
@@ -2188,10 +2190,14 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 	float eval_ms = 0;
 	rc = replay_batch(b, &eval_ms);
 	if (rc) return rc;
-	std::vector<unsigned long long> wk(2 * size_t(count));
-	TG_CHECK_HIP(hipMemcpy(wk.data(), b->work.ptr, wk.size() * 8, hipMemcpyDeviceToHost), "work read");
+	std::vector<unsigned long long> slots(size_t(count) * (kWorkBytes / 8)), wk(2 * size_t(count));
+	TG_CHECK_HIP(hipMemcpy(slots.data(), b->work.ptr, slots.size() * 8, hipMemcpyDeviceToHost), "work read");
 	for (uint32_t i = 0; i < count; ++i)
-		if (b->by_tiles[i]) wk[2 * i] = uint64_t(b->meshers[i]->blocks.ncells) * kTileSamples;
+	{
+		const unsigned long long* w = slots.data() + size_t(i) * (kWorkBytes / 8);
+		wk[2 * i] = b->by_tiles[i] ? uint64_t(b->meshers[i]->blocks.ncells) * kTileSamples : work_sum(w, 0);
+		wk[2 * i + 1] = work_sum(w, 1);
+	}
 	auto t2 = std::chrono::steady_clock::now();
 	double mesh_ms = 0;
 	uint64_t evals = 0;

@@ -59,7 +59,7 @@ bool entry_levels(const DecodedProgram& d, std::vector<uint32_t>& order, std::ve
 
 // Grids of at most this many cells (twice as many for programs of 1024
 // entries or more) emit a wave per cell (PruneArgs::columns).
-constexpr uint64_t kColumnCells = 2048;
+constexpr uint64_t kColumnCells = 8192;
 
 namespace {
 
@@ -101,15 +101,17 @@ PruneArgs prune_args(const tg_program* p, const float origin[3], const float cel
 	// A wave per cell (a lane per entry) scans the whole program for every
 	// cell: it wins on grids of few cells, whose programs are long (the walk's
 	// time is the longest walk), and loses on many cells with short programs
-	// (1024^3 blocks: 32,768 cells, 2.3 ms against the walk's 1.0 ms).
+	// (4913 cells of 4095 entries 0.10 ms against the walk's 0.69, 35,937 cells
+	// of the same 0.39 against 0.41, 266,240 of 511 0.57 against 0.21).
 	const bool few = ps.ncells <= kColumnCells || (ps.ncells <= 2 * kColumnCells && d.entries.size() >= 1024);
 	pa.columns = (ps.level_parallel && (ps.words || out.emission == 2 || (out.emission == 0 && few))) ? 1 : 0;
 	pa.words = ps.words ? 1 : 0;
 	// One pool reservation (a device-wide atomic) for each workgroup's cells:
 	// large workgroups, and several cells to a wave once the waves fill the GPU
 	// anyway (30k tiles of a 31-entry program: 537 us with 4 cells to a
-	// workgroup).  Whole entries keep 4 waves: each has a position table in LDS.
-	pa.emit_waves = pa.words ? kEmitWaves : 4u;
+	// workgroup).  Whole entries: each wave has a position table in LDS (12
+	// bytes per 64 entries of the program).
+	pa.emit_waves = pa.words || d.entries.size() <= 8192 ? kEmitWaves : 4u;
 	pa.emit_cells = ps.ncells >= 4 * 8192 ? 4u : ps.ncells >= 8192 ? 2u : 1u;
 	return pa;
 }

@@ -261,7 +261,7 @@ extern "C" int tg_tracer_render(tg_tracer* tr, const tg_program* p, const tg_cam
 	int rc = tr->t.ensure(n * 4);
 	if (!rc) rc = tr->normals.ensure(n * 12);
 	if (!rc) rc = tr->steps.ensure(n * 4);
-	if (!rc) rc = tr->work.ensure(64);
+	if (!rc) rc = tr->work.ensure(kWorkBytes);
 	if (!rc) rc = tr->qctl.ensure(size_t(npass) * 4);
 	if (!rc && passes) rc = ensure_pass_buffers(tr, n);
 	if (rc) return rc;
@@ -346,7 +346,7 @@ extern "C" int tg_tracer_render(tg_tracer* tr, const tg_program* p, const tg_cam
 	ta.n_out = tr->normals.as<float>();
 	ta.steps_out = tr->steps.as<uint32_t>();
 	ta.work = tr->work.as<unsigned long long>();
-	TG_CHECK_HIP(hipMemsetAsync(tr->work.ptr, 0, 64, tr->stream), "work reset");
+	TG_CHECK_HIP(hipMemsetAsync(tr->work.ptr, 0, kWorkBytes, tr->stream), "work reset");
 	// per pass: the count of rays it queued
 	uint32_t* ctl = tr->qctl.as<uint32_t>();
 	TG_CHECK_HIP(hipMemsetAsync(ctl, 0, size_t(npass) * 4, tr->stream), "pass counters");
@@ -384,15 +384,15 @@ extern "C" int tg_tracer_render(tg_tracer* tr, const tg_program* p, const tg_cam
 		taken += ta.budget;
 	}
 	TG_CHECK_HIP(hipEventRecord(tr->ev[2], tr->stream), "event");
-	unsigned long long wk[3] = { 0, 0, 0 };
-	TG_CHECK_HIP(hipMemcpyAsync(wk, tr->work.ptr, 24, hipMemcpyDeviceToHost, tr->stream), "work read");
+	unsigned long long wk[kWorkBytes / 8] = {};
+	TG_CHECK_HIP(hipMemcpyAsync(wk, tr->work.ptr, kWorkBytes, hipMemcpyDeviceToHost, tr->stream), "work read");
 	TG_CHECK_HIP(hipStreamSynchronize(tr->stream), "trace");
 	float t_prune = 0, t_trace = 0;
 	hipEventElapsedTime(&t_prune, tr->ev[0], tr->ev[1]);
 	hipEventElapsedTime(&t_trace, tr->ev[1], tr->ev[2]);
 	tr->width = cam->width;
 	tr->height = cam->height;
-	tr->stats = tg_trace_stats{ t_trace, t_prune, n, wk[2], wk[0], double(wk[1]) };
+	tr->stats = tg_trace_stats{ t_trace, t_prune, n, work_sum(wk, 2), work_sum(wk, 0), double(work_sum(wk, 1)) };
 	return TG_OK;
 }
 
