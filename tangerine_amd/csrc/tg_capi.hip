@@ -304,8 +304,16 @@ int tg::upload_program(const DecodedProgram& d, tg_program** out)
 	auto p = std::make_unique<tg_program>();
 	p->uid = next_uid++;
 	p->decoded = d;
+	p->plan = prune_plan(d);
+	static_assert(sizeof(HostEntry) == 16 && sizeof(TreeletItem) == 16 && sizeof(Treelet) == 16, "one array of 16-byte words");
+	std::vector<HostEntry> blob(d.entries);
+	const size_t items = blob.size(), treelets = items + p->plan.items.size();
+	blob.resize(std::max<size_t>(treelets + p->plan.treelets.size(), 1));
+	if (!p->plan.items.empty()) std::memcpy(&blob[items], p->plan.items.data(), p->plan.items.size() * sizeof(TreeletItem));
+	if (!p->plan.treelets.empty())
+		std::memcpy(&blob[treelets], p->plan.treelets.data(), p->plan.treelets.size() * sizeof(Treelet));
 	rc = p->device.ensure(d.instrs.size() * sizeof(Instr));
-	if (!rc) rc = p->entries.ensure(std::max<size_t>(d.entries.size(), 1) * sizeof(HostEntry));
+	if (!rc) rc = p->entries.ensure(blob.size() * sizeof(HostEntry));
 	if (rc)
 	{
 		p->device.release();
@@ -313,7 +321,7 @@ int tg::upload_program(const DecodedProgram& d, tg_program** out)
 	}
 	TG_CHECK_HIP(hipMemcpy(p->device.ptr, d.instrs.data(), d.instrs.size() * sizeof(Instr), hipMemcpyHostToDevice),
 		"program upload");
-	TG_CHECK_HIP(hipMemcpy(p->entries.ptr, d.entries.data(), d.entries.size() * sizeof(HostEntry), hipMemcpyHostToDevice),
+	TG_CHECK_HIP(hipMemcpy(p->entries.ptr, blob.data(), blob.size() * sizeof(HostEntry), hipMemcpyHostToDevice),
 		"program entries upload");
 	*out = p.release();
 	return TG_OK;

@@ -33,8 +33,14 @@ struct tg_program
 {
 	uint64_t uid = 0;    // unique per uploaded program (caches of derived device data key on it)
 	tg::DecodedProgram decoded;
+	tg::PrunePlan plan;  // its treelets
 	tg::DevBuf device;   // Instr records
-	tg::DevBuf entries;  // whole program as pruning entries
+	tg::DevBuf entries;  // whole program as pruning entries, then the plan's items and treelets
+	const tg::TreeletItem* items() const
+	{
+		return reinterpret_cast<const tg::TreeletItem*>(entries.as<const tg::HostEntry>() + decoded.entries.size());
+	}
+	const tg::Treelet* treelets() const { return reinterpret_cast<const tg::Treelet*>(items() + plan.items.size()); }
 };
 
 namespace tg {
@@ -44,21 +50,18 @@ int upload_program(const DecodedProgram& d, tg_program** out);
 struct PruneState
 {
 	bool pending = false;        // a pass was issued; its counters are not read yet
-	bool level_parallel = false;
+	bool treelets = false;       // grid-wide treelet passes (else one wave walks the program per cell group)
 	bool words = false;          // one word per entry (PruneArgs::words)
 	uint64_t ncells = 0, waves = 0, capacity = 0;
 	uint32_t cells_per_wave = 0;
 	float decide_radius = 0.0f;
-	size_t heights = 0;
-	std::vector<uint32_t> level_first;  // first entry position of every height
-	std::vector<uint32_t> level_order;  // entry positions by height (the upload's source, kept until finish)
 };
 
 // Level-1 pruned programs of a cell grid (BlockDesc per cell + entry pool).
 struct CellPrograms
 {
 	DevBuf pool, desc, counters, scratch;
-	DevBuf values, levels, lens;  // level-parallel passes: entry values per cell, entries by height, program lengths
+	DevBuf values, lens;      // treelet passes: treelet root values per cell, program lengths
 	uint64_t ncells = 0;
 	uint64_t entries = 0;     // pool entries in use
 	uint32_t max_stack = 0;   // over all cells
@@ -67,9 +70,7 @@ struct CellPrograms
 	uint64_t whole_cells = 0; // cells left with the whole program (pool overflow)
 	bool valid = false;       // false: the program is not prunable here
 	bool reran = false;       // the last pruning emitted again after a pool overflow (desc changed)
-	int emission = 0;         // after level-parallel passes: 0 automatic, 1 sequential walk, 2 a wave per cell
-	uint64_t levels_uid = 0;  // program whose entries by height `levels` holds (0: none)
-	size_t levels_bytes = 0;  // ... in the allocation of this size (a grown buffer is a new one)
+	int emission = 0;         // after treelet passes: 0 automatic, 1 sequential walk, 2 a wave per cell
 	PruneState state;
 	unsigned long long* host = nullptr;  // pinned copy of the pass counters
 	void release()
@@ -81,19 +82,17 @@ struct CellPrograms
 		counters.release();
 		scratch.release();
 		values.release();
-		levels.release();
-		levels_uid = 0;
 		lens.release();
 	}
 };
 
 // With `words` the cells' programs are one word per entry; the result is only
-// valid where the level-parallel passes apply.
+// valid where the treelet passes apply.
 int prune_cells(hipStream_t stream, const tg_program* p, const float origin[3], const float cell[3], float radius,
 	const uint32_t counts[3], bool fast, CellPrograms& out);
 
-// Whether `p` can be pruned over ncells cells by the level-parallel passes.
-bool level_prunable(const tg_program* p, uint64_t ncells);
+// Whether `p` can be pruned over ncells cells by the treelet passes.
+bool treelet_prunable(const tg_program* p, uint64_t ncells);
 
 // A cell grid to prune a program over.
 struct CellGrid
@@ -110,9 +109,8 @@ struct PruneLaunches
 	std::vector<uint8_t> host;
 };
 
-// prune_cells_start for n programs on one stream: every program's height-h
-// pass in one launch per height, then every emission in one launch (instead
-// of a launch per program and height).  Each is then finished with
+// prune_cells_start for n programs on one stream: every program's treelet
+// passes of one stage in one launch, then every emission in one launch.  Each is then finished with
 // prune_cells_finish on the same stream.
 int prune_cells_many(hipStream_t stream, const tg_program* const* progs, const CellGrid* grids, uint32_t n, bool fast,
 	CellPrograms* const* outs, PruneLaunches& work);

@@ -440,7 +440,7 @@ constexpr uint64_t kTileEntryCells = 150ull << 20;
 bool tile_programs(const tg_program* p, const MeshArgs& ma)
 {
 	const uint64_t tiles = uint64_t(ma.tx) * ma.ty * ma.tz;
-	return tiles * p->decoded.entries.size() <= kTileEntryCells && level_prunable(p, tiles);
+	return tiles * p->decoded.entries.size() <= kTileEntryCells && treelet_prunable(p, tiles);
 }
 
 // The 8^3-sample tiles as cells (samples lie within 3.5 |d| of a tile's centre).

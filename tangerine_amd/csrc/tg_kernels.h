@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "tg_program.h"
 #include "tg_types.h"
 
 namespace tg {
@@ -112,7 +113,7 @@ struct PruneArgs
 	unsigned long long* counters;
 	uint64_t* scratch;      // per wave: 2 n_binary + n_entries words (decision masks, liveness)
 	uint32_t cells_per_wave;  // 1..64 (lanes beyond carry no cell)
-	int masks_ready;          // decision masks and liveness already in scratch (k_prune_level): skip both passes
+	int masks_ready;          // decision masks and liveness already in scratch (k_prune_treelets): skip both passes
 	const uint32_t* counts;   // with masks_ready: program length per lane, [group][64]
 	uint32_t splits;          // with masks_ready: waves per cell group (1, 2 or 4), each emitting 64 / splits columns
 	int columns;              // with masks_ready: a wave per cell, a lane per entry (k_prune_columns)
@@ -122,29 +123,30 @@ struct PruneArgs
 };
 constexpr uint32_t kEmitWaves = 16;
 
-// Level-parallel decision pass: one launch per entry height (leaves 0, a
-// parent one above its highest child); wave = (entry of the level, cell
-// group of k_prune_cells), lane = cell.  Every entry's value at every cell
-// centre is kept in `values`, so a parent reads its operands instead of
-// re-running the program; binary entries record the same decision masks as
-// k_prune_cells' own pass.
-struct LevelArgs
+// Treelet passes (PrunePlan): one launch per stage, wave = (treelet of the
+// stage, cell group of k_prune_cells), lane = cell.  Upward, a wave runs its
+// treelet at the cell centres, records the decision masks of its binary
+// entries and stores its root's value for the stage above; downward, it turns
+// its root's live columns into its entries' and adds up the lengths of the
+// cells' programs.  Both directions at once for the program's root treelet.
+struct TreeletArgs
 {
 	const Instr* prog;
-	const Entry* entries;
-	const uint32_t* list;     // entry positions of this height
-	uint32_t count;           // entries of this height
-	uint32_t ngroups;         // cell groups (waves of k_prune_cells)
-	uint32_t groups_per_wave; // consecutive cell groups one wave runs (the entry's record loaded once)
+	const TreeletItem* items;
+	const Treelet* treelets;
+	uint32_t first, count;    // treelets of this stage
+	uint32_t ngroups;         // cell groups
 	uint32_t cells_per_wave;
 	float ox, oy, oz, cx, cy, cz, radius;
 	uint32_t nx, ny, nz;
-	float* values;            // [entry][group][64 lanes]
+	float* values;            // [value slot][group][64 lanes]
 	uint64_t* scratch;        // decision masks and liveness, as PruneArgs::scratch
 	uint32_t n_binary, n_entries;
-	int liveness;             // 0: values and decisions (heights upward); 1: liveness (heights downward)
-	uint32_t* counts;         // liveness: entries each lane's program will hold, [group][64] (zeroed)
+	uint32_t slots;           // LDS spill slots (whole-program max stack - 1)
+	int up, down;             // directions of this launch
+	uint32_t* counts;         // downward: entries each lane's program will hold, [group][64] (zeroed)
 };
+constexpr uint32_t kTreeletWaves = 4;  // waves per workgroup
 
 // Level 2 + evaluation: one workgroup per block.
 struct BlockEvalArgs
@@ -368,10 +370,11 @@ struct GradArgs
 // fast = contracted FP32).  `p` is points per lane for the tile kernel (4 or 8).
 namespace exact {
 hipError_t launch_points(const PointArgs& a, hipStream_t s);
-hipError_t launch_prune_level(const LevelArgs& a, hipStream_t s);
+uint32_t treelet_waves(const TreeletArgs& a);
+hipError_t launch_prune_treelets(const TreeletArgs& a, hipStream_t s);
 // many programs' passes in one launch: job k owns waves [wave_base[k], wave_base[k + 1]) of `waves`
-hipError_t launch_prune_level_multi(const LevelArgs* jobs, const uint32_t* wave_base, uint32_t njobs, uint32_t waves,
-	hipStream_t s);
+hipError_t launch_prune_treelets_multi(const TreeletArgs* jobs, const uint32_t* wave_base, uint32_t njobs, uint32_t waves,
+	uint32_t max_slots, hipStream_t s);
 // many programs' emissions in one launch: job k owns blocks [block_base[k], ...) of `blocks`
 hipError_t launch_prune_cells_multi(const PruneArgs* jobs, const uint32_t* block_base, uint32_t njobs, uint32_t blocks,
 	uint32_t max_slots, hipStream_t s);
@@ -402,10 +405,11 @@ hipError_t launch_quotient_check(float b, unsigned long long* counts, hipStream_
 }
 namespace fast {
 hipError_t launch_points(const PointArgs& a, hipStream_t s);
-hipError_t launch_prune_level(const LevelArgs& a, hipStream_t s);
+uint32_t treelet_waves(const TreeletArgs& a);
+hipError_t launch_prune_treelets(const TreeletArgs& a, hipStream_t s);
 // many programs' passes in one launch: job k owns waves [wave_base[k], wave_base[k + 1]) of `waves`
-hipError_t launch_prune_level_multi(const LevelArgs* jobs, const uint32_t* wave_base, uint32_t njobs, uint32_t waves,
-	hipStream_t s);
+hipError_t launch_prune_treelets_multi(const TreeletArgs* jobs, const uint32_t* wave_base, uint32_t njobs, uint32_t waves,
+	uint32_t max_slots, hipStream_t s);
 // many programs' emissions in one launch: job k owns blocks [block_base[k], ...) of `blocks`
 hipError_t launch_prune_cells_multi(const PruneArgs* jobs, const uint32_t* block_base, uint32_t njobs, uint32_t blocks,
 	uint32_t max_slots, hipStream_t s);

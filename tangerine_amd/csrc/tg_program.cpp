@@ -188,6 +188,94 @@ float rounding_slack(const DecodedProgram& d, float pmax)
 	return float(std::max(s, 2.0e-4));
 }
 
+PrunePlan prune_plan(const DecodedProgram& d)
+{
+	PrunePlan plan;
+	const uint32_t n = uint32_t(d.entries.size());
+	if (n == 0) return plan;
+	auto op_of = [&](uint32_t e) { return (d.entries[e].rec >> 24) & 0x3fu; };
+	auto operands = [&](uint32_t e, uint32_t (&c)[2]) -> uint32_t {
+		const uint32_t op = op_of(e);
+		if (op - OP_SPHERE <= OP_PLANE - OP_SPHERE) return 0;
+		c[0] = d.entries[e].l;
+		if (op == OP_FLATE || op == OP_SCALE_FIELD) return 1;
+		c[1] = d.entries[e].r;
+		return 2;
+	};
+	// Bottom up: an entry whose items (its own, its operands' uncut ones, one
+	// for each cut operand) would exceed a treelet cuts the larger operand, then
+	// the other.
+	std::vector<uint32_t> size(n, 1), stage(n, 0);
+	std::vector<uint8_t> cut(n, 0);
+	for (uint32_t e = 0; e < n; ++e)
+	{
+		uint32_t c[2] = { 0, 0 };
+		const uint32_t k = operands(e, c);
+		uint32_t total = 1;
+		for (uint32_t i = 0; i < k; ++i) total += size[c[i]];
+		for (uint32_t i = 0; i < k && total > kTreeletItems; ++i)
+		{
+			uint32_t which = 0;
+			if (k == 2 && (cut[c[0]] || (!cut[c[1]] && size[c[1]] > size[c[0]]))) which = 1;
+			const uint32_t x = c[which];
+			total -= size[x] - 1;
+			cut[x] = 1;
+			size[x] = 1;
+		}
+		size[e] = total;
+		for (uint32_t i = 0; i < k; ++i) stage[e] = std::max(stage[e], stage[c[i]] + (cut[c[i]] ? 1u : 0u));
+	}
+	cut[n - 1] = 1;
+	uint32_t stages = 0;
+	for (uint32_t e = 0; e < n; ++e)
+		if (cut[e]) stages = std::max(stages, stage[e] + 1);
+	// treelet roots by stage; their value slots in that order
+	std::vector<uint32_t> slot(n, 0xffffffffu), roots;
+	for (uint32_t s = 0; s < stages; ++s)
+	{
+		plan.stage_first.push_back(uint32_t(roots.size()));
+		for (uint32_t e = 0; e < n; ++e)
+			if (cut[e] && stage[e] == s) roots.push_back(e);
+	}
+	plan.stage_first.push_back(uint32_t(roots.size()));
+	for (uint32_t e : roots)
+		if (e + 1 != n) slot[e] = plan.slots++;
+	for (uint32_t root : roots)
+	{
+		// the root's items top down, then reversed into postfix order by entry
+		struct Node
+		{
+			uint32_t entry, parent, side, depth;  // parent: index into `nodes`
+		};
+		std::vector<Node> nodes{ { root, 0, 0, 1 } };
+		Treelet t{ uint32_t(plan.items.size()), 0, slot[root], 0 };
+		for (size_t i = 0; i < nodes.size(); ++i)
+		{
+			const Node x = nodes[i];
+			t.depth = std::max(t.depth, x.depth);
+			if (i > 0 && cut[x.entry]) continue;
+			uint32_t c[2] = { 0, 0 };
+			const uint32_t k = operands(x.entry, c);
+			for (uint32_t j = 0; j < k; ++j) nodes.push_back({ c[j], uint32_t(i), j, x.depth + 1 });
+		}
+		t.count = uint32_t(nodes.size());
+		// postfix order is the order of the source entries
+		std::vector<uint32_t> order(t.count), at(t.count);
+		for (uint32_t i = 0; i < t.count; ++i) order[i] = i;
+		std::sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return nodes[a].entry < nodes[b].entry; });
+		for (uint32_t i = 0; i < t.count; ++i) at[order[i]] = i;
+		for (uint32_t i = 0; i < t.count; ++i)
+		{
+			const Node& x = nodes[order[i]];
+			const bool load = order[i] != 0 && cut[x.entry];
+			plan.items.push_back({ load ? kItemLoad : d.entries[x.entry].rec, load ? slot[x.entry] : d.entries[x.entry].ord,
+			                       x.entry, at[x.parent] | (x.side << 8) });
+		}
+		plan.treelets.push_back(t);
+	}
+	return plan;
+}
+
 bool decode_words(const uint32_t* w, size_t n, DecodedProgram& out, std::string& err)
 {
 	out = DecodedProgram();

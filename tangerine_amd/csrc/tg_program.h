@@ -44,6 +44,39 @@ struct DecodedProgram
 	bool scene_finite = false;
 };
 
+// A program cut into treelets for the grid-wide pruning passes: subtrees of at
+// most kTreeletItems items, each run by one wave per group of cells.  An item
+// is an entry of the treelet, or stands for a smaller treelet's root (a cut).
+// Treelets are ordered by stage; a treelet's cuts belong to earlier stages.
+constexpr uint32_t kTreeletItems = 32;
+constexpr uint32_t kItemLoad = 33u << 24;  // op of a cut item: the root's value is loaded
+
+struct TreeletItem
+{
+	uint32_t rec;     // the entry's word, or kItemLoad
+	uint32_t index;   // binary entry: its ordinal; cut: the value slot of its treelet
+	uint32_t entry;   // source entry (cut: its treelet's root entry)
+	uint32_t parent;  // position of the parent's item in the treelet (root: itself) | 1 << 8 for a right operand
+};
+
+struct Treelet
+{
+	uint32_t first, count;  // its items, in postfix order
+	uint32_t slot;          // value slot of its root (~0: the program's root)
+	uint32_t depth;         // items on the longest path to its root
+};
+
+struct PrunePlan
+{
+	std::vector<TreeletItem> items;
+	std::vector<Treelet> treelets;      // by stage
+	std::vector<uint32_t> stage_first;  // first treelet of every stage, then their number
+	uint32_t slots = 0;                 // value slots
+	uint32_t stages() const { return stage_first.empty() ? 0u : uint32_t(stage_first.size()) - 1; }
+};
+
+PrunePlan prune_plan(const DecodedProgram& d);
+
 // Validates stack discipline and opcodes the way SDFInterpreter::Eval would
 // (tangerine/sdf_evaluator.cpp:1397-1600) and re-encodes the program.
 // Returns false with a message on malformed input.

@@ -22,38 +22,10 @@ namespace tg {
 
 namespace {
 
-constexpr uint32_t kMaxLevels = 64;                 // more heights: the in-kernel decision pass
-constexpr uint64_t kMaxValueBytes = 2ull << 30;    // entry values kept for the level-parallel pass
-
-// Entry positions ordered by height (leaves 0, a parent one above its highest
-// child) and the first position of every height.  Returns false when the
-// program has more than kMaxLevels heights.
-bool entry_levels(const DecodedProgram& d, std::vector<uint32_t>& order, std::vector<uint32_t>& first)
-{
-	const size_t n = d.entries.size();
-	std::vector<uint32_t> h(n, 0);
-	uint32_t top = 0;
-	for (size_t e = 0; e < n; ++e)
-	{
-		const HostEntry& x = d.entries[e];
-		const uint32_t op = entry_op(x.rec);
-		if (op - OP_SPHERE <= OP_PLANE - OP_SPHERE)
-			h[e] = 0;
-		else if (op == OP_FLATE || op == OP_SCALE_FIELD)
-			h[e] = h[x.l] + 1;
-		else
-			h[e] = std::max(h[x.l], h[x.r]) + 1;
-		top = std::max(top, h[e]);
-		if (top >= kMaxLevels) return false;
-	}
-	first.assign(top + 2, 0);
-	for (size_t e = 0; e < n; ++e) ++first[h[e] + 1];
-	for (uint32_t k = 1; k < first.size(); ++k) first[k] += first[k - 1];
-	order.assign(n, 0);
-	std::vector<uint32_t> at(first.begin(), first.end() - 1);
-	for (size_t e = 0; e < n; ++e) order[at[h[e]]++] = uint32_t(e);
-	return true;
-}
+// More stages than this (a chain of thousands of operators), or values beyond
+// this: the in-kernel decision pass, one wave walking the program per group.
+constexpr uint32_t kMaxStages = 32;
+constexpr uint64_t kMaxValueBytes = 2ull << 30;
 
 }  // namespace
 
@@ -63,7 +35,7 @@ constexpr uint64_t kColumnCells = 8192;
 
 namespace {
 
-// One emission pass (and, on the first, the level-parallel decision passes)
+// One emission pass (and, on the first, the treelet passes)
 // with the pool capacity out.state.capacity; the five counters are copied to
 // out.host (pinned) on `stream`.
 // Bytes of a pool entry.
@@ -93,18 +65,18 @@ PruneArgs prune_args(const tg_program* p, const float origin[3], const float cel
 	pa.scratch = out.scratch.as<uint64_t>();
 	pa.cells_per_wave = ps.cells_per_wave;
 	// masks, liveness and lengths stay in scratch for the rerun after a pool overflow
-	pa.masks_ready = ps.level_parallel ? 1 : 0;
+	pa.masks_ready = ps.treelets ? 1 : 0;
 	pa.counts = out.lens.as<const uint32_t>();
 	// emission only: four waves per cell group while that leaves under ~8
 	// waves per SIMD
-	pa.splits = (ps.level_parallel && ps.waves * 4 <= 8192) ? 4u : 1u;
+	pa.splits = (ps.treelets && ps.waves * 4 <= 8192) ? 4u : 1u;
 	// A wave per cell (a lane per entry) scans the whole program for every
 	// cell: it wins on grids of few cells, whose programs are long (the walk's
 	// time is the longest walk), and loses on many cells with short programs
 	// (4913 cells of 4095 entries 0.10 ms against the walk's 0.69, 35,937 cells
 	// of the same 0.39 against 0.41, 266,240 of 511 0.57 against 0.21).
 	const bool few = ps.ncells <= kColumnCells || (ps.ncells <= 2 * kColumnCells && d.entries.size() >= 1024);
-	pa.columns = (ps.level_parallel && (ps.words || out.emission == 2 || (out.emission == 0 && few))) ? 1 : 0;
+	pa.columns = (ps.treelets && (ps.words || out.emission == 2 || (out.emission == 0 && few))) ? 1 : 0;
 	pa.words = ps.words ? 1 : 0;
 	// One pool reservation (a device-wide atomic) for each workgroup's cells:
 	// large workgroups, and several cells to a wave once the waves fill the GPU
@@ -116,53 +88,44 @@ PruneArgs prune_args(const tg_program* p, const float origin[3], const float cel
 	return pa;
 }
 
-// Level-parallel pass arguments (without the height's list) of a prepared pruning.
-LevelArgs level_args(const PruneArgs& pa, const CellPrograms& out)
+// Treelet pass arguments (without the stage) of a prepared pruning.
+TreeletArgs treelet_args(const tg_program* p, const PruneArgs& pa, const CellPrograms& out)
 {
 	const PruneState& ps = out.state;
-	LevelArgs la{};
-	la.prog = pa.prog;
-	la.entries = pa.entries;
-	la.ngroups = uint32_t(ps.waves);
-	la.cells_per_wave = ps.cells_per_wave;
-	la.ox = pa.ox; la.oy = pa.oy; la.oz = pa.oz;
-	la.cx = pa.cx; la.cy = pa.cy; la.cz = pa.cz;
-	la.radius = ps.decide_radius;
-	la.nx = pa.nx; la.ny = pa.ny; la.nz = pa.nz;
-	la.values = out.values.as<float>();
-	la.scratch = pa.scratch;
-	la.n_binary = pa.n_binary;
-	la.n_entries = pa.n_entries;
-	la.counts = out.lens.as<uint32_t>();
-	return la;
+	TreeletArgs ta{};
+	ta.prog = pa.prog;
+	ta.items = p->items();
+	ta.treelets = p->treelets();
+	ta.ngroups = uint32_t(ps.waves);
+	ta.cells_per_wave = ps.cells_per_wave;
+	ta.ox = pa.ox; ta.oy = pa.oy; ta.oz = pa.oz;
+	ta.cx = pa.cx; ta.cy = pa.cy; ta.cz = pa.cz;
+	ta.radius = ps.decide_radius;
+	ta.nx = pa.nx; ta.ny = pa.ny; ta.nz = pa.nz;
+	ta.values = out.values.as<float>();
+	ta.scratch = pa.scratch;
+	ta.n_binary = pa.n_binary;
+	ta.n_entries = pa.n_entries;
+	ta.slots = pa.slots;
+	ta.counts = out.lens.as<uint32_t>();
+	return ta;
 }
 
-// Steps of the level-parallel pass: heights 1 .. H - 1 upward, then H - 1 ..
-// 1 downward (the parents count their leaf children), or, for a leaf root
-// (H = 1), the root's own liveness step.
-size_t level_steps(const PruneState& ps)
+// Launches of the treelet passes: the stages upward, the last of them (the
+// root's) in both directions, then the others downward.
+size_t treelet_steps(const tg_program* p) { return 2 * size_t(p->plan.stages()) - 1; }
+
+void treelet_step(TreeletArgs& ta, const PrunePlan& plan, size_t step)
 {
-	return ps.heights >= 2 ? 2 * ps.heights - 1 : 2 * ps.heights;
+	const size_t stages = plan.stages();
+	const size_t k = step < stages ? step : 2 * stages - 2 - step;
+	ta.first = plan.stage_first[k];
+	ta.count = plan.stage_first[k + 1] - ta.first;
+	ta.up = step < stages ? 1 : 0;
+	ta.down = step + 1 >= stages ? 1 : 0;
 }
 
-// Height step `step` (1 .. level_steps - 1) of the level-parallel pass: values
-// and decisions upward from height 1 (leaf operands are evaluated in place),
-// then liveness and lengths downward.
-void level_step(LevelArgs& la, const CellPrograms& out, size_t step)
-{
-	const PruneState& ps = out.state;
-	const size_t heights = ps.heights;
-	const size_t h = step < heights ? step : 2 * heights - 1 - step;
-	la.liveness = step < heights ? 0 : 1;
-	la.list = out.levels.as<const uint32_t>() + ps.level_first[h];
-	la.count = ps.level_first[h + 1] - ps.level_first[h];
-	// a few cell groups per wave while enough waves remain to fill the GPU
-	la.groups_per_wave = 1;
-	while (la.groups_per_wave < 8 && uint64_t(la.count) * ps.waves / (la.groups_per_wave * 2) >= 8192)
-		la.groups_per_wave *= 2;
-}
-
-// One emission pass (and, on the first, the level-parallel decision passes)
+// One emission pass (and, on the first, the treelet passes)
 // with the pool capacity out.state.capacity; the five counters are copied to
 // out.host (pinned) on `stream`.
 int prune_pass(hipStream_t stream, const tg_program* p, const float origin[3], const float cell[3],
@@ -175,16 +138,16 @@ int prune_pass(hipStream_t stream, const tg_program* p, const float origin[3], c
 	if (e != hipSuccess) return hip_fail(e, "prune counters");
 	const PruneArgs pa = prune_args(p, origin, cell, counts, out);
 	const uint64_t waves = ps.waves;
-	if (first && ps.level_parallel)
+	if (first && ps.treelets)
 	{
-		LevelArgs la = level_args(pa, out);
+		TreeletArgs ta = treelet_args(p, pa, out);
 		e = hipMemsetAsync(out.lens.ptr, 0, waves * 64 * 4, stream);
 		if (e != hipSuccess) return hip_fail(e, "length reset");
-		for (size_t step = 1; step < level_steps(ps); ++step)
+		for (size_t step = 0; step < treelet_steps(p); ++step)
 		{
-			level_step(la, out, step);
-			e = fast ? fast::launch_prune_level(la, stream) : exact::launch_prune_level(la, stream);
-			if (e != hipSuccess) return hip_fail(e, "level pruning launch");
+			treelet_step(ta, p->plan, step);
+			e = fast ? fast::launch_prune_treelets(ta, stream) : exact::launch_prune_treelets(ta, stream);
+			if (e != hipSuccess) return hip_fail(e, "treelet pruning launch");
 		}
 	}
 	e = fast ? fast::launch_prune_cells(pa, stream) : exact::launch_prune_cells(pa, stream);
@@ -243,29 +206,15 @@ int prune_prepare(hipStream_t stream, const tg_program* p, const float origin[3]
 	if (!rc) rc = out.counters.ensure(64);
 	if (!rc) rc = out.scratch.ensure(ps.waves * prune_scratch_words(d.binary_entries, uint32_t(d.entries.size())) * 8);
 	if (rc) return rc;
-	// Level-parallel decision pass when the heights are few and the entry
-	// values fit: it replaces the per-wave walk over the whole program.
-	std::vector<uint32_t>& level_order = ps.level_order;
-	ps.level_parallel = entry_levels(d, level_order, ps.level_first) &&
-	                    uint64_t(d.entries.size()) * ps.waves * 64 * 4 <= kMaxValueBytes;
-	if (words && !ps.level_parallel) return TG_OK;
-	if (ps.level_parallel)
+	// Grid-wide treelet passes when the stages are few and the treelets' values
+	// fit: they replace the per-wave walk over the whole program.
+	ps.treelets = treelet_prunable(p, ncells);
+	if (words && !ps.treelets) return TG_OK;
+	if (ps.treelets)
 	{
-		ps.heights = ps.level_first.size() - 1;
-		rc = out.values.ensure(uint64_t(d.entries.size()) * ps.waves * 64 * 4);
-		if (!rc) rc = out.levels.ensure(level_order.size() * 4);
+		rc = out.values.ensure(std::max<uint64_t>(uint64_t(p->plan.slots) * ps.waves * 64 * 4, 256));
 		if (!rc) rc = out.lens.ensure(ps.waves * 64 * 4);
 		if (rc) return rc;
-		// the entries by height depend on the program alone: uploaded once per
-		// program (and buffer)
-		if (out.levels_uid != p->uid || out.levels_bytes != out.levels.bytes)
-		{
-			hipError_t e = hipMemcpyAsync(out.levels.ptr, level_order.data(), level_order.size() * 4,
-				hipMemcpyHostToDevice, stream);
-			if (e != hipSuccess) return hip_fail(e, "level upload");
-			out.levels_uid = p->uid;
-			out.levels_bytes = out.levels.bytes;
-		}
 	}
 	// First guess: a quarter of the whole program per cell, at most 1 GiB; grown
 	// to the exact total and rerun if any cell did not fit (prune_cells_finish).
@@ -280,12 +229,12 @@ int prune_prepare(hipStream_t stream, const tg_program* p, const float origin[3]
 
 }  // namespace
 
-bool level_prunable(const tg_program* p, uint64_t ncells)
+bool treelet_prunable(const tg_program* p, uint64_t ncells)
 {
 	const DecodedProgram& d = p->decoded;
 	if (!d.prunable() || d.entries.empty() || d.entries.size() >= 65535 || ncells == 0 || ncells >= (1ull << 31)) return false;
-	std::vector<uint32_t> order, first;
-	return uint64_t(d.entries.size()) * ((ncells + 63) / 64) * 256 <= kMaxValueBytes && entry_levels(d, order, first);
+	// (16 cells to a group at the least)
+	return p->plan.stages() <= kMaxStages && uint64_t(p->plan.slots) * ((ncells + 15) / 16) * 256 <= kMaxValueBytes;
 }
 
 int prune_cells_start(hipStream_t stream, const tg_program* p, const float origin[3], const float cell[3],
@@ -312,21 +261,21 @@ int prune_cells_many(hipStream_t stream, const tg_program* const* progs, const C
 		int rc = prune_prepare(stream, progs[i], grids[i].origin, grids[i].cell, grids[i].radius, grids[i].counts,
 			*outs[i], grids[i].words, &r);
 		if (rc) return rc;
-		if (!r && grids[i].words) return fail(TG_ERR_LIMIT, "tile programs need the level-parallel pruning");
+		if (!r && grids[i].words) return fail(TG_ERR_LIMIT, "tile programs need the treelet passes");
 		if (!r) continue;
 		CellPrograms& out = *outs[i];
 		ready[i] = 1;
 		rc = out.pool.ensure(out.state.capacity * entry_bytes(out.state));
 		if (rc) return rc;
 		TG_CHECK_HIP(hipMemsetAsync(out.counters.ptr, 0, 64, stream), "prune counters");
-		if (out.state.level_parallel)
+		if (out.state.treelets)
 		{
 			TG_CHECK_HIP(hipMemsetAsync(out.lens.ptr, 0, out.state.waves * 64 * 4, stream), "length reset");
-			steps = std::max(steps, level_steps(out.state));
+			steps = std::max(steps, treelet_steps(progs[i]));
 		}
 		pas[i] = prune_args(progs[i], grids[i].origin, grids[i].cell, grids[i].counts, out);
 	}
-	// host blob: per height step, its level jobs then their wave bases; then
+	// host blob: per step, its treelet jobs then their wave bases; then
 	// the emission jobs and their block bases
 	std::vector<uint8_t>& blob = work.host;
 	blob.clear();
@@ -341,27 +290,32 @@ int prune_cells_many(hipStream_t stream, const tg_program* const* progs, const C
 		size_t jobs, bases;
 		uint32_t njobs, units;
 	};
-	std::vector<Launch> level_launches;
-	for (size_t step = 1; step < steps; ++step)
+	struct StageLaunch
 	{
-		std::vector<LevelArgs> jobs;
+		Launch l;
+		uint32_t slots;  // most spill slots of a job that runs upward
+	};
+	std::vector<StageLaunch> stage_launches;
+	for (size_t step = 0; step < steps; ++step)
+	{
+		std::vector<TreeletArgs> jobs;
 		std::vector<uint32_t> base;
-		uint32_t waves = 0;
+		uint32_t waves = 0, slots = 0;
 		for (uint32_t i = 0; i < n; ++i)
 		{
 			const CellPrograms& out = *outs[i];
-			if (!ready[i] || !out.state.level_parallel || step >= level_steps(out.state)) continue;
-			LevelArgs la = level_args(pas[i], out);
-			level_step(la, out, step);
-			const uint32_t per_entry = (la.ngroups + la.groups_per_wave - 1) / la.groups_per_wave;
+			if (!ready[i] || !out.state.treelets || step >= treelet_steps(progs[i])) continue;
+			TreeletArgs ta = treelet_args(progs[i], pas[i], out);
+			treelet_step(ta, progs[i]->plan, step);
 			base.push_back(waves);
-			waves += la.count * per_entry;
-			jobs.push_back(la);
+			waves += fast ? fast::treelet_waves(ta) : exact::treelet_waves(ta);
+			if (ta.up) slots = std::max(slots, ta.slots);
+			jobs.push_back(ta);
 		}
 		if (jobs.empty()) continue;
-		const size_t j = put(jobs.data(), jobs.size() * sizeof(LevelArgs));
+		const size_t j = put(jobs.data(), jobs.size() * sizeof(TreeletArgs));
 		const size_t b = put(base.data(), base.size() * 4);
-		level_launches.push_back(Launch{ j, b, uint32_t(jobs.size()), waves });
+		stage_launches.push_back(StageLaunch{ Launch{ j, b, uint32_t(jobs.size()), waves }, slots });
 	}
 	// emission jobs: the sequential walk's (a wave per group part) and the
 	// column emission's (a wave per cell), one launch each; `cells`: the
@@ -408,13 +362,15 @@ int prune_cells_many(hipStream_t stream, const tg_program* const* progs, const C
 			"pruning job upload");
 	}
 	const uint8_t* dev = work.dev.as<const uint8_t>();
-	for (const Launch& l : level_launches)
+	for (const StageLaunch& sl : stage_launches)
 	{
-		const LevelArgs* jobs = reinterpret_cast<const LevelArgs*>(dev + l.jobs);
+		const Launch& l = sl.l;
+		const TreeletArgs* jobs = reinterpret_cast<const TreeletArgs*>(dev + l.jobs);
 		const uint32_t* base = reinterpret_cast<const uint32_t*>(dev + l.bases);
-		const hipError_t e = fast ? fast::launch_prune_level_multi(jobs, base, l.njobs, l.units, stream)
-		                          : exact::launch_prune_level_multi(jobs, base, l.njobs, l.units, stream);
-		if (e != hipSuccess) return hip_fail(e, "level pruning launch");
+		const hipError_t e =
+			fast ? fast::launch_prune_treelets_multi(jobs, base, l.njobs, l.units, sl.slots, stream)
+			     : exact::launch_prune_treelets_multi(jobs, base, l.njobs, l.units, sl.slots, stream);
+		if (e != hipSuccess) return hip_fail(e, "treelet pruning launch");
 	}
 	if (!ejobs.empty())
 	{
