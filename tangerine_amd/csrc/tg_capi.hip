@@ -7,6 +7,7 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -75,6 +76,96 @@ int ensure_device()
 	}
 	ready = 1;
 	return TG_OK;
+}
+
+namespace {
+
+constexpr size_t kPoolSpaces = 4;
+constexpr size_t kPoolBytes = size_t(256) << 20;
+
+std::mutex g_pool_mutex;
+std::vector<Workspace*>& pool()
+{
+	// never destroyed: the device runtime may be gone before static destructors
+	static std::vector<Workspace*>* idle = new std::vector<Workspace*>;
+	return *idle;
+}
+
+}  // namespace
+
+size_t Workspace::bytes() const
+{
+	size_t n = in.bytes + out.bytes + queue.bytes + ctl.bytes + pinned_bytes;
+	for (const CellPrograms& l : levels)
+		n += l.pool.bytes + l.desc.bytes + l.counters.bytes + l.scratch.bytes + l.values.bytes + l.lens.bytes;
+	return n;
+}
+
+void Workspace::release()
+{
+	for (DevBuf* b : { &in, &out, &queue, &ctl }) b->release();
+	for (CellPrograms& l : levels) l.release();
+	if (pinned) (void)hipHostFree(pinned);
+	pinned = nullptr;
+	pinned_bytes = 0;
+}
+
+int WorkspaceLease::take()
+{
+	int dev = 0;
+	const hipError_t e = hipGetDevice(&dev);
+	if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
+	{
+		std::lock_guard<std::mutex> lock(g_pool_mutex);
+		std::vector<Workspace*>& idle = pool();
+		for (size_t i = 0; i < idle.size(); ++i)
+			if (idle[i]->device == dev)
+			{
+				ws_ = idle[i];
+				idle.erase(idle.begin() + std::ptrdiff_t(i));
+				return TG_OK;
+			}
+	}
+	ws_ = new Workspace;
+	ws_->device = dev;
+	return TG_OK;
+}
+
+int WorkspaceLease::pinned(size_t bytes)
+{
+	if (bytes <= ws_->pinned_bytes) return TG_OK;
+	if (ws_->pinned) (void)hipHostFree(ws_->pinned);
+	ws_->pinned = nullptr;
+	ws_->pinned_bytes = 0;
+	const size_t room = std::max(bytes, size_t(4096));
+	const hipError_t e = hipHostMalloc(&ws_->pinned, room, hipHostMallocDefault);
+	if (e != hipSuccess)
+	{
+		ws_->pinned = nullptr;
+		hipGetLastError();
+		return fail(TG_ERR_NOMEM, std::string("pinned staging: ") + hipGetErrorString(e));
+	}
+	ws_->pinned_bytes = room;
+	return TG_OK;
+}
+
+WorkspaceLease::~WorkspaceLease()
+{
+	if (!ws_) return;
+	if (ws_->bytes() <= kPoolBytes)
+	{
+		std::lock_guard<std::mutex> lock(g_pool_mutex);
+		std::vector<Workspace*>& idle = pool();
+		size_t mine = 0;
+		for (const Workspace* w : idle) mine += w->device == ws_->device ? 1 : 0;
+		if (mine < kPoolSpaces)
+		{
+			idle.push_back(ws_);
+			return;
+		}
+	}
+	ws_->release();
+	delete ws_;
 }
 
 }  // namespace tg

@@ -124,6 +124,40 @@ int prune_cells_finish(hipStream_t stream, const tg_program* p, const float orig
 	const uint32_t counts[3], bool fast, CellPrograms& out);
 }
 
+namespace tg {
+
+// Buffers of one host query (tg_eval_points, tg_gradient_points, tg_raymarch),
+// kept between calls.  A call leases a workspace of its device for its whole
+// length, so calls of several threads never share one; the pool keeps at most
+// kPoolSpaces idle ones per device, and none larger than kPoolBytes.
+struct Workspace
+{
+	int device = 0;
+	DevBuf in, out, queue, ctl;
+	CellPrograms levels[2];
+	void* pinned = nullptr;   // host staging, also addressed by kernels
+	size_t pinned_bytes = 0;
+	size_t bytes() const;
+	void release();
+};
+
+class WorkspaceLease
+{
+public:
+	WorkspaceLease() = default;
+	~WorkspaceLease();
+	WorkspaceLease(const WorkspaceLease&) = delete;
+	WorkspaceLease& operator=(const WorkspaceLease&) = delete;
+	int take();                       // a workspace of the current device
+	int pinned(size_t bytes);         // its staging, at least this large
+	Workspace* operator->() const { return ws_; }
+
+private:
+	Workspace* ws_ = nullptr;
+};
+
+}  // namespace tg
+
 struct tg_mesher;
 struct tg_surrogate;
 #include "tg_mlp.h"

@@ -67,9 +67,10 @@ PruneArgs prune_args(const tg_program* p, const float origin[3], const float cel
 	// masks, liveness and lengths stay in scratch for the rerun after a pool overflow
 	pa.masks_ready = ps.treelets ? 1 : 0;
 	pa.counts = out.lens.as<const uint32_t>();
-	// emission only: four waves per cell group while that leaves under ~8
-	// waves per SIMD
-	pa.splits = (ps.treelets && ps.waves * 4 <= 8192) ? 4u : 1u;
+	// the walk: four waves per cell group while that leaves under ~4 waves per
+	// SIMD (562 groups of 4095 entries: 395 us, one wave each 504; 1728 groups
+	// of 511 entries: 188 us, one wave each 85)
+	pa.splits = (ps.treelets && ps.waves * 4 <= 4096) ? 4u : 1u;
 	// A wave per cell (a lane per entry) scans the whole program for every
 	// cell: it wins on grids of few cells, whose programs are long (the walk's
 	// time is the longest walk), and loses on many cells with short programs
