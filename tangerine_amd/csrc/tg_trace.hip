@@ -41,10 +41,12 @@ struct Transform8
 // the cell they are in, at most kPassBudget steps, packed so that about
 // kResumeWaves waves run them (at most 64 rays, at least one to a wave): the
 // long marches of a frame no longer share a wave, where each waited on the
-// others' cell programs.  (1920x1080, 256 primitives: 10.6 ms in one pass,
-// 9.0 ms as 48 + 208 steps with the rays left one to a wave.)
-constexpr int kFirstBudget = 48;
-constexpr int kPassBudget = 208;
+// others' cell programs.  (1920x1080, 256 primitives: 10.6 ms in one pass;
+// two passes, the rays left one to a wave, two cameras: 64 + 192 steps 9.0 /
+// 10.2 ms, 48 + 208 8.0 / 9.4, 40 7.6 / 8.6, 32 7.1 / 7.8, 24 7.2 / 8.7, 16 7.2 /
+// 8.2.  Earlier than 32 the waves of single rays are more than run at once.)
+constexpr int kFirstBudget = 32;
+constexpr int kPassBudget = 224;
 constexpr uint32_t kResumeWaves = 65536;
 constexpr int kKeyBits = 27;  // trace_key: level above an 18-bit Morton code
 
@@ -66,8 +68,8 @@ struct tg_tracer
 
 namespace {
 
-// Cell hierarchy: an outer level of 8^3 cells over `outer` (the cube holding
-// the eye), then 8, 16, 32, 64 cells per axis over `inner` (the scene's cube,
+// Cell hierarchy: an outer level of 16^3 cells over `outer` (the cube holding
+// the eye), then 16 and 64 cells per axis over `inner` (the scene's cube,
 // where rays spend their steps).  Each level is a cube (lowest corner, edge).
 struct CubeDomain
 {
@@ -313,6 +315,9 @@ extern "C" int tg_tracer_render(tg_tracer* tr, const tg_program* p, const tg_cam
 		}
 		// far cube (rays leaving the scene march on through few, small cell
 		// programs), the eye's cube, then 16^3 and 64^3 cells over the scene.
+		// (Far / eye's cells at 1080p, 256 primitives, pruning + marching: 8/8
+		// 7.60 ms, 8/16 7.36, 8/32 7.46, 8/48 7.39, 16/32 7.45; 512 primitives
+		// 16.16, 16.15, 16.55, 16.67; 16 primitives 1.40, 1.42, 1.45, 1.42.)
 		// (1080p, 256 primitives, pruning + marching: 8/16/32/64 levels over
 		// the scene 11.2 ms, 16/64 10.7, 32/64 10.6, 64 alone 10.5, 48/96 12.3:
 		// the waterfall over per-ray cells makes the middle levels cheap to drop.)
@@ -325,7 +330,7 @@ extern "C" int tg_tracer_render(tg_tracer* tr, const tg_program* p, const tg_cam
 			ns[count++] = 8;
 		}
 		doms[count] = outer;
-		ns[count++] = 8;
+		ns[count++] = 16;
 		for (uint32_t n : { 16u, 64u })
 		{
 			doms[count] = inner;
