@@ -54,11 +54,9 @@ struct TrainArgs
 	const float* xyz;         // training points
 	const float* target;      // exact distances
 	const uint32_t* order;    // sample permutation
-	uint64_t batch_offset;    // first sample of the batch in `order` (or a device counter)
-	const uint64_t* batch_counter;  // if set: batch index -> offset = (*counter % batches) * batch
-	uint32_t batches;
+	uint64_t batch_offset;    // first sample of the batch in `order`
 	uint32_t batch;           // samples per batch (multiple of 32)
-	uint32_t groups_per_block;
+	uint32_t groups_per_block;  // 1 or 2
 	float* partial;           // [blocks][kParams] gradients of the mean squared error
 	float* loss_partial;      // [blocks] sum of squared errors
 };
@@ -71,7 +69,8 @@ struct AdamArgs
 	const float* partial;     // [blocks][kParams]
 	const float* loss_partial;
 	uint32_t blocks;
-	uint64_t* step;           // device step counter (incremented by the step kernel)
+	const uint64_t* epoch;    // device counter: step = epoch * batches + batch_index
+	uint32_t batches, batch_index;
 	float lr, beta1, beta2, eps;
 	uint32_t decay_steps;     // cosine decay of lr to 5% over this many steps
 	float* loss_log;          // [steps] mean loss per step (or null)
@@ -85,7 +84,7 @@ hipError_t prepare();
 hipError_t launch_predict(const PredictArgs& a, hipStream_t s);
 hipError_t launch_train_grad(const TrainArgs& a, uint32_t blocks, hipStream_t s);
 hipError_t launch_adam(const AdamArgs& a, hipStream_t s);
-hipError_t launch_step_advance(uint64_t* step, uint64_t* batch_counter, hipStream_t s);
+hipError_t launch_epoch_advance(uint64_t* epoch, hipStream_t s);
 
 }  // namespace mlp
 }  // namespace tg

@@ -302,7 +302,6 @@ extern "C" int tg_surrogate_gradients(tg_surrogate* s, const float* xyz, const f
 	ta.order = dord.as<const uint32_t>();
 	ta.batch_offset = 0;
 	ta.batch = uint32_t(n);
-	ta.batches = 1;
 	ta.groups_per_block = 1;
 	ta.partial = dpart.as<float>();
 	ta.loss_partial = dloss.as<float>();
@@ -330,7 +329,7 @@ extern "C" int tg_surrogate_fit(tg_surrogate* s, const tg_program* exact, uint64
 	float surface_sigma, uint32_t epochs, uint32_t flags, tg_surrogate_stats* stats)
 {
 	if (!s || !exact) return fail(TG_ERR_INVALID, "tg_surrogate_fit: null argument");
-	// two waves per workgroup, a group of 32 points each: 256 workgroups
+	// two groups of 32 points per workgroup: 256 workgroups
 	const uint32_t batch = 16384, groups_per_block = 2;
 	const uint32_t blocks = batch / (mlp::kGroup * groups_per_block);
 	const uint64_t batches = samples / batch;
@@ -362,19 +361,17 @@ extern "C" int tg_surrogate_fit(tg_surrogate* s, const tg_program* exact, uint64
 	rc = tg_eval_points_device(exact, s->xyz.as<const float>(), n_all, s->target.as<float>(), flags & TG_FLAG_FAST,
 		s->stream);
 	if (rc) return rc;
+	// 3. training: one permutation (drawn while the device samples), batches in
+	// order, Adam; one epoch captured as a graph
+	std::vector<uint32_t> ord(n_train);
+	std::iota(ord.begin(), ord.end(), 0u);
+	std::mt19937_64 rng(s->seed ^ 0x5eedull);
+	std::shuffle(ord.begin(), ord.end(), rng);
 	TG_CHECK_HIP(hipStreamSynchronize(s->stream), "sampling");
 	auto t1 = std::chrono::steady_clock::now();
-
-	// 3. training: one permutation, batches in order, Adam; one epoch captured as a graph
-	{
-		std::vector<uint32_t> ord(n_train);
-		std::iota(ord.begin(), ord.end(), 0u);
-		std::mt19937_64 rng(s->seed ^ 0x5eedull);
-		std::shuffle(ord.begin(), ord.end(), rng);
-		rc = s->order.ensure(n_train * 4);
-		if (rc) return rc;
-		TG_CHECK_HIP(hipMemcpy(s->order.ptr, ord.data(), n_train * 4, hipMemcpyHostToDevice), "order upload");
-	}
+	rc = s->order.ensure(n_train * 4);
+	if (rc) return rc;
+	TG_CHECK_HIP(hipMemcpy(s->order.ptr, ord.data(), n_train * 4, hipMemcpyHostToDevice), "order upload");
 	const uint64_t total_steps = batches * epochs;
 	rc = s->partial.ensure(size_t(blocks) * mlp::kParams * 4);
 	if (!rc) rc = s->loss_partial.ensure(blocks * 4);
@@ -384,15 +381,12 @@ extern "C" int tg_surrogate_fit(tg_surrogate* s, const tg_program* exact, uint64
 	TG_CHECK_HIP(hipMemset(s->counters.ptr, 0, 64), "counter reset");
 	TG_CHECK_HIP(hipMemset(s->adam_m.ptr, 0, mlp::kParams * 4), "adam reset");
 	TG_CHECK_HIP(hipMemset(s->adam_v.ptr, 0, mlp::kParams * 4), "adam reset");
-	uint64_t* step = s->counters.as<uint64_t>();
-	uint64_t* batch_counter = step + 1;
+	uint64_t* epoch = s->counters.as<uint64_t>();
 	mlp::TrainArgs ta{};
 	ta.net = surrogate_net(s);
 	ta.xyz = s->xyz.as<const float>();
 	ta.target = s->target.as<const float>();
 	ta.order = s->order.as<const uint32_t>();
-	ta.batch_counter = batch_counter;
-	ta.batches = uint32_t(batches);
 	ta.batch = batch;
 	ta.groups_per_block = groups_per_block;
 	ta.partial = s->partial.as<float>();
@@ -404,7 +398,8 @@ extern "C" int tg_surrogate_fit(tg_surrogate* s, const tg_program* exact, uint64
 	aa.partial = s->partial.as<const float>();
 	aa.loss_partial = s->loss_partial.as<const float>();
 	aa.blocks = blocks;
-	aa.step = step;
+	aa.epoch = epoch;
+	aa.batches = uint32_t(batches);
 	aa.lr = 2e-3f;
 	aa.beta1 = 0.9f;
 	aa.beta2 = 0.999f;
@@ -420,10 +415,12 @@ extern "C" int tg_surrogate_fit(tg_surrogate* s, const tg_program* exact, uint64
 	hipError_t ce = hipSuccess;
 	for (uint64_t b = 0; b < batches && ce == hipSuccess; ++b)
 	{
+		ta.batch_offset = b * batch;
+		aa.batch_index = uint32_t(b);
 		ce = mlp::launch_train_grad(ta, blocks, s->stream);
 		if (ce == hipSuccess) ce = mlp::launch_adam(aa, s->stream);
-		if (ce == hipSuccess) ce = mlp::launch_step_advance(step, batch_counter, s->stream);
 	}
+	if (ce == hipSuccess) ce = mlp::launch_epoch_advance(epoch, s->stream);
 	hipError_t ee = hipStreamEndCapture(s->stream, &graph);
 	if (ce != hipSuccess) return hip_fail(ce, "training capture");
 	if (ee != hipSuccess) return hip_fail(ee, "capture end");
