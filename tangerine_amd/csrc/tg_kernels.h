@@ -341,6 +341,12 @@ struct CloudArgs
 	uint64_t npoints;
 	int iterations;            // refinement steps
 	uint32_t slots;
+	// one program per 8^3 cells (PruneArgs::words), or desc null
+	const uint32_t* words;
+	const BlockDesc* desc;
+	uint32_t tx, ty, tz;       // tiles per axis
+	uint32_t parts;            // select: waves per tile (2, 4 or 8)
+	float reach;               // a tile's program holds within this of the tile's centre
 };
 
 // VoxExport's voxel selection: cell (x, y, z) of a size[0] x size[1] x size[2]
@@ -409,7 +415,7 @@ hipError_t launch_eval_tile_programs_multi(const TileEvalArgs* jobs, const uint3
 	uint32_t blocks, size_t lds_per_wave, hipStream_t s);
 hipError_t launch_vox(const VoxArgs& a, int stage, hipStream_t s);  // 0 select, 1 list
 hipError_t launch_pivot(const PivotArgs& a, hipStream_t s);
-hipError_t launch_cloud(const CloudArgs& a, int stage, hipStream_t s);  // 0 select, 1 points, 2 refine
+hipError_t launch_cloud(const CloudArgs& a, int stage, hipStream_t s);  // 0 select, 1 points, 2 refine (with desc: both)
 hipError_t launch_batch(const BatchArgs& b, int p, uint32_t waves, uint32_t workgroups, hipStream_t s);
 hipError_t launch_batch_reset(unsigned int* head, unsigned long long* work, uint32_t nwork, hipStream_t s);
 hipError_t launch_certify(const CertifyArgs& a, hipStream_t s);
@@ -446,7 +452,7 @@ hipError_t launch_eval_tile_programs_multi(const TileEvalArgs* jobs, const uint3
 	uint32_t blocks, size_t lds_per_wave, hipStream_t s);
 hipError_t launch_vox(const VoxArgs& a, int stage, hipStream_t s);  // 0 select, 1 list
 hipError_t launch_pivot(const PivotArgs& a, hipStream_t s);
-hipError_t launch_cloud(const CloudArgs& a, int stage, hipStream_t s);  // 0 select, 1 points, 2 refine
+hipError_t launch_cloud(const CloudArgs& a, int stage, hipStream_t s);  // 0 select, 1 points, 2 refine (with desc: both)
 hipError_t launch_batch(const BatchArgs& b, int p, uint32_t waves, uint32_t workgroups, hipStream_t s);
 hipError_t launch_batch_reset(unsigned int* head, unsigned long long* work, uint32_t nwork, hipStream_t s);
 hipError_t launch_certify(const CertifyArgs& a, hipStream_t s);
