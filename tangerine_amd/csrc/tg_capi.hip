@@ -480,6 +480,50 @@ extern "C" void tg_program_destroy(tg_program* p)
 // ---------------------------------------------------------------------------
 // point queries
 
+bool tg::split_program(const tg_program* p, SplitProgram& out)
+{
+	const DecodedProgram& d = p->decoded;
+	const PrunePlan& plan = p->plan;
+	out = SplitProgram{};
+	out.slots = std::max<uint32_t>(1, d.max_stack - 1);
+	if (plan.stages() < 2 || plan.stages() > kSplitStages ||
+		split_lds_bytes(plan.slots, out.slots, kSplitWaves) > kSplitMaxLds)
+		return false;
+	out.prog = static_cast<const Instr*>(p->device.ptr);
+	out.items = p->items();
+	out.treelets = p->treelets();
+	out.records = uint32_t(d.entries.size());
+	out.stages = plan.stages();
+	for (uint32_t s = 0; s <= out.stages; ++s) out.stage_first[s] = plan.stage_first[s];
+	out.value_slots = plan.slots;
+	return true;
+}
+
+namespace {
+
+// Field evaluations up to which a workgroup shares 64 of them (SplitProgram):
+// while they leave the GPU idle, an evaluation's latency is the call's.  (Whole
+// program in one wave / split, us: 256 primitives 16384 evaluations 149 / 20, 131072
+// 150 / 89, 262144 158 / 163; 2048 primitives 131072 1170 / 552; 64 primitives 131072
+// 39 / 24; 24 primitives 16384 16 / 15, 131072 16 / 18.)
+uint64_t split_evaluations(const tg_program* p) { return p->decoded.entries.size() >= 96 ? 131072 : 32768; }
+
+}  // namespace
+
+int tg::launch_gradients(const tg_program* p, const GradArgs& a, uint32_t flags, hipStream_t stream)
+{
+	const bool fast = (flags & TG_FLAG_FAST) != 0;
+	SplitProgram sp;
+	hipError_t e;
+	// (four taps to a point and k_gradient a lane to a tap: half the evaluations;
+	// 256 primitives 16384 points 210 / 105 us, 65536 276 / 275, 512 primitives 437 / 579)
+	if (a.count <= split_evaluations(p) / 8 && split_program(p, sp))
+		e = fast ? fast::launch_gradient_split(a, sp, stream) : exact::launch_gradient_split(a, sp, stream);
+	else
+		e = fast ? fast::launch_gradient(a, stream) : exact::launch_gradient(a, stream);
+	return e == hipSuccess ? TG_OK : hip_fail(e, "gradient launch");
+}
+
 extern "C" int tg_eval_points_device(const tg_program* p, const float* xyz, uint64_t n, float* out, uint32_t flags,
 	void* stream)
 {
@@ -492,7 +536,13 @@ extern "C" int tg_eval_points_device(const tg_program* p, const float* xyz, uint
 	a.count = n;
 	a.slots = std::max<uint32_t>(1, p->decoded.max_stack - 1);
 	hipStream_t s = static_cast<hipStream_t>(stream);
-	hipError_t e = (flags & TG_FLAG_FAST) ? fast::launch_points(a, s) : exact::launch_points(a, s);
+	const bool fast = (flags & TG_FLAG_FAST) != 0;
+	SplitProgram sp;
+	hipError_t e;
+	if (n <= split_evaluations(p) && split_program(p, sp))
+		e = fast ? fast::launch_points_split(a, sp, s) : exact::launch_points_split(a, sp, s);
+	else
+		e = fast ? fast::launch_points(a, s) : exact::launch_points(a, s);
 	if (e != hipSuccess) return hip_fail(e, "eval points launch");
 	return TG_OK;
 }

@@ -91,6 +91,14 @@ struct CellPrograms
 int prune_cells(hipStream_t stream, const tg_program* p, const float origin[3], const float cell[3], float radius,
 	const uint32_t counts[3], bool fast, CellPrograms& out);
 
+struct GradArgs;
+struct SplitProgram;
+// `p` split over a workgroup; false where it is not (one treelet, too many
+// stages, LDS).
+bool split_program(const tg_program* p, SplitProgram& out);
+// The gradients of `a` (prog, slots: p's) on `stream`.
+int launch_gradients(const tg_program* p, const GradArgs& a, uint32_t flags, hipStream_t stream);
+
 // Whether `p` can be pruned over ncells cells by the treelet passes.
 bool treelet_prunable(const tg_program* p, uint64_t ncells);
 

@@ -1300,8 +1300,8 @@ int gradients_at(tg_mesher* m, const tg_program* p, const float* dev_xyz, uint64
 	ga.h = 1.0e-4f;
 	ga.tetra = 1;
 	ga.slots = std::max<uint32_t>(1, p->decoded.max_stack - 1);
-	hipError_t e = (flags & TG_FLAG_FAST) ? fast::launch_gradient(ga, m->stream) : exact::launch_gradient(ga, m->stream);
-	if (e != hipSuccess) return hip_fail(e, "gradient launch");
+	rc = launch_gradients(p, ga, flags, m->stream);
+	if (rc) return rc;
 	TG_CHECK_HIP(hipMemcpyAsync(out.data(), dout.ptr, n * 12, hipMemcpyDeviceToHost, m->stream), "normal download");
 	TG_CHECK_HIP(hipStreamSynchronize(m->stream), "normals");
 	return TG_OK;

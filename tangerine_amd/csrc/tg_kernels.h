@@ -303,26 +303,34 @@ struct TraceArgs
 	uint32_t* q_out_count;
 };
 
+// A whole program split over a workgroup: the waves run its treelets, stage by
+// stage, at 64 points (lane = point).
+constexpr uint32_t kSplitStages = 32, kSplitWaves = 16;
+struct SplitProgram
+{
+	const Instr* prog;
+	const TreeletItem* items;
+	const Treelet* treelets;
+	uint32_t records;         // of the program (one per entry)
+	uint32_t stage_first[kSplitStages + 1];
+	uint32_t stages;          // at least 2
+	uint32_t value_slots;     // LDS floats x 64 for the treelets' values
+	uint32_t slots;           // LDS spill slots per wave
+};
+constexpr size_t kSplitMaxLds = 160 * 1024 - 2048;  // beside the kernels' static LDS
+inline size_t split_lds_bytes(uint32_t value_slots, uint32_t slots, uint32_t waves)
+{
+	return size_t(value_slots) * 256 + waves * spill_bytes_per_wave(slots, 1);
+}
+
 // Rays from arrays marched through cell programs (k_march), then the rays that
-// left every level's cube with the whole program (k_march_far): a workgroup
-// to 64 of them, its waves running the program's treelets.
-constexpr uint32_t kFarStages = 32, kFarWaves = 16;
+// left every level's cube with the whole program (k_march_far), split.
 struct FarArgs
 {
 	TraceArgs t;              // q_in, q_count: the rays; outputs
 	const uint32_t* count;    // device word holding q_count (the host does not wait for it)
-	const TreeletItem* items;
-	const Treelet* treelets;
-	uint32_t stage_first[kFarStages + 1];
-	uint32_t stages;
-	uint32_t value_slots;     // LDS floats x 64 for the treelets' values
-	uint32_t slots;           // LDS spill slots per wave
+	SplitProgram split;
 };
-constexpr size_t kFarMaxLds = 160 * 1024 - 2048;  // beside the kernel's static LDS
-inline size_t far_lds_bytes(uint32_t value_slots, uint32_t slots, uint32_t waves)
-{
-	return size_t(value_slots) * 256 + waves * spill_bytes_per_wave(slots, 1);
-}
 
 // Point-cloud export: cells of a regular point grid kept near the surface,
 // then refined along the gradient.
@@ -427,6 +435,8 @@ hipError_t launch_trace(const TraceArgs& a, hipStream_t s);
 hipError_t launch_trace_resume(const TraceArgs& a, hipStream_t s);
 hipError_t launch_march(const TraceArgs& a, hipStream_t s);
 hipError_t launch_march_far(const FarArgs& a, uint32_t max_rays, hipStream_t s);
+hipError_t launch_points_split(const PointArgs& a, const SplitProgram& p, hipStream_t s);
+hipError_t launch_gradient_split(const GradArgs& a, const SplitProgram& p, hipStream_t s);
 hipError_t launch_gradient(const GradArgs& a, hipStream_t s);
 // all 2^32 float inputs of the exact build's square root against sqrtf
 hipError_t launch_sqrt_check(uint32_t scramble, unsigned long long* mismatches, hipStream_t s);
@@ -464,6 +474,8 @@ hipError_t launch_trace(const TraceArgs& a, hipStream_t s);
 hipError_t launch_trace_resume(const TraceArgs& a, hipStream_t s);
 hipError_t launch_march(const TraceArgs& a, hipStream_t s);
 hipError_t launch_march_far(const FarArgs& a, uint32_t max_rays, hipStream_t s);
+hipError_t launch_points_split(const PointArgs& a, const SplitProgram& p, hipStream_t s);
+hipError_t launch_gradient_split(const GradArgs& a, const SplitProgram& p, hipStream_t s);
 hipError_t launch_gradient(const GradArgs& a, hipStream_t s);
 }
 

@@ -471,9 +471,7 @@ constexpr size_t kRayEntries = 112;
 int ray_cubes(const tg_program* p, const float* starts, uint64_t count, CubeDomain* doms, uint32_t* ns)
 {
 	const DecodedProgram& d = p->decoded;
-	if (d.entries.size() < kRayEntries || p->plan.stages() > kFarStages || !treelet_prunable(p, 64 * 64 * 64) ||
-		far_lds_bytes(p->plan.slots, std::max<uint32_t>(1, d.max_stack - 1), kFarWaves) > kFarMaxLds)
-		return 0;
+	if (d.entries.size() < kRayEntries || !treelet_prunable(p, 64 * 64 * 64)) return 0;
 	float reach = 1.0f, scene = 0.0f;
 	for (uint64_t i = 0; i < 3 * count; ++i)
 	{
@@ -567,7 +565,8 @@ extern "C" int tg_raymarch(const tg_program* p, const float* starts, const float
 	uint8_t* dh = reinterpret_cast<uint8_t*>(dp + 3 * count);
 	CubeDomain doms[2];
 	uint32_t ns[2];
-	const int cubes = max_steps > 0 ? ray_cubes(p, starts, count, doms, ns) : 0;
+	FarArgs fa{};
+	const int cubes = max_steps > 0 && split_program(p, fa.split) ? ray_cubes(p, starts, count, doms, ns) : 0;
 	if (cubes == 0)
 		return raymarch_staged(p, starts, dirs, count, max_steps, eps, far_distance, flags, hit, travel, position, ds, dd,
 			dt, dp, dh);
@@ -578,7 +577,6 @@ extern "C" int tg_raymarch(const tg_program* p, const float* starts, const float
 	TG_CHECK_HIP(hipMemcpyAsync(ds, starts, count * 12, hipMemcpyHostToDevice, nullptr), "ray upload");
 	TG_CHECK_HIP(hipMemcpyAsync(dd, dirs, count * 12, hipMemcpyHostToDevice, nullptr), "ray upload");
 	TG_CHECK_HIP(hipMemsetAsync(ws->ctl.ptr, 0, 256, nullptr), "ray queue reset");
-	FarArgs fa{};
 	TraceArgs& ta = fa.t;
 	base_args(ta, p);
 	rc = build_levels(nullptr, p, doms, ns, cubes, fast, ws->levels, ta);
@@ -596,15 +594,8 @@ extern "C" int tg_raymarch(const tg_program* p, const float* starts, const float
 	ta.q_out_count = ws->ctl.as<uint32_t>();
 	hipError_t e = fast ? fast::launch_march(ta, nullptr) : exact::launch_march(ta, nullptr);
 	if (e != hipSuccess) return hip_fail(e, "raymarch launch");
-	const PrunePlan& plan = p->plan;
 	ta.q_in = ws->queue.as<const TraceRay>();
 	fa.count = ws->ctl.as<const uint32_t>();
-	fa.items = p->items();
-	fa.treelets = p->treelets();
-	fa.stages = plan.stages();
-	for (uint32_t s = 0; s <= fa.stages; ++s) fa.stage_first[s] = plan.stage_first[s];
-	fa.value_slots = plan.slots;
-	fa.slots = ta.slots;
 	e = fast ? fast::launch_march_far(fa, uint32_t(count), nullptr) : exact::launch_march_far(fa, uint32_t(count), nullptr);
 	if (e != hipSuccess) return hip_fail(e, "raymarch launch");
 	TG_CHECK_HIP(hipMemcpy(travel, dt, count * 4, hipMemcpyDeviceToHost), "travel download");
@@ -656,8 +647,8 @@ extern "C" int tg_gradient_points(const tg_program* p, const float* xyz, uint64_
 	ga.h = h;
 	ga.tetra = mode == 0 ? 1 : 0;
 	ga.slots = std::max<uint32_t>(1, p->decoded.max_stack - 1);
-	hipError_t e = (flags & TG_FLAG_FAST) ? fast::launch_gradient(ga, nullptr) : exact::launch_gradient(ga, nullptr);
-	if (e != hipSuccess) return hip_fail(e, "gradient launch");
+	rc = launch_gradients(p, ga, flags, nullptr);
+	if (rc) return rc;
 	TG_CHECK_HIP(hipMemcpy(out, dout.ptr, count * 12, hipMemcpyDeviceToHost), "gradient download");
 	return TG_OK;
 }
