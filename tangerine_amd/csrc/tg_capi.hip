@@ -149,6 +149,53 @@ int WorkspaceLease::pinned(size_t bytes)
 	return TG_OK;
 }
 
+namespace {
+
+// Queries whose points and results are within this are read and written by the
+// kernel in pinned memory, which is faster than a copy each way at every size
+// measured (3 primitives, whole call, device buffers / pinned: 1 point 28 / 18 us,
+// 4000 52 / 19, 40000 58 / 36, 400000 258 / 238; 100000 gradients of 256 primitives
+// 373 / 335).  The bound is for the pinned memory an idle workspace keeps.
+constexpr size_t kDirectBytes = size_t(16) << 20;
+
+}  // namespace
+
+int WorkspaceLease::stage(const float* host_xyz, uint64_t count, uint32_t width, const float** xyz, float** out)
+{
+	const uint64_t bytes = count * (12 + 4 * width);
+	size_t room = 65536;
+	while (room < bytes && room < kDirectBytes) room *= 2;
+	direct_ = bytes <= kDirectBytes && pinned(room) == TG_OK;
+	if (direct_)
+	{
+		std::memcpy(ws_->pinned, host_xyz, count * 12);
+		*xyz = static_cast<const float*>(ws_->pinned);
+		*out = static_cast<float*>(ws_->pinned) + 3 * count;
+		return TG_OK;
+	}
+	int rc = ws_->in.ensure(count * 12);
+	if (!rc) rc = ws_->out.ensure(count * 4 * width);
+	if (rc) return rc;
+	const hipError_t e = hipMemcpy(ws_->in.ptr, host_xyz, count * 12, hipMemcpyHostToDevice);
+	if (e != hipSuccess) return hip_fail(e, "points upload");
+	*xyz = ws_->in.as<const float>();
+	*out = ws_->out.as<float>();
+	return TG_OK;
+}
+
+int WorkspaceLease::collect(float* host_out, uint64_t count, uint32_t width)
+{
+	hipError_t e;
+	if (direct_)
+	{
+		e = hipStreamSynchronize(nullptr);
+		if (e == hipSuccess) std::memcpy(host_out, static_cast<const float*>(ws_->pinned) + 3 * count, count * 4 * width);
+	}
+	else
+		e = hipMemcpy(host_out, ws_->out.ptr, count * 4 * width, hipMemcpyDeviceToHost);
+	return e == hipSuccess ? TG_OK : hip_fail(e, "results download");
+}
+
 WorkspaceLease::~WorkspaceLease()
 {
 	if (!ws_) return;
@@ -583,14 +630,12 @@ extern "C" int tg_eval_points(const tg_program* p, const float* xyz, uint64_t n,
 {
 	if (!p || (n && (!xyz || !out))) return fail(TG_ERR_INVALID, "tg_eval_points: null argument");
 	if (n == 0) return TG_OK;
-	DevBuf din, dout;
-	int rc = din.ensure(n * 12);
-	if (!rc) rc = dout.ensure(n * 4);
-	if (rc) return rc;
-	struct Guard { DevBuf& a; DevBuf& b; ~Guard() { a.release(); b.release(); } } g{ din, dout };
-	TG_CHECK_HIP(hipMemcpy(din.ptr, xyz, n * 12, hipMemcpyHostToDevice), "points upload");
-	rc = tg_eval_points_device(p, static_cast<const float*>(din.ptr), n, static_cast<float*>(dout.ptr), flags, nullptr);
-	if (rc) return rc;
-	TG_CHECK_HIP(hipMemcpy(out, dout.ptr, n * 4, hipMemcpyDeviceToHost), "points download");
-	return TG_OK;
+	WorkspaceLease ws;
+	const float* in = nullptr;
+	float* res = nullptr;
+	int rc = ws.take();
+	if (!rc) rc = ws.stage(xyz, n, 1, &in, &res);
+	if (!rc) rc = tg_eval_points_device(p, in, n, res, flags, nullptr);
+	if (!rc) rc = ws.collect(out, n, 1);
+	return rc;
 }

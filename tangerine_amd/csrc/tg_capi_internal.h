@@ -158,10 +158,17 @@ public:
 	WorkspaceLease& operator=(const WorkspaceLease&) = delete;
 	int take();                       // a workspace of the current device
 	int pinned(size_t bytes);         // its staging, at least this large
+	// `count` points for a kernel to read at `xyz` and `width` floats each for it
+	// to write at `out`: the pinned staging itself for few points, else device
+	// buffers (stage copies the points there, on the default stream).
+	int stage(const float* host_xyz, uint64_t count, uint32_t width, const float** xyz, float** out);
+	// Waits for the default stream's kernel and copies the staged results out.
+	int collect(float* host_out, uint64_t count, uint32_t width);
 	Workspace* operator->() const { return ws_; }
 
 private:
 	Workspace* ws_ = nullptr;
+	bool direct_ = false;             // staged in pinned memory
 };
 
 }  // namespace tg

@@ -633,24 +633,19 @@ extern "C" int tg_gradient_points(const tg_program* p, const float* xyz, uint64_
 	if (count == 0) return TG_OK;
 	int rc = ensure_device();
 	if (rc) return rc;
-	DevBuf din, dout;
-	struct Guard { DevBuf* b[2]; ~Guard() { for (DevBuf* x : b) x->release(); } } guard{ { &din, &dout } };
-	rc = din.ensure(count * 12);
-	if (!rc) rc = dout.ensure(count * 12);
-	if (rc) return rc;
-	TG_CHECK_HIP(hipMemcpy(din.ptr, xyz, count * 12, hipMemcpyHostToDevice), "points upload");
 	GradArgs ga{};
+	WorkspaceLease ws;
+	rc = ws.take();
+	if (!rc) rc = ws.stage(xyz, count, 3, &ga.xyz, &ga.out);
+	if (rc) return rc;
 	ga.prog = static_cast<const Instr*>(p->device.ptr);
-	ga.xyz = din.as<const float>();
-	ga.out = dout.as<float>();
 	ga.count = count;
 	ga.h = h;
 	ga.tetra = mode == 0 ? 1 : 0;
 	ga.slots = std::max<uint32_t>(1, p->decoded.max_stack - 1);
 	rc = launch_gradients(p, ga, flags, nullptr);
-	if (rc) return rc;
-	TG_CHECK_HIP(hipMemcpy(out, dout.ptr, count * 12, hipMemcpyDeviceToHost), "gradient download");
-	return TG_OK;
+	if (!rc) rc = ws.collect(out, count, 3);
+	return rc;
 }
 
 // ---- Lua queries: pivot_towards and mouse picking --------------------------------
