@@ -141,8 +141,12 @@ namespace tg {
 struct Workspace
 {
 	int device = 0;
+	hipEvent_t busy = nullptr;  // the work still reading it, of a call that returned before its end
+	bool in_flight = false;
 	DevBuf in, out, queue, ctl;
 	CellPrograms levels[2];
+	PruneLaunches launches;
+	std::vector<std::vector<uint8_t>> retired;  // job tables of work that may still read them
 	void* pinned = nullptr;   // host staging, also addressed by kernels
 	size_t pinned_bytes = 0;
 	size_t bytes() const;
@@ -156,7 +160,11 @@ public:
 	~WorkspaceLease();
 	WorkspaceLease(const WorkspaceLease&) = delete;
 	WorkspaceLease& operator=(const WorkspaceLease&) = delete;
-	int take();                       // a workspace of the current device
+	// A workspace of the current device, for work on `stream`: an idle one whose
+	// last work is over, a new one, or one that `stream` is made to wait for.
+	int take(hipStream_t stream = nullptr);
+	// The work on `stream` so far goes on reading the workspace after the lease.
+	int leave_to(hipStream_t stream);
 	int pinned(size_t bytes);         // its staging, at least this large
 	// `count` points for a kernel to read at `xyz` and `width` floats each for it
 	// to write at `out`: the pinned staging itself for few points, else device
