@@ -56,6 +56,7 @@ struct tg_mesher
 	bool have_grid = false;
 	tg_export_stats stats{};
 	int points_per_lane = 4;      // block kernel: points per lane (2, 4, 8; tg_mesher_autotune)
+	bool shape_set = false;       // by the caller or autotune; else block_points
 	int waves = 2;                // block kernel: waves per workgroup (1, 2, 4)
 	int workgroups_per_cu = 8;    // 0: a workgroup per block (LDS tables); else persistent, global tables
 	// launch shape of culled exports (tg_mesher_set_culled_tuning): their
@@ -561,6 +562,16 @@ int block_order(tg_mesher* m, const BlockDesc* desc, const uint32_t* list, uint3
 	return TG_OK;
 }
 
+// Points per lane of a plain export's blocks where the caller has not set them:
+// 8 share an entry's decode and transform among more samples, 4 leave more waves
+// per block.  (Whole export, 4 / 8 points: 1024^3 of 2048 primitives 12.05 / 11.6 ms, of
+// 512 9.95 / 9.52, of 16 3.45 / 3.06; 800^3 of 2048 8.03 / 8.26, of 256 3.11 / 2.86; 700^3 of
+// 256 2.74 / 2.57; 600^3 of 512 2.44 / 2.76.)
+int block_points(const tg_program* p, uint32_t nblocks)
+{
+	return nblocks >= 24576 || (nblocks >= 8192 && p->decoded.entries.size() <= 1024) ? 8 : 4;
+}
+
 // Pruned evaluation (k_eval_blocks) of the listed blocks' masked tiles, or of
 // every tile.  Needs m->blocks.valid.  `sorted`: m->order already holds the
 // queue of every block (block_order, enqueued with the pruning).
@@ -576,7 +587,7 @@ int eval_blocks(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t fl
 	BlockEvalArgs ba = block_args(m, p, g, tile_mask, block_list, n_listed, work);
 	// culled exports (a block list) have their own launch shape
 	const bool culled = block_list != nullptr;
-	int pts = culled ? m->culled_points_per_lane : m->points_per_lane;
+	int pts = culled ? m->culled_points_per_lane : m->shape_set ? m->points_per_lane : block_points(p, ba.nblocks);
 	const int shape_waves = culled ? m->culled_waves : m->waves;
 	const int shape_wgs = culled ? m->culled_workgroups_per_cu : m->workgroups_per_cu;
 	ba.waves = shape_waves;
@@ -1072,7 +1083,7 @@ extern "C" int tg_mesher_set_tuning(tg_mesher* m, uint32_t points_per_lane, uint
 	m->waves = int(waves);
 	m->workgroups_per_cu = int(workgroups_per_cu);
 	m->min_prune_len = min_prune_len;
-	m->by_blocks = true;
+	m->by_blocks = m->shape_set = true;
 	return TG_OK;
 }
 
@@ -1115,6 +1126,7 @@ extern "C" int tg_mesher_autotune(tg_mesher* m, const tg_program* p, const tg_gr
 	rc = prune_blocks(m, p, g, flags);
 	if (rc) return rc;
 	if (!m->blocks.valid) return fail(TG_ERR_INVALID, "tg_mesher_autotune: program not prunable here");
+	m->shape_set = true;
 	tg_tune_result res{};
 	// (waves, workgroups per CU): a workgroup per block (0) with LDS tables,
 	// or persistent workgroups with global tables
