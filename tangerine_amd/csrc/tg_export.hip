@@ -36,7 +36,7 @@ struct tg_mesher
 {
 	hipStream_t stream = nullptr;
 	hipEvent_t ev[6] = {};
-	DevBuf pool, signs, active, word_count, word_base, quad_count, quad_base, vertices, triangles, scan_tmp, dense, cubes;
+	DevBuf pool, signs, active, word_count, word_base, quad_count, vertices, triangles, scan_tmp, dense, cubes;
 	DevBuf normals, exchange;
 	DevBuf cloud_flags, cloud_rank, vox_list;
 	uint64_t nvox = 0;            // voxels of the last MagicaVoxel export
@@ -126,77 +126,29 @@ int layout(tg_mesher* m, const tg_grid* g)
 	return TG_OK;
 }
 
-// Surface nets over the samples already in pool/signs: classify cube rows,
-// scan the per-word counts into vertex ids, list the active cubes, then one
-// thread per active cube places its vertex and counts and (after a scan of the
-// counts) writes its quads.  Three stages on the mesher's stream; each of the
-// first two ends with an asynchronous copy of two counts into the pinned
-// m->tail, which the next stage reads after the caller has synchronised the
-// stream (the batch runs each stage over all its trees before waiting).
-int surface_nets_classify(tg_mesher* m, bool copy_counts = true)
+// Surface nets over the samples already in pool/signs (MeshStage): the buffers of
+// the stages up to the vertex ids, which need no room.
+int surface_nets_buffers(tg_mesher* m, uint64_t cap_v)
 {
 	MeshArgs& a = m->args;
 	const uint64_t words = uint64_t(a.sy) * a.sz * a.aw;
+	const uint64_t word_chunks = (words + kMeshWords - 1) / kMeshWords, cube_chunks = (cap_v + kMeshCubes - 1) / kMeshCubes;
 	int rc = m->active.ensure(words * 8);
 	if (!rc) rc = m->word_count.ensure(words * 4);
 	if (!rc) rc = m->word_base.ensure(words * 4);
+	if (!rc) rc = m->scan_tmp.ensure((word_chunks + cube_chunks) * 4);
 	if (rc) return rc;
 	a.active = m->active.as<uint64_t>();
 	a.word_count = m->word_count.as<uint32_t>();
 	a.word_base = m->word_base.as<uint32_t>();
-	size_t tmp = 0;
-	TG_CHECK_HIP(exclusive_scan_u32(nullptr, nullptr, words, nullptr, tmp, m->stream), "scan sizing");
-	rc = m->scan_tmp.ensure(tmp);
-	if (rc) return rc;
-	TG_CHECK_HIP(mesh_classify(a, m->stream), "classify launch");
-	tmp = m->scan_tmp.bytes;
-	TG_CHECK_HIP(exclusive_scan_u32(a.word_count, a.word_base, words, m->scan_tmp.ptr, tmp, m->stream), "vertex scan");
-	if (copy_counts)
-	{
-		TG_CHECK_HIP(hipMemcpyAsync(&m->tail[0], a.word_base + words - 1, 4, hipMemcpyDeviceToHost, m->stream),
-			"count copy");
-		TG_CHECK_HIP(hipMemcpyAsync(&m->tail[1], a.word_count + words - 1, 4, hipMemcpyDeviceToHost, m->stream),
-			"count copy");
-	}
+	a.word_sums = m->scan_tmp.as<uint32_t>();
+	a.quad_sums = a.word_sums + word_chunks;
+	a.tail = m->tail_dev;
 	return TG_OK;
 }
 
 // Room for a mesh after one of n vertices (or quads): a quarter more.
 uint64_t room_for(uint64_t n) { return n + n / 4 + 4096; }
-
-int surface_nets_vertices(tg_mesher* m)
-{
-	MeshArgs& a = m->args;
-	m->nverts = uint64_t(m->tail[0]) + m->tail[1];
-	const uint64_t nv = m->nverts;
-	if (nv >= (1ull << 31)) return fail(TG_ERR_LIMIT, "surface nets: more than 2^31 vertices");
-	// sized for the room the next mesh will run in (size_next_mesh), so
-	// that it allocates nothing
-	const uint64_t room = room_for(nv);
-	int rc = m->vertices.ensure(room * 12);
-	if (!rc) rc = m->cubes.ensure(room * 4);
-	if (!rc) rc = m->quad_count.ensure(room * 4);
-	if (!rc) rc = m->quad_base.ensure(room * 4);
-	if (rc) return rc;
-	a.vertices = m->vertices.as<float>();
-	a.cubes = m->cubes.as<uint32_t>();
-	a.cube_quads = m->quad_count.as<uint32_t>();
-	a.cube_qbase = m->quad_base.as<uint32_t>();
-	a.cap_verts = nv;
-	m->tail[2] = m->tail[3] = 0;
-	if (!nv) return TG_OK;
-	TG_CHECK_HIP(mesh_list_cubes(a, m->stream), "cube list launch");
-	TG_CHECK_HIP(mesh_vertices(a, nv, m->stream), "vertex launch");  // also each cube's quad flags
-	size_t tmp = 0;
-	TG_CHECK_HIP(exclusive_scan_quads(nullptr, nullptr, room, nullptr, tmp, m->stream), "scan sizing");
-	rc = m->scan_tmp.ensure(tmp);
-	if (rc) return rc;
-	tmp = m->scan_tmp.bytes;
-	TG_CHECK_HIP(exclusive_scan_quads(a.cube_quads, a.cube_qbase, nv, m->scan_tmp.ptr, tmp, m->stream), "quad scan");
-	TG_CHECK_HIP(hipMemcpyAsync(&m->tail[2], a.cube_qbase + nv - 1, 4, hipMemcpyDeviceToHost, m->stream), "count copy");
-	TG_CHECK_HIP(hipMemcpyAsync(&m->tail[3], a.cube_quads + nv - 1, 4, hipMemcpyDeviceToHost, m->stream), "count copy");
-	return TG_OK;
-}
 
 // Room for the next mesh of this mesher: a quarter more than this one.
 void size_next_mesh(tg_mesher* m)
@@ -205,72 +157,43 @@ void size_next_mesh(tg_mesher* m)
 	m->spec_quads = room_for(m->ntris / 2);
 }
 
-// Quads of the vertex stage's flags (m->tail[2..3]: the last cube's scanned
-// base and its flags).
-uint64_t quads_from_tail(const tg_mesher* m)
+// The stages [from, to) on the mesher's stream.
+int surface_nets_stages(tg_mesher* m, int from, int to)
 {
-	return uint64_t(m->tail[2]) + uint64_t(__builtin_popcount(m->tail[3] & 7u));
-}
-
-int surface_nets_quads(tg_mesher* m)
-{
-	MeshArgs& a = m->args;
-	const uint64_t quads = quads_from_tail(m);
-	m->ntris = quads * 2;
-	int rc = m->triangles.ensure(room_for(quads) * 24);
-	if (rc) return rc;
-	a.triangles = m->triangles.as<uint32_t>();
-	a.cap_quads = quads;
-	if (quads) TG_CHECK_HIP(mesh_quad_write(a, m->nverts, m->stream), "quad write launch");
+	for (int stage = from; stage < to; ++stage) TG_CHECK_HIP(mesh_stage(m->args, stage, m->stream), "surface nets launch");
 	return TG_OK;
 }
 
-// All three stages at once, in the room m->spec_verts / m->spec_quads that an
-// earlier mesh left: the kernels take the vertex count from the device and
+// Buffers for all stages at once, in the room m->spec_verts / m->spec_quads that
+// an earlier mesh left: the kernels take the vertex count from the device and
 // write within the room, and the host reads the counts once, at the end
-// (surface_nets_room_check, after the stream is synchronised).
+// (surface_nets_room_check, after the stages' stream is synchronised).
 int surface_nets_in_room(tg_mesher* m)
 {
 	MeshArgs& a = m->args;
 	const uint64_t cap_v = m->spec_verts, cap_q = m->spec_quads;
-	// every buffer sized before the first launch (growing one frees it)
-	size_t tmp = 0;
-	TG_CHECK_HIP(exclusive_scan_quads(nullptr, nullptr, cap_v, nullptr, tmp, m->stream), "scan sizing");
-	int rc = m->scan_tmp.ensure(tmp);
+	int rc = surface_nets_buffers(m, cap_v);
 	if (!rc) rc = m->vertices.ensure(cap_v * 12);
 	if (!rc) rc = m->cubes.ensure(cap_v * 4);
 	if (!rc) rc = m->quad_count.ensure(cap_v * 4);
-	if (!rc) rc = m->quad_base.ensure(cap_v * 4);
 	if (!rc) rc = m->triangles.ensure(cap_q * 24);
-	if (rc) return rc;
-	rc = surface_nets_classify(m, false);
 	if (rc) return rc;
 	a.vertices = m->vertices.as<float>();
 	a.cubes = m->cubes.as<uint32_t>();
 	a.cube_quads = m->quad_count.as<uint32_t>();
-	a.cube_qbase = m->quad_base.as<uint32_t>();
 	a.triangles = m->triangles.as<uint32_t>();
 	a.cap_verts = cap_v;
 	a.cap_quads = cap_q;
-	a.tail = m->tail_dev;  // the kernels write the totals: no copies to issue
-	TG_CHECK_HIP(mesh_list_cubes(a, m->stream), "cube list launch");
-	TG_CHECK_HIP(mesh_vertices(a, cap_v, m->stream), "vertex launch");
-	tmp = m->scan_tmp.bytes;
-	TG_CHECK_HIP(exclusive_scan_quads(a.cube_quads, a.cube_qbase, cap_v, m->scan_tmp.ptr, tmp, m->stream), "quad scan");
-	TG_CHECK_HIP(mesh_quad_write(a, cap_v, m->stream), "quad write launch");
-	a.tail = nullptr;
 	return TG_OK;
 }
 
-// After surface_nets_in_room and a wait for the stream: whether the mesh fit
-// the room (else it is incomplete and must be made the waiting way); sets the
-// counts when it did.
+// After the stages in the room and a wait for them: whether the mesh fit (else
+// it is incomplete and must be made the waiting way); sets the counts when it did.
 bool surface_nets_room_check(tg_mesher* m)
 {
-	const uint64_t nv = uint64_t(m->tail[0]) + m->tail[1];
+	const uint64_t nv = m->tail[0];
 	if (nv > m->spec_verts) return false;
-	// flags past the active cubes are zero, so the scan's total is the mesh's
-	const uint64_t quads = quads_from_tail(m);
+	const uint64_t quads = m->tail[1];
 	if (quads > m->spec_quads) return false;
 	m->nverts = nv;
 	m->ntris = quads * 2;
@@ -279,10 +202,58 @@ bool surface_nets_room_check(tg_mesher* m)
 	return true;
 }
 
-// The waiting way: each stage after the previous stage's counts.
+// The waiting way in three parts, each after a wait for the one before: vertex
+// ids without a list, the vertices and the quads' count in room of exactly that
+// many, the triangles.  (The batch runs each part over all its trees before
+// waiting.)
+int surface_nets_count(tg_mesher* m)
+{
+	MeshArgs& a = m->args;
+	int rc = surface_nets_buffers(m, 0);
+	if (rc) return rc;
+	a.cap_verts = a.cap_quads = 0;
+	m->tail[0] = m->tail[1] = 0;
+	return surface_nets_stages(m, kMeshClassify, kMeshVertices);
+}
+
+int surface_nets_vertices(tg_mesher* m)
+{
+	MeshArgs& a = m->args;
+	m->nverts = m->tail[0];
+	const uint64_t nv = m->nverts;
+	if (nv >= (1ull << 31)) return fail(TG_ERR_LIMIT, "surface nets: more than 2^31 vertices");
+	// sized for the room the next mesh will run in (size_next_mesh), so
+	// that it allocates nothing
+	const uint64_t room = room_for(nv);
+	int rc = surface_nets_buffers(m, room);
+	if (!rc) rc = m->vertices.ensure(room * 12);
+	if (!rc) rc = m->cubes.ensure(room * 4);
+	if (!rc) rc = m->quad_count.ensure(room * 4);
+	if (rc) return rc;
+	a.vertices = m->vertices.as<float>();
+	a.cubes = m->cubes.as<uint32_t>();
+	a.cube_quads = m->quad_count.as<uint32_t>();
+	a.cap_verts = nv;
+	if (!nv) return TG_OK;
+	// (the sums again: their buffer may have moved)
+	return surface_nets_stages(m, kMeshSums, kMeshStages);
+}
+
+int surface_nets_quads(tg_mesher* m)
+{
+	MeshArgs& a = m->args;
+	const uint64_t quads = m->nverts ? m->tail[1] : 0;
+	m->ntris = quads * 2;
+	int rc = m->triangles.ensure(room_for(quads) * 24);
+	if (rc) return rc;
+	a.triangles = m->triangles.as<uint32_t>();
+	a.cap_quads = quads;
+	return quads ? surface_nets_stages(m, kMeshQuads, kMeshStages) : int(TG_OK);
+}
+
 int surface_nets_waiting(tg_mesher* m)
 {
-	int rc = surface_nets_classify(m);
+	int rc = surface_nets_count(m);
 	if (rc) return rc;
 	TG_CHECK_HIP(hipStreamSynchronize(m->stream), "vertex count");
 	rc = surface_nets_vertices(m);
@@ -294,12 +265,12 @@ int surface_nets_waiting(tg_mesher* m)
 	return TG_OK;
 }
 
-
 int surface_nets(tg_mesher* m)
 {
 	if (m->spec_verts > 0)
 	{
 		int rc = surface_nets_in_room(m);
+		if (!rc) rc = surface_nets_stages(m, kMeshClassify, kMeshStages);
 		if (rc) return rc;
 		TG_CHECK_HIP(hipStreamSynchronize(m->stream), "surface nets");
 		if (surface_nets_room_check(m)) return TG_OK;
@@ -753,7 +724,7 @@ void destroy_mesher(tg_mesher* m)
 {
 	if (m->stream) (void)hipStreamSynchronize(m->stream);
 	if (m->tail) (void)hipHostFree(m->tail);
-	for (DevBuf* b : { &m->pool, &m->signs, &m->active, &m->word_count, &m->word_base, &m->quad_count, &m->quad_base,
+	for (DevBuf* b : { &m->pool, &m->signs, &m->active, &m->word_count, &m->word_base, &m->quad_count,
 	                   &m->vertices, &m->triangles, &m->scan_tmp, &m->dense, &m->counters, &m->brick_flags,
 	                   &m->brick_active, &m->tile_mask, &m->block_list, &m->tile_list, &m->cubes, &m->normals,
 	                   &m->exchange, &m->persist_args, &m->persist_head, &m->persist_tables, &m->order_keys,
@@ -1244,7 +1215,9 @@ extern "C" int tg_mesher_copy_mesh(const tg_mesher* m, float* v, uint32_t* t)
 {
 	if (!m) return fail(TG_ERR_INVALID, "tg_mesher_copy_mesh: null argument");
 	if (m->nverts && v)
-		TG_CHECK_HIP(hipMemcpy(v, m->vertices.ptr, m->nverts * 12, hipMemcpyDeviceToHost), "vertex download");
+		TG_CHECK_HIP(m->ntris && t
+				? hipMemcpyAsync(v, m->vertices.ptr, m->nverts * 12, hipMemcpyDeviceToHost, nullptr)  // (waited for below)
+				: hipMemcpy(v, m->vertices.ptr, m->nverts * 12, hipMemcpyDeviceToHost), "vertex download");
 	if (m->ntris && t)
 		TG_CHECK_HIP(hipMemcpy(t, m->triangles.ptr, m->ntris * 12, hipMemcpyDeviceToHost), "triangle download");
 	return TG_OK;
@@ -1929,7 +1902,7 @@ extern "C" int tg_mesher_grid_get(const tg_mesher* m, tg_grid* out)
 // of k_eval_batch over a device queue of (tree, block) items, most expensive
 // block program first (so that the tail of the queue holds short items); the
 // launch and the reset of the queue head and work counters are captured in a
-// hipGraph, replayed by tg_batch_export and tg_batch_replay.  Each workgroup
+// hipGraph for tg_batch_replay.  Each workgroup
 // keeps its block's decision tables and tile programs in its own slice of
 // global scratch (LDS holds only the tile descriptors and the spill region),
 // so programs of any length run at the same occupancy.
@@ -1951,9 +1924,13 @@ struct tg_batch
 	size_t tile_lds = 0;          // per wave
 	bool by_blocks = false;       // tg_batch_set_tuning was called: every tree by blocks
 	PruneLaunches prune;          // every tree's level pruning and emission as shared launches
+	DevBuf mesh_jobs;             // the trees' surface-nets arguments and first workgroups
 	DevBuf queue_sort;            // the queue's keys, values, tree offsets and sort storage
-	hipGraph_t graph = nullptr;
+	hipGraph_t graph = nullptr;   // the evaluation, captured at the first replay
 	hipGraphExec_t exec = nullptr;
+	bool exported = false;        // the last export's evaluation can be replayed
+	unsigned long long* host_work = nullptr;  // pinned copy of `work`
+	size_t host_work_bytes = 0;
 	BatchArgs args = {};
 	bool fast = false;
 	int points_per_lane = 4;      // launch shape (tg_batch_set_tuning / autotune)
@@ -1998,14 +1975,11 @@ int shape_batch(tg_batch* b, int points, int waves, int wgs_per_cu)
 	return TG_OK;
 }
 
-// Captures the queue reset and the persistent launch with the current tuning.
-int capture_batch(tg_batch* b)
+// The evaluation's launches: the queue's and counters' reset, the persistent
+// launch, the tile programs.
+hipError_t launch_evaluation(tg_batch* b)
 {
-	drop_graph(b);
-	int rc = shape_batch(b, b->points_per_lane, b->waves, b->workgroups_per_cu);
-	if (rc) return rc;
 	const uint32_t nwork = uint32_t(b->meshers.size() * (kWorkBytes / 8));
-	TG_CHECK_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal), "capture begin");
 	hipError_t e = b->fast ? fast::launch_batch_reset(b->args.head, b->work.as<unsigned long long>(), nwork, b->stream)
 	                       : exact::launch_batch_reset(b->args.head, b->work.as<unsigned long long>(), nwork, b->stream);
 	if (e == hipSuccess)
@@ -2021,6 +1995,17 @@ int capture_batch(tg_batch* b)
 			? fast::launch_eval_tile_programs_multi(jobs, base, b->tile_njobs, b->tile_blocks, b->tile_lds, b->stream)
 			: exact::launch_eval_tile_programs_multi(jobs, base, b->tile_njobs, b->tile_blocks, b->tile_lds, b->stream);
 	}
+	return e;
+}
+
+// Captures them with the current tuning.
+int capture_batch(tg_batch* b)
+{
+	drop_graph(b);
+	int rc = shape_batch(b, b->points_per_lane, b->waves, b->workgroups_per_cu);
+	if (rc) return rc;
+	TG_CHECK_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal), "capture begin");
+	const hipError_t e = launch_evaluation(b);
 	hipGraph_t g = nullptr;
 	const hipError_t ee = hipStreamEndCapture(b->stream, &g);
 	if (e != hipSuccess)
@@ -2031,6 +2016,52 @@ int capture_batch(tg_batch* b)
 	if (ee != hipSuccess) return hip_fail(ee, "batch capture end");
 	b->graph = g;
 	TG_CHECK_HIP(hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0), "batch graph instantiate");
+	return TG_OK;
+}
+
+// Surface nets of every tree that has room from an earlier export, a launch per
+// stage for all of them, behind the evaluation on the batch's stream; waits for
+// the stream and marks the trees whose mesh fit in `done`.
+int batch_nets_in_room(tg_batch* b, std::vector<uint8_t>& done)
+{
+	std::vector<uint32_t> who;
+	std::vector<MeshArgs> jobs;
+	for (uint32_t i = 0; i < b->meshers.size(); ++i)
+	{
+		tg_mesher* m = b->meshers[i];
+		if (m->spec_verts == 0) continue;
+		int rc = surface_nets_in_room(m);
+		if (rc) return rc;
+		who.push_back(i);
+		jobs.push_back(m->args);
+	}
+	if (jobs.empty())
+	{
+		TG_CHECK_HIP(hipStreamSynchronize(b->stream), "batch evaluation");
+		return TG_OK;
+	}
+	const size_t n = jobs.size(), jb = n * sizeof(MeshArgs);
+	std::vector<uint8_t> blob(jb + kMeshStages * n * 4);
+	std::memcpy(blob.data(), jobs.data(), jb);
+	uint32_t* base = reinterpret_cast<uint32_t*>(blob.data() + jb);
+	uint64_t blocks[kMeshStages] = {};
+	for (int stage = 0; stage < kMeshStages; ++stage)
+		for (size_t k = 0; k < n; ++k)
+		{
+			base[stage * n + k] = uint32_t(blocks[stage]);
+			blocks[stage] += mesh_blocks(jobs[k], stage);
+			if (blocks[stage] >= (1ull << 31)) return fail(TG_ERR_LIMIT, "batch: too many surface-nets workgroups");
+		}
+	int rc = b->mesh_jobs.ensure(blob.size());
+	if (rc) return rc;
+	TG_CHECK_HIP(hipMemcpyAsync(b->mesh_jobs.ptr, blob.data(), blob.size(), hipMemcpyHostToDevice, b->stream), "mesh job upload");
+	const MeshArgs* dev = b->mesh_jobs.as<const MeshArgs>();
+	const uint32_t* dev_base = reinterpret_cast<const uint32_t*>(dev + n);
+	for (int stage = 0; stage < kMeshStages; ++stage)
+		TG_CHECK_HIP(mesh_stage_multi(dev, dev_base + stage * n, uint32_t(n), uint32_t(blocks[stage]), stage, b->stream),
+			"surface nets launch");
+	TG_CHECK_HIP(hipStreamSynchronize(b->stream), "surface nets");
+	for (uint32_t i : who) done[i] = surface_nets_room_check(b->meshers[i]) ? 1 : 0;
 	return TG_OK;
 }
 
@@ -2071,8 +2102,9 @@ extern "C" void tg_batch_destroy(tg_batch* b)
 	if (!b) return;
 	if (b->stream) (void)hipStreamSynchronize(b->stream);
 	drop_graph(b);
+	if (b->host_work) (void)hipHostFree(b->host_work);
 	for (tg_mesher* m : b->meshers) destroy_mesher(m);
-	for (DevBuf* d : { &b->trees, &b->items, &b->head, &b->work, &b->tables, &b->prune.dev, &b->queue_sort, &b->tile_jobs })
+	for (DevBuf* d : { &b->trees, &b->items, &b->head, &b->work, &b->tables, &b->prune.dev, &b->queue_sort, &b->tile_jobs, &b->mesh_jobs })
 		d->release();
 	for (hipEvent_t e : b->ev)
 		if (e) (void)hipEventDestroy(e);
@@ -2089,7 +2121,11 @@ extern "C" int tg_batch_set_tuning(tg_batch* b, uint32_t points_per_lane, uint32
 	b->waves = int(waves);
 	b->workgroups_per_cu = int(workgroups_per_cu);
 	b->by_blocks = true;
-	if (b->exec) return capture_batch(b);
+	if (b->exported)
+	{
+		drop_graph(b);
+		return shape_batch(b, b->points_per_lane, b->waves, b->workgroups_per_cu);
+	}
 	return TG_OK;
 }
 
@@ -2109,6 +2145,7 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 		if (rc) return rc;
 	}
 	drop_graph(b);
+	b->exported = false;
 	b->fast = (flags & TG_FLAG_FAST) != 0;
 	while (b->meshers.size() < count)
 	{
@@ -2190,6 +2227,7 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 		ba.max_len = std::max(ba.max_len, args[i].max_len);
 	}
 	b->tile_njobs = uint32_t(tile_jobs.size());
+	std::vector<uint8_t> blob;  // (uploaded on the stream: kept to the end)
 	if (b->tile_njobs)
 	{
 		// the jobs with the longest programs first (a wave's time is its
@@ -2203,12 +2241,13 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 			b->tile_blocks += tile_eval_blocks(ta);
 		}
 		const size_t jb = tile_jobs.size() * sizeof(TileEvalArgs);
-		std::vector<uint8_t> blob(jb + tile_base.size() * 4);
+		blob.resize(jb + tile_base.size() * 4);
 		std::memcpy(blob.data(), tile_jobs.data(), jb);
 		std::memcpy(blob.data() + jb, tile_base.data(), tile_base.size() * 4);
 		rc = b->tile_jobs.ensure(blob.size());
 		if (rc) return rc;
-		TG_CHECK_HIP(hipMemcpy(b->tile_jobs.ptr, blob.data(), blob.size(), hipMemcpyHostToDevice), "tile job upload");
+		TG_CHECK_HIP(hipMemcpyAsync(b->tile_jobs.ptr, blob.data(), blob.size(), hipMemcpyHostToDevice, b->stream),
+			"tile job upload");
 	}
 	// 2. the queue, sorted on the device: every tree's blocks, the most
 	// expensive block program first
@@ -2232,13 +2271,16 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 	uint32_t* first_dev = sort_buf + 4 * size_t(total);
 	void* sort_temp = reinterpret_cast<unsigned char*>(b->queue_sort.ptr) +
 	                  ((4 * size_t(total) + count + 1) * 4 + 255) / 256 * 256;
-	TG_CHECK_HIP(hipMemcpyAsync(b->trees.ptr, args.data(), size_t(count) * sizeof(BlockEvalArgs), hipMemcpyHostToDevice,
-		b->stream), "upload");
-	TG_CHECK_HIP(hipMemcpyAsync(first_dev, first.data(), (size_t(count) + 1) * 4, hipMemcpyHostToDevice, b->stream),
-		"upload");
-	TG_CHECK_HIP(batch_queue_by_cost(b->trees.as<const BlockEvalArgs>(), first_dev, count, total, sort_buf,
-		b->items.as<uint32_t>(), sort_temp, sort_tmp, b->stream), "queue sort");
-	TG_CHECK_HIP(hipStreamSynchronize(b->stream), "queue sort");
+	if (total)
+	{
+		TG_CHECK_HIP(hipMemcpyAsync(b->trees.ptr, args.data(), size_t(count) * sizeof(BlockEvalArgs), hipMemcpyHostToDevice,
+			b->stream), "upload");
+		TG_CHECK_HIP(hipMemcpyAsync(first_dev, first.data(), (size_t(count) + 1) * 4, hipMemcpyHostToDevice, b->stream),
+			"upload");
+		TG_CHECK_HIP(batch_queue_by_cost(b->trees.as<const BlockEvalArgs>(), first_dev, count, total, sort_buf,
+			b->items.as<uint32_t>(), sort_temp, sort_tmp, b->stream), "queue sort");
+		TG_CHECK_HIP(hipStreamSynchronize(b->stream), "queue sort");
+	}
 	ba.trees = b->trees.as<const BlockEvalArgs>();
 	ba.items = b->items.as<const uint32_t>();
 	ba.ntrees = count;
@@ -2246,46 +2288,45 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 	ba.head = b->head.as<unsigned int>();
 	b->args = ba;
 	auto t1 = std::chrono::steady_clock::now();
-	// 3. one persistent launch (captured), then surface nets per tree
-	rc = capture_batch(b);
+	// 3. the evaluation, the work counters' copy and, behind them on the stream,
+	// surface nets
+	rc = shape_batch(b, b->points_per_lane, b->waves, b->workgroups_per_cu);
+	if (rc) return rc;
+	const size_t work_bytes = size_t(count) * kWorkBytes;
+	if (work_bytes > b->host_work_bytes)
+	{
+		if (b->host_work) (void)hipHostFree(b->host_work);
+		b->host_work = nullptr;
+		b->host_work_bytes = 0;
+		TG_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&b->host_work), work_bytes, hipHostMallocDefault), "work counters");
+		b->host_work_bytes = work_bytes;
+	}
+	TG_CHECK_HIP(hipEventRecord(b->ev[0], b->stream), "event");
+	TG_CHECK_HIP(launch_evaluation(b), "batch evaluation");
+	TG_CHECK_HIP(hipEventRecord(b->ev[1], b->stream), "event");
+	b->exported = true;
+	TG_CHECK_HIP(hipMemcpyAsync(b->host_work, b->work.ptr, work_bytes, hipMemcpyDeviceToHost, b->stream), "work read");
+	uint64_t evals = 0;
+	double flops = 0;
+	// surface nets: in the room an earlier export left, every such tree's stage in
+	// one launch; the others, with those that outgrew their room, the waiting
+	// way on the trees' streams, each part over every tree before waiting
+	std::vector<uint8_t> done(count, 0);
+	rc = batch_nets_in_room(b, done);
 	if (rc) return rc;
 	float eval_ms = 0;
-	rc = replay_batch(b, &eval_ms);
-	if (rc) return rc;
-	std::vector<unsigned long long> slots(size_t(count) * (kWorkBytes / 8)), wk(2 * size_t(count));
-	TG_CHECK_HIP(hipMemcpy(slots.data(), b->work.ptr, slots.size() * 8, hipMemcpyDeviceToHost), "work read");
+	TG_CHECK_HIP(hipEventElapsedTime(&eval_ms, b->ev[0], b->ev[1]), "timing");
+	std::vector<unsigned long long> wk(2 * size_t(count));
 	for (uint32_t i = 0; i < count; ++i)
 	{
-		const unsigned long long* w = slots.data() + size_t(i) * (kWorkBytes / 8);
+		const unsigned long long* w = b->host_work + size_t(i) * (kWorkBytes / 8);
 		wk[2 * i] = b->by_tiles[i] ? uint64_t(b->meshers[i]->blocks.ncells) * kTileSamples : work_sum(w, 0);
 		wk[2 * i + 1] = work_sum(w, 1);
 	}
-	auto t2 = std::chrono::steady_clock::now();
-	double mesh_ms = 0;
-	uint64_t evals = 0;
-	double flops = 0;
-	// surface nets on the trees' streams: in the room an earlier export left
-	// (all stages of every such tree issued before any wait), and the others,
-	// with those that outgrew their room, the waiting way, each stage over
-	// every tree before waiting
-	std::vector<uint8_t> done(count, 0);
-	for (uint32_t i = 0; i < count; ++i)
-		if (b->meshers[i]->spec_verts > 0)
-		{
-			rc = surface_nets_in_room(b->meshers[i]);
-			if (rc) return rc;
-			done[i] = 1;
-		}
-	for (uint32_t i = 0; i < count; ++i)
-		if (done[i])
-		{
-			TG_CHECK_HIP(hipStreamSynchronize(b->meshers[i]->stream), "surface nets");
-			done[i] = surface_nets_room_check(b->meshers[i]) ? 1 : 0;
-		}
 	for (uint32_t i = 0; i < count; ++i)
 	{
 		if (done[i]) continue;
-		rc = surface_nets_classify(b->meshers[i]);
+		rc = surface_nets_count(b->meshers[i]);
 		if (rc) return rc;
 	}
 	for (uint32_t i = 0; i < count; ++i)
@@ -2306,7 +2347,7 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 	for (uint32_t i = 0; i < count; ++i)
 	{
 		tg_mesher* m = b->meshers[i];
-		TG_CHECK_HIP(hipStreamSynchronize(m->stream), "batch mesh");
+		if (!done[i]) TG_CHECK_HIP(hipStreamSynchronize(m->stream), "batch mesh");
 		m->have_grid = true;
 		tg_export_stats& s = m->stats;
 		s = tg_export_stats{};
@@ -2318,7 +2359,8 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 		flops += double(wk[2 * i + 1]);
 	}
 	auto t3 = std::chrono::steady_clock::now();
-	mesh_ms = std::chrono::duration<double, std::milli>(t3 - t2).count();
+	// (from the evaluation's launch to the meshes, less the evaluation)
+	const double mesh_ms = std::max(0.0, std::chrono::duration<double, std::milli>(t3 - t1).count() - double(eval_ms));
 	tg_batch_stats& st = b->stats;
 	st = tg_batch_stats{};
 	st.prune_ms = std::chrono::duration<double, std::milli>(t1 - t0).count();
@@ -2345,9 +2387,10 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 extern "C" int tg_batch_replay(tg_batch* b, double* eval_ms)
 {
 	if (!b || !eval_ms) return fail(TG_ERR_INVALID, "tg_batch_replay: null argument");
-	if (!b->exec) return fail(TG_ERR_INVALID, "tg_batch_replay: no batch exported yet");
+	if (!b->exported) return fail(TG_ERR_INVALID, "tg_batch_replay: no batch exported yet");
 	float ms = 0;
-	int rc = replay_batch(b, &ms);
+	int rc = b->exec ? int(TG_OK) : capture_batch(b);
+	if (!rc) rc = replay_batch(b, &ms);
 	if (rc) return rc;
 	*eval_ms = ms;
 	return TG_OK;
@@ -2356,7 +2399,7 @@ extern "C" int tg_batch_replay(tg_batch* b, double* eval_ms)
 extern "C" int tg_batch_autotune(tg_batch* b, tg_batch_tune_result* out)
 {
 	if (!b) return fail(TG_ERR_INVALID, "tg_batch_autotune: null argument");
-	if (!b->exec) return fail(TG_ERR_INVALID, "tg_batch_autotune: export a batch first");
+	if (!b->exported) return fail(TG_ERR_INVALID, "tg_batch_autotune: export a batch first");
 	// points per lane x (waves, workgroups per CU): 18 shapes
 	const int pts_c[3] = { 2, 4, 8 };
 	const int shape_c[6][2] = { { 4, 2 }, { 4, 3 }, { 4, 4 }, { 4, 6 }, { 2, 6 }, { 2, 8 } };

@@ -29,12 +29,12 @@ struct MeshArgs
 	uint32_t* word_base;
 	uint32_t* cubes;              // active cubes in vertex-id order: i + sx (j + sy k)
 	uint32_t* cube_quads;         // quad flags per active cube (tg_mesh.hip: quad_flags)
-	uint32_t* cube_qbase;         // exclusive scan of the quad counts
-	uint64_t cap_verts;           // room for active cubes (cubes, vertices, quad flags and bases)
+	uint32_t* word_sums;          // active cubes of every kMeshWords words
+	uint32_t* quad_sums;          // quads of every kMeshCubes active cubes
+	uint64_t cap_verts;           // room for active cubes (cubes, vertices, quad flags)
 	uint64_t cap_quads;           // room for quads (triangle pairs)
-	uint32_t* tail;               // non-null: pinned host words the kernels write the totals to
-	                              // (k_vertices: the last word's vertex base and count,
-	                              // k_quad_write: the last cube's quad base and flags)
+	uint32_t* tail;               // pinned host words the stages write the totals to
+	                              // (list: [0] vertices, quads: [1] quads)
 	// outputs
 	float* vertices;
 	uint32_t* triangles;
@@ -45,18 +45,22 @@ struct MeshArgs
 // Practice and Experience 49(6), 2019); M = 0 stands for d = 1.
 inline uint64_t mesh_div_magic(uint32_t d) { return d <= 1 ? 0ull : ~0ull / d + 1ull; }
 
-hipError_t mesh_classify(const MeshArgs& a, hipStream_t s);
-// Thread per active cube (after the vertex-id scan): cube list, vertices,
-// quad flags and, after the scan of their counts, triangles.
-hipError_t mesh_list_cubes(const MeshArgs& a, hipStream_t s);
-hipError_t mesh_vertices(const MeshArgs& a, uint64_t nverts, hipStream_t s);
-hipError_t mesh_quad_write(const MeshArgs& a, uint64_t nverts, hipStream_t s);
+constexpr uint32_t kMeshWords = 4096, kMeshCubes = 1024;  // to a workgroup of the scanning stages
+
+// Surface nets in five launches: active bits of the cubes, the sums of
+// their words, vertex ids and the list of active cubes, vertices and quad
+// flags, triangles.  The first two do not look at the room (cap_verts, cap_quads);
+// the others write within it.
+enum MeshStage { kMeshClassify, kMeshSums, kMeshList, kMeshVertices, kMeshQuads, kMeshStages };
+uint32_t mesh_blocks(const MeshArgs& a, int stage);  // workgroups (0: nothing to do)
+hipError_t mesh_stage(const MeshArgs& a, int stage, hipStream_t s);
+// The stage for many grids in one launch: job k (device array) owns the
+// workgroups base[k] .. base[k + 1) of `blocks`.
+hipError_t mesh_stage_multi(const MeshArgs* jobs, const uint32_t* base, uint32_t njobs, uint32_t blocks, int stage,
+	hipStream_t s);
 hipError_t mesh_pool_to_dense(const MeshArgs& a, float* dense, uint32_t k0, uint32_t nk, hipStream_t s);
 hipError_t mesh_dense_to_pool(const MeshArgs& a, const float* dense, hipStream_t s);
 hipError_t exclusive_scan_u32(const uint32_t* in, uint32_t* out, uint64_t n, void* temp, size_t& temp_bytes, hipStream_t s);
-// Exclusive scan of the quad counts (bits 0..2) of n quad-flag words.
-hipError_t exclusive_scan_quads(const uint32_t* flags, uint32_t* out, uint64_t n, void* temp, size_t& temp_bytes,
-	hipStream_t s);
 // Blocks (all n, or the n of `list`) ordered by their pruned program's cost,
 // most expensive first, into `order`; keys needs 2n words, values n.  With
 // temp = null only sizes temp_bytes.

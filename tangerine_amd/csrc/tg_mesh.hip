@@ -106,12 +106,12 @@ __device__ __forceinline__ uint32_t xcd_contiguous(uint32_t b, uint32_t n)
 	return x < rem ? x * (per + 1) + k : rem * (per + 1) + (x - rem) * per + k;
 }
 
-__global__ void __launch_bounds__(256) k_classify(MeshArgs a, uint32_t nseg)
+__device__ __forceinline__ void classify_block(const MeshArgs& a, uint32_t blk)
 {
 	constexpr uint32_t kTiles = kSegWords * 8 + 1;  // + the next tile, for the x + 1 corner
 	__shared__ uint64_t lds[8 * 8 * kSegWords];      // [kk][jj][8 tiles per word] bytes
 	__shared__ uint64_t all_s[kTiles * 8], any_s[kTiles * 8];
-	const uint32_t blk = xcd_contiguous(blockIdx.x, gridDim.x);
+	const uint32_t nseg = (a.aw + kSegWords - 1) / kSegWords;
 	const uint32_t seg = blk % nseg;
 	const uint32_t cy = (blk / nseg) % a.cby, cz = blk / (nseg * a.cby);
 	const uint32_t t0 = seg * kSegWords * 8;
@@ -223,27 +223,106 @@ __device__ __forceinline__ void place_vertex(const MeshArgs& a, uint32_t i, uint
 	v[2] = a.gz + (maxz - a.gz) * (gcz - 0.0f) / (fsz - 0.0f);
 }
 
-// Thread per four cube-row words (one 32-byte load when whole): each word's
-// active cubes into the cube list at their vertex ids.
-constexpr uint32_t kListWords = 4;
-
-__global__ void __launch_bounds__(256) k_list_cubes(MeshArgs a)
+// Sum of v over the workgroup (of 1024), in every thread; `part`: 16 words of LDS.
+__device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t* part)
 {
-	const uint64_t t = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-	const uint64_t total = uint64_t(a.sy) * a.sz * a.aw;
-	const uint64_t w0 = t * kListWords;
-	if (w0 >= total) return;
-	uint64_t act[kListWords] = { 0, 0, 0, 0 };
-	if (w0 + kListWords <= total)
+#pragma unroll
+	for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+	if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+	__syncthreads();
+	uint32_t total = 0;
+#pragma unroll
+	for (int w = 0; w < 16; ++w) total += part[w];
+	__syncthreads();
+	return total;
+}
+
+// Exclusive sum of v below the thread, and the workgroup's (of 1024) total.
+__device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t* part, uint32_t& total)
+{
+	const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	uint32_t p = v;
+#pragma unroll
+	for (uint32_t o = 1; o < 64; o <<= 1)
+	{
+		const uint32_t u = __shfl_up(p, o);
+		if (lane >= o) p += u;
+	}
+	if (lane == 63) part[wave] = p;
+	__syncthreads();
+	p -= v;
+	total = 0;
+#pragma unroll
+	for (uint32_t w = 0; w < 16; ++w)
+	{
+		if (w < wave) p += part[w];
+		total += part[w];
+	}
+	__syncthreads();
+	return p;
+}
+
+// Sum of the chunks' sums before chunk c.  (Every workgroup adds up those before
+// its own, 16 KiB for the last of 4096: less than a scan of its own costs in
+// launches, and no workgroup waits for another.)
+__device__ __forceinline__ uint32_t chunks_before(const uint32_t* sums, uint32_t c, uint32_t* part)
+{
+	uint32_t v = 0;
+	for (uint32_t k = threadIdx.x; k < c; k += 1024) v += sums[k];
+	return block_sum(v, part);
+}
+
+__device__ __forceinline__ uint64_t mesh_words(const MeshArgs& a) { return uint64_t(a.sy) * a.sz * a.aw; }
+
+// Workgroup per kMeshWords words: their active cubes.
+__device__ __forceinline__ void word_sums_block(const MeshArgs& a, uint32_t c)
+{
+	__shared__ uint32_t part[16];
+	const uint64_t total = mesh_words(a), w0 = uint64_t(c) * kMeshWords + threadIdx.x * 4;
+	uint32_t v = 0;
+	if (w0 + 4 <= total)
+	{
+		const uint4 n = *reinterpret_cast<const uint4*>(a.word_count + w0);
+		v = (n.x + n.y) + (n.z + n.w);
+	}
+	else
+		for (uint64_t w = w0; w < total; ++w) v += a.word_count[w];
+	v = block_sum(v, part);
+	if (threadIdx.x == 0) a.word_sums[c] = v;
+}
+
+// Workgroup per kMeshWords words, four to a thread (32 bytes of active bits in one
+// go): the words' vertex bases, and their active cubes into the cube list at
+// their vertex ids.  The last one writes the total.
+__device__ __forceinline__ void list_cubes_block(const MeshArgs& a, uint32_t c)
+{
+	__shared__ uint32_t part[16];
+	const uint64_t total = mesh_words(a), w0 = uint64_t(c) * kMeshWords + threadIdx.x * 4;
+	uint64_t act[4] = { 0, 0, 0, 0 };
+	const bool whole = w0 + 4 <= total;
+	if (whole)
 	{
 		const ulonglong2* src = reinterpret_cast<const ulonglong2*>(a.active + w0);
 		const ulonglong2 lo = src[0], hi = src[1];
 		act[0] = lo.x; act[1] = lo.y; act[2] = hi.x; act[3] = hi.y;
 	}
 	else
-		for (uint32_t q = 0; q < kListWords && w0 + q < total; ++q) act[q] = a.active[w0 + q];
+		for (uint32_t q = 0; q < 4 && w0 + q < total; ++q) act[q] = a.active[w0 + q];
+	const uint32_t before = chunks_before(a.word_sums, c, part);
+	uint32_t n[4], base[4];
 #pragma unroll
-	for (uint32_t q = 0; q < kListWords; ++q)
+	for (int q = 0; q < 4; ++q) n[q] = uint32_t(__popcll(act[q]));
+	uint32_t all;
+	base[0] = before + block_scan((n[0] + n[1]) + (n[2] + n[3]), part, all);
+#pragma unroll
+	for (int q = 1; q < 4; ++q) base[q] = base[q - 1] + n[q - 1];
+	if (whole)
+		*reinterpret_cast<uint4*>(a.word_base + w0) = make_uint4(base[0], base[1], base[2], base[3]);
+	else
+		for (uint32_t q = 0; q < 4 && w0 + q < total; ++q) a.word_base[w0 + q] = base[q];
+	if (threadIdx.x == 0 && (uint64_t(c) + 1) * kMeshWords >= total) a.tail[0] = before + all;
+#pragma unroll
+	for (uint32_t q = 0; q < 4; ++q)
 	{
 		uint64_t bits = act[q];
 		if (!bits) continue;
@@ -251,7 +330,7 @@ __global__ void __launch_bounds__(256) k_list_cubes(MeshArgs a)
 		const uint32_t row = div_magic(wi, a.aw_div);
 		const uint32_t w = wi - row * a.aw;
 		const uint32_t base_index = w * 64 + row * a.sx;  // i + sx (j + sy k) for i = 64 w
-		uint32_t id = a.word_base[wi];
+		uint32_t id = base[q];
 		while (bits)
 		{
 			const int b = __ffsll((long long)bits) - 1;
@@ -300,56 +379,55 @@ __device__ __forceinline__ uint32_t quad_flags(const MeshArgs& a, uint32_t i, ui
 	return flags;
 }
 
-// Active cubes (vertices) of the classified grid: the scanned word counts' total.
-__device__ __forceinline__ uint64_t active_cubes(const MeshArgs& a)
+// Active cubes (vertices) of the listed grid, at most the room.
+__device__ __forceinline__ uint32_t active_cubes(const MeshArgs& a)
 {
-	const uint64_t last = uint64_t(a.sy) * a.sz * a.aw - 1;
-	return uint64_t(a.word_base[last]) + a.word_count[last];
+	const uint64_t last = mesh_words(a) - 1;
+	const uint64_t n = uint64_t(a.word_base[last]) + a.word_count[last];
+	return uint32_t(n < a.cap_verts ? n : a.cap_verts);
 }
 
-// Thread per active cube (launched for n >= the active cubes, within the
-// room cap_verts): vertex placement and the cube's quad flags (their quad
-// counts are scanned before k_quad_write); threads past the active cubes
-// write zero flags.
-__global__ void __launch_bounds__(256) k_vertices(MeshArgs a, uint64_t n)
+// Workgroup per kMeshCubes of the room, thread per active cube: vertex
+// placement, the cube's quad flags, and the workgroup's quads for k_mesh's next
+// stage.
+__device__ __forceinline__ void vertices_block(const MeshArgs& a, uint32_t c)
 {
-	const uint64_t id = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-	if (id >= n) return;
-	if (id == 0 && a.tail)
+	__shared__ uint32_t part[16];
+	const uint32_t n = active_cubes(a), id = c * kMeshCubes + threadIdx.x;
+	if (c * kMeshCubes >= n) return;
+	uint32_t flags = 0;
+	if (id < n)
 	{
-		const uint64_t last = uint64_t(a.sy) * a.sz * a.aw - 1;
-		a.tail[0] = a.word_base[last];
-		a.tail[1] = a.word_count[last];
+		uint32_t i, j, k;
+		cube_coords(a, a.cubes[id], i, j, k);
+		float s[8];
+		cube_corners(a, i, j, k, s);
+		place_vertex(a, i, j, k, s, a.vertices + size_t(id) * 3);
+		flags = quad_flags(a, i, j, k, s);
+		a.cube_quads[id] = flags;
 	}
-	if (id >= active_cubes(a))
+	const uint32_t quads = block_sum(uint32_t(__popc(flags & 7u)), part);
+	if (threadIdx.x == 0) a.quad_sums[c] = quads;
+}
+
+// The same workgroups: the active cubes' quads (vertex `id`: active cubes are
+// listed in vertex order), each as the two triangles (v0, v1, v2), (v0, v2, v3), when
+// they fit the room cap_quads.  The last one writes the total.
+__device__ __forceinline__ void quads_block(const MeshArgs& a, uint32_t c)
+{
+	__shared__ uint32_t part[16];
+	const uint32_t count = active_cubes(a), id = c * kMeshCubes + threadIdx.x;
+	if (c * kMeshCubes >= count)
 	{
-		a.cube_quads[id] = 0;
+		if (count == 0 && c == 0 && threadIdx.x == 0) a.tail[1] = 0;
 		return;
 	}
-	uint32_t i, j, k;
-	cube_coords(a, a.cubes[id], i, j, k);
-	float s[8];
-	cube_corners(a, i, j, k, s);
-	place_vertex(a, i, j, k, s, a.vertices + size_t(id) * 3);
-	a.cube_quads[id] = quad_flags(a, i, j, k, s);
-}
-
-// Thread per active cube (vertex `id`: active cubes are listed in vertex
-// order; launched like k_vertices): its quads at the scanned base, each as
-// the two triangles (v0, v1, v2), (v0, v2, v3), when they fit the room
-// cap_quads.
-__global__ void __launch_bounds__(256) k_quad_write(MeshArgs a, uint64_t n)
-{
-	const uint64_t id = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-	if (id >= n) return;
-	if (id == 0 && a.tail)
-	{
-		a.tail[2] = a.cube_qbase[n - 1];
-		a.tail[3] = a.cube_quads[n - 1];
-	}
-	const uint32_t flags = a.cube_quads[id];
+	const uint32_t flags = id < count ? a.cube_quads[id] : 0u;
+	const uint32_t before = chunks_before(a.quad_sums, c, part);
+	uint32_t all;
+	const uint32_t base = before + block_scan(uint32_t(__popc(flags & 7u)), part, all);
+	if (threadIdx.x == 0 && c * kMeshCubes + kMeshCubes >= count) a.tail[1] = before + all;
 	if ((flags & 7u) == 0) return;
-	const uint32_t base = a.cube_qbase[id];
 	if (uint64_t(base) + uint32_t(__popc(flags & 7u)) > a.cap_quads) return;  // no room: the caller redoes the mesh
 	uint32_t i, j, k;
 	cube_coords(a, a.cubes[id], i, j, k);
@@ -379,6 +457,48 @@ __global__ void __launch_bounds__(256) k_quad_write(MeshArgs a, uint64_t n)
 		tri[2] = make_uint2(v2, v3);
 		out += 6;
 	}
+}
+
+template <int STAGE>
+__device__ __forceinline__ void mesh_block(const MeshArgs& a, uint32_t blk)
+{
+	if (STAGE == kMeshClassify)
+		classify_block(a, blk);
+	else if (STAGE == kMeshSums)
+		word_sums_block(a, blk);
+	else if (STAGE == kMeshList)
+		list_cubes_block(a, blk);
+	else if (STAGE == kMeshVertices)
+		vertices_block(a, blk);
+	else
+		quads_block(a, blk);
+}
+
+constexpr unsigned mesh_threads(int stage) { return stage == kMeshClassify ? 256u : 1024u; }
+
+template <int STAGE>
+__global__ void __launch_bounds__(mesh_threads(STAGE)) k_mesh(MeshArgs a)
+{
+	mesh_block<STAGE>(a, STAGE == kMeshClassify ? xcd_contiguous(blockIdx.x, gridDim.x) : blockIdx.x);
+}
+
+// A batch's grids in one launch: with a launch per grid and stage, 24 grids were
+// 190 launches of a few microseconds each, one after another as they were issued.
+template <int STAGE>
+__global__ void __launch_bounds__(mesh_threads(STAGE)) k_mesh_multi(const MeshArgs* __restrict__ jobs,
+	const uint32_t* __restrict__ base, uint32_t njobs)
+{
+	const uint32_t blk = STAGE == kMeshClassify ? xcd_contiguous(blockIdx.x, gridDim.x) : blockIdx.x;
+	uint32_t lo = 0, hi = njobs;
+	while (hi - lo > 1)
+	{
+		const uint32_t mid = (lo + hi) / 2;
+		if (base[mid] <= blk)
+			lo = mid;
+		else
+			hi = mid;
+	}
+	mesh_block<STAGE>(jobs[lo], blk - base[lo]);
 }
 
 // Pool tiles -> dense x-fastest grid (for copying samples back to the host).
@@ -430,34 +550,32 @@ inline unsigned blocks_for(uint64_t n, unsigned threads) { return unsigned((n + 
 
 }  // namespace
 
-hipError_t mesh_classify(const MeshArgs& a, hipStream_t s)
+uint32_t mesh_blocks(const MeshArgs& a, int stage)
 {
-	const uint32_t nseg = (a.aw + kSegWords - 1) / kSegWords;
-	const uint64_t blocks = uint64_t(nseg) * a.cby * a.cbz;
+	const uint64_t words = uint64_t(a.sy) * a.sz * a.aw;
+	if (stage == kMeshClassify) return uint32_t(uint64_t((a.aw + kSegWords - 1) / kSegWords) * a.cby * a.cbz);
+	if (stage == kMeshSums || stage == kMeshList) return blocks_for(words, kMeshWords);
+	return blocks_for(a.cap_verts, kMeshCubes);
+}
+
+hipError_t mesh_stage(const MeshArgs& a, int stage, hipStream_t s)
+{
+	static void (*const kernels[kMeshStages])(MeshArgs) = { &k_mesh<0>, &k_mesh<1>, &k_mesh<2>, &k_mesh<3>, &k_mesh<4> };
+	const uint32_t blocks = mesh_blocks(a, stage);
 	if (blocks == 0) return hipSuccess;
-	if (blocks >= (1ull << 31)) return hipErrorInvalidValue;
-	hipLaunchKernelGGL(k_classify, dim3(unsigned(blocks)), dim3(256), 0, s, a, nseg);
+	if (blocks >= (1u << 31)) return hipErrorInvalidValue;
+	hipLaunchKernelGGL(kernels[stage], dim3(blocks), dim3(mesh_threads(stage)), 0, s, a);
 	return hipGetLastError();
 }
 
-hipError_t mesh_list_cubes(const MeshArgs& a, hipStream_t s)
+hipError_t mesh_stage_multi(const MeshArgs* jobs, const uint32_t* base, uint32_t njobs, uint32_t blocks, int stage,
+	hipStream_t s)
 {
-	const uint64_t n = uint64_t(a.sy) * a.sz * a.aw;
-	hipLaunchKernelGGL(k_list_cubes, dim3(blocks_for((n + kListWords - 1) / kListWords, 256)), dim3(256), 0, s, a);
-	return hipGetLastError();
-}
-
-hipError_t mesh_vertices(const MeshArgs& a, uint64_t nverts, hipStream_t s)
-{
-	if (nverts == 0) return hipSuccess;
-	hipLaunchKernelGGL(k_vertices, dim3(blocks_for(nverts, 256)), dim3(256), 0, s, a, nverts);
-	return hipGetLastError();
-}
-
-hipError_t mesh_quad_write(const MeshArgs& a, uint64_t nverts, hipStream_t s)
-{
-	if (nverts == 0) return hipSuccess;
-	hipLaunchKernelGGL(k_quad_write, dim3(blocks_for(nverts, 256)), dim3(256), 0, s, a, nverts);
+	static void (*const kernels[kMeshStages])(const MeshArgs*, const uint32_t*, uint32_t) = { &k_mesh_multi<0>,
+		&k_mesh_multi<1>, &k_mesh_multi<2>, &k_mesh_multi<3>, &k_mesh_multi<4> };
+	if (blocks == 0) return hipSuccess;
+	if (blocks >= (1u << 31)) return hipErrorInvalidValue;
+	hipLaunchKernelGGL(kernels[stage], dim3(blocks), dim3(mesh_threads(stage)), 0, s, jobs, base, njobs);
 	return hipGetLastError();
 }
 
@@ -480,20 +598,6 @@ hipError_t mesh_dense_to_pool(const MeshArgs& a, const float* dense, hipStream_t
 hipError_t exclusive_scan_u32(const uint32_t* in, uint32_t* out, uint64_t n, void* temp, size_t& temp_bytes, hipStream_t s)
 {
 	return hipcub::DeviceScan::ExclusiveSum(temp, temp_bytes, in, out, int(n), s);
-}
-
-namespace {
-struct QuadCount
-{
-	__host__ __device__ uint32_t operator()(uint32_t flags) const { return uint32_t(__builtin_popcount(flags & 7u)); }
-};
-}  // namespace
-
-hipError_t exclusive_scan_quads(const uint32_t* flags, uint32_t* out, uint64_t n, void* temp, size_t& temp_bytes,
-	hipStream_t s)
-{
-	hipcub::TransformInputIterator<uint32_t, QuadCount, const uint32_t*> counts(flags, QuadCount{});
-	return hipcub::DeviceScan::ExclusiveSum(temp, temp_bytes, counts, out, int(n), s);
 }
 
 namespace {
