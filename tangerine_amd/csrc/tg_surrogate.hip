@@ -48,6 +48,7 @@ struct tg_surrogate
 	float sigma = 2.0f;
 	float clamp = 0.5f;
 	uint64_t seed = 1;
+	tg_mesher* coarse = nullptr;  // of fits: the coarse export that surface samples come from
 	float margin = -1.0f;       // caller's fixed margin (< 0: use the calibration)
 	bool calibrated = false;
 	std::vector<float> calib_pred, calib_dist;  // held-out predictions and exact distances
@@ -233,6 +234,7 @@ extern "C" void tg_surrogate_destroy(tg_surrogate* s)
 		b->release();
 	for (hipEvent_t e : s->ev)
 		if (e) hipEventDestroy(e);
+	if (s->coarse) tg_mesher_destroy(s->coarse);
 	if (s->stream) hipStreamDestroy(s->stream);
 	delete s;
 }
@@ -340,10 +342,11 @@ extern "C" int tg_surrogate_fit(tg_surrogate* s, const tg_program* exact, uint64
 	auto t0 = std::chrono::steady_clock::now();
 
 	// 1. surface vertices from a coarse exact export of the domain (128 cells per axis)
-	tg_mesher* coarse = nullptr;
-	int rc = tg_mesher_create(&coarse);
+	// (its mesher is kept for the next fit: its two dozen allocations took longer
+	// than the export)
+	int rc = s->coarse ? int(TG_OK) : tg_mesher_create(&s->coarse);
 	if (rc) return rc;
-	struct MesherGuard { tg_mesher* m; ~MesherGuard() { tg_mesher_destroy(m); } } mg{ coarse };
+	tg_mesher* coarse = s->coarse;
 	tg_grid g{ s->lo[0], s->lo[1], s->lo[2], s->size / 128.0f, s->size / 128.0f, s->size / 128.0f, 128, 128, 128 };
 	rc = tg_mesher_export(coarse, exact, &g, flags & TG_FLAG_FAST);
 	if (rc) return rc;
