@@ -140,7 +140,13 @@ int WorkspaceLease::take(hipStream_t stream)
 	}
 	if (ws_)
 	{
-		if (!ws_->in_flight) return TG_OK;
+		if (!ws_->in_flight)
+		{
+			ws_->retired.clear();
+			return TG_OK;
+		}
+		ws_->retired.push_back(std::move(ws_->launches.host));
+		ws_->launches.host = {};
 		e = hipStreamWaitEvent(stream, ws_->busy, 0);
 		return e == hipSuccess ? TG_OK : hip_fail(e, "workspace wait");
 	}
@@ -661,11 +667,6 @@ int sorted_launches(const tg_program* p, SortedPointsArgs& sa, float edge, float
 		g.radius = 0.5f * cell * 1.7320508f * (1.0f + 1.0e-3f) + 1.0e-6f * (reach + 4.0f * edge);
 		g.words = true;
 	}
-	if (ws.in_flight)
-		ws.retired.push_back(std::move(ws.launches.host));
-	else
-		ws.retired.clear();
-	ws.launches.host = {};
 	const tg_program* progs[2] = { p, p };
 	CellPrograms* outs[2] = { &ws.levels[0], &ws.levels[1] };
 	int rc = prune_cells_many(s, progs, grids, 2, fast, outs, ws.launches);

@@ -60,6 +60,7 @@ struct tg_tracer
 	int first_budget = kFirstBudget, budget = kPassBudget;
 	uint32_t resume_waves = kResumeWaves;
 	CellPrograms levels[kTraceLevels];
+	PruneLaunches launches;
 	float dom_lo[3] = { 0, 0, 0 };
 	float dom_size = 0.0f;        // 0: derived from the camera
 	uint32_t width = 0, height = 0;
@@ -78,20 +79,32 @@ struct CubeDomain
 };
 
 // Levels coarse to fine: doms[L] split into ns[L]^3 cells.  Every level's
-// passes are issued before the first is waited for.
+// passes of a stage are one launch: the coarse levels' are shorter than a launch
+// is apart from the next (a frame of 256 primitives, four levels one after another 0.55 ms, so 0.39).
 int build_levels(hipStream_t stream, const tg_program* p, const CubeDomain* doms, const uint32_t* ns, int count,
-	bool fast, CellPrograms* levels, TraceArgs& ta)
+	bool fast, CellPrograms* levels, PruneLaunches& work, TraceArgs& ta)
 {
 	ta.nlevels = 0;
 	count = std::min(count, kTraceLevels);
+	const tg_program* progs[kTraceLevels];
+	CellPrograms* outs[kTraceLevels];
+	CellGrid grids[kTraceLevels];
 	for (int L = 0; L < count; ++L)
 	{
 		const float cell = doms[L].size / float(ns[L]);
-		const float c3[3] = { cell, cell, cell };
-		const uint32_t counts[3] = { ns[L], ns[L], ns[L] };
-		int rc = prune_cells_start(stream, p, doms[L].lo, c3, 0.5f * cell * 1.7320508f, counts, fast, levels[L]);
-		if (rc) return rc;
+		CellGrid& g = grids[L];
+		for (int i = 0; i < 3; ++i)
+		{
+			g.origin[i] = doms[L].lo[i];
+			g.cell[i] = cell;
+			g.counts[i] = ns[L];
+		}
+		g.radius = 0.5f * cell * 1.7320508f;
+		progs[L] = p;
+		outs[L] = &levels[L];
 	}
+	int rc = prune_cells_many(stream, progs, grids, uint32_t(count), fast, outs, work);
+	if (rc) return rc;
 	for (int L = 0; L < count; ++L)
 	{
 		const CubeDomain& dom = doms[L];
@@ -99,7 +112,7 @@ int build_levels(hipStream_t stream, const tg_program* p, const CubeDomain* doms
 		const float cell = dom.size / float(n);
 		const float c3[3] = { cell, cell, cell };
 		const uint32_t counts[3] = { n, n, n };
-		int rc = prune_cells_finish(stream, p, dom.lo, c3, counts, fast, levels[L]);
+		rc = prune_cells_finish(stream, p, dom.lo, c3, counts, fast, levels[L]);
 		if (rc) return rc;
 		if (!levels[L].valid) return TG_OK;
 		ta.levels[L] = TraceLevel{ levels[L].desc.as<const BlockDesc>(), levels[L].pool.as<const Entry>(), n, cell,
@@ -234,6 +247,7 @@ extern "C" void tg_tracer_destroy(tg_tracer* tr)
 		b->release();
 	if (tr->host_count) (void)hipHostFree(tr->host_count);
 	for (CellPrograms& l : tr->levels) l.release();
+	tr->launches.dev.release();
 	for (hipEvent_t e : tr->ev)
 		if (e) hipEventDestroy(e);
 	if (tr->stream) hipStreamDestroy(tr->stream);
@@ -336,7 +350,7 @@ extern "C" int tg_tracer_render(tg_tracer* tr, const tg_program* p, const tg_cam
 			doms[count] = inner;
 			ns[count++] = n;
 		}
-		rc = build_levels(tr->stream, p, doms, ns, count, fast, tr->levels, ta);
+		rc = build_levels(tr->stream, p, doms, ns, count, fast, tr->levels, tr->launches, ta);
 		if (rc) return rc;
 	}
 	TG_CHECK_HIP(hipEventRecord(tr->ev[1], tr->stream), "event");
@@ -579,7 +593,7 @@ extern "C" int tg_raymarch(const tg_program* p, const float* starts, const float
 	TG_CHECK_HIP(hipMemsetAsync(ws->ctl.ptr, 0, 256, nullptr), "ray queue reset");
 	TraceArgs& ta = fa.t;
 	base_args(ta, p);
-	rc = build_levels(nullptr, p, doms, ns, cubes, fast, ws->levels, ta);
+	rc = build_levels(nullptr, p, doms, ns, cubes, fast, ws->levels, ws->launches, ta);
 	if (rc) return rc;
 	ta.starts = ds;
 	ta.dirs = dd;
