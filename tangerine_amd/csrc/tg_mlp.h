@@ -51,10 +51,8 @@ struct PredictArgs
 struct TrainArgs
 {
 	Net net;
-	const float* xyz;         // training points
-	const float* target;      // exact distances
-	const uint32_t* order;    // sample permutation
-	uint64_t batch_offset;    // first sample of the batch in `order`
+	const float4* samples;    // in training order: x, y, z, exact distance
+	uint64_t batch_offset;    // first sample of the batch
 	uint32_t batch;           // samples per batch (multiple of 32)
 	uint32_t groups_per_block;  // 1 or 2
 	float* partial;           // [blocks][kParams] gradients of the mean squared error
@@ -84,6 +82,9 @@ hipError_t prepare();
 hipError_t launch_predict(const PredictArgs& a, hipStream_t s);
 hipError_t launch_train_grad(const TrainArgs& a, uint32_t blocks, hipStream_t s);
 hipError_t launch_adam(const AdamArgs& a, hipStream_t s);
+// samples[k] = point and distance order[k] (order null: k).
+hipError_t launch_gather_samples(const float* xyz, const float* target, const uint32_t* order, float4* samples,
+	uint64_t n, hipStream_t s);
 hipError_t launch_epoch_advance(uint64_t* epoch, hipStream_t s);
 
 }  // namespace mlp

@@ -336,15 +336,15 @@ __global__ void __launch_bounds__(64 * kTrainWaves) k_train_grad(TrainArgs t)
 	const float scale = 2.0f / float(t.batch);
 	float target[2];
 #pragma unroll
-	for (int n = 0; n < 2; ++n) target[n] = t.target[t.order[s0 + 16 * n + r]];
+	for (int n = 0; n < 2; ++n) target[n] = t.samples[s0 + 16 * n + r].w;
+	const float4 sample = t.samples[s0 + (lane & 31)];
 	if (live)
 	{
 		// 12 of the 96 features of a point to each lane (lanes 0..31 sines, 32..63 cosines)
 		const int pt = lane & 31, c = lane >> 5;
-		const uint32_t idx = t.order[s0 + pt];
-		const float x = (t.xyz[3 * idx] - t.net.lo[0]) * t.net.inv_half - 1.0f;
-		const float y = (t.xyz[3 * idx + 1] - t.net.lo[1]) * t.net.inv_half - 1.0f;
-		const float z = (t.xyz[3 * idx + 2] - t.net.lo[2]) * t.net.inv_half - 1.0f;
+		const float x = (sample.x - t.net.lo[0]) * t.net.inv_half - 1.0f;
+		const float y = (sample.y - t.net.lo[1]) * t.net.inv_half - 1.0f;
+		const float z = (sample.z - t.net.lo[2]) * t.net.inv_half - 1.0f;
 		const float* fr = t.net.fourier + 3 * (kFreq / 4) * m;
 		const int k0 = kFreq * c + (kFreq / 4) * m;
 		uint16_t b[kFreq / 4];
@@ -588,6 +588,15 @@ __global__ void __launch_bounds__(64 * kAdamWaves) k_adam(AdamArgs a)
 	}
 }
 
+__global__ void __launch_bounds__(256) k_gather_samples(const float* xyz, const float* target, const uint32_t* order,
+	float4* samples, uint64_t n)
+{
+	const uint64_t k = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+	if (k >= n) return;
+	const uint64_t i = order ? order[k] : k;
+	samples[k] = make_float4(xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2], target[i]);
+}
+
 __global__ void k_epoch_advance(uint64_t* epoch) { *epoch += 1; }
 
 }  // namespace
@@ -620,6 +629,14 @@ hipError_t launch_train_grad(const TrainArgs& t, uint32_t blocks, hipStream_t s)
 hipError_t launch_adam(const AdamArgs& a, hipStream_t s)
 {
 	hipLaunchKernelGGL(k_adam, dim3((kParams + 63) / 64), dim3(64 * kAdamWaves), 0, s, a);
+	return hipGetLastError();
+}
+
+hipError_t launch_gather_samples(const float* xyz, const float* target, const uint32_t* order, float4* samples,
+	uint64_t n, hipStream_t s)
+{
+	if (n == 0) return hipSuccess;
+	hipLaunchKernelGGL(k_gather_samples, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, xyz, target, order, samples, n);
 	return hipGetLastError();
 }
 

@@ -56,7 +56,7 @@ struct tg_surrogate
 	// last threshold per mode (uncertified, certified) and the r it was for;
 	// cleared whenever the calibration changes
 	mutable float cache_r[2] = { -1.0f, -1.0f }, cache_t[2] = { 0.0f, 0.0f };
-	DevBuf params, fourier, adam_m, adam_v, xyz, target, order, partial, loss_partial, counters, loss_log, tmp;
+	DevBuf params, fourier, adam_m, adam_v, xyz, target, order, samples, partial, loss_partial, counters, loss_log, tmp;
 	tg_surrogate_stats stats{};
 };
 
@@ -229,7 +229,7 @@ extern "C" void tg_surrogate_destroy(tg_surrogate* s)
 {
 	if (!s) return;
 	if (s->stream) hipStreamSynchronize(s->stream);
-	for (DevBuf* b : { &s->params, &s->fourier, &s->adam_m, &s->adam_v, &s->xyz, &s->target, &s->order, &s->partial,
+	for (DevBuf* b : { &s->params, &s->fourier, &s->adam_m, &s->adam_v, &s->xyz, &s->target, &s->order, &s->samples, &s->partial,
 	                   &s->loss_partial, &s->counters, &s->loss_log, &s->tmp })
 		b->release();
 	for (hipEvent_t e : s->ev)
@@ -283,25 +283,22 @@ extern "C" int tg_surrogate_gradients(tg_surrogate* s, const float* xyz, const f
 	if (!s || !xyz || !target || !grad) return fail(TG_ERR_INVALID, "tg_surrogate_gradients: null argument");
 	if (n == 0 || n % mlp::kGroup || n >= (1ull << 31))
 		return fail(TG_ERR_INVALID, "tg_surrogate_gradients: n must be a positive multiple of 32");
-	DevBuf dx, dt, dord, dpart, dloss;
-	struct Guard { DevBuf* b[5]; ~Guard() { for (DevBuf* x : b) x->release(); } } guard{ { &dx, &dt, &dord, &dpart, &dloss } };
+	DevBuf dx, dt, dsamples, dpart, dloss;
+	struct Guard { DevBuf* b[5]; ~Guard() { for (DevBuf* x : b) x->release(); } } guard{ { &dx, &dt, &dsamples, &dpart, &dloss } };
 	const uint32_t blocks = uint32_t(n / mlp::kGroup);
 	int rc = dx.ensure(n * 12);
 	if (!rc) rc = dt.ensure(n * 4);
-	if (!rc) rc = dord.ensure(n * 4);
+	if (!rc) rc = dsamples.ensure(n * 16);
 	if (!rc) rc = dpart.ensure(size_t(blocks) * mlp::kParams * 4);
 	if (!rc) rc = dloss.ensure(blocks * 4);
 	if (rc) return rc;
-	std::vector<uint32_t> ord(n);
-	std::iota(ord.begin(), ord.end(), 0u);
 	TG_CHECK_HIP(hipMemcpy(dx.ptr, xyz, n * 12, hipMemcpyHostToDevice), "upload");
 	TG_CHECK_HIP(hipMemcpy(dt.ptr, target, n * 4, hipMemcpyHostToDevice), "upload");
-	TG_CHECK_HIP(hipMemcpy(dord.ptr, ord.data(), n * 4, hipMemcpyHostToDevice), "upload");
+	TG_CHECK_HIP(mlp::launch_gather_samples(dx.as<const float>(), dt.as<const float>(), nullptr, dsamples.as<float4>(), n,
+		s->stream), "samples launch");
 	mlp::TrainArgs ta{};
 	ta.net = surrogate_net(s);
-	ta.xyz = dx.as<const float>();
-	ta.target = dt.as<const float>();
-	ta.order = dord.as<const uint32_t>();
+	ta.samples = dsamples.as<const float4>();
 	ta.batch_offset = 0;
 	ta.batch = uint32_t(n);
 	ta.groups_per_block = 1;
@@ -375,6 +372,11 @@ extern "C" int tg_surrogate_fit(tg_surrogate* s, const tg_program* exact, uint64
 	rc = s->order.ensure(n_train * 4);
 	if (rc) return rc;
 	TG_CHECK_HIP(hipMemcpy(s->order.ptr, ord.data(), n_train * 4, hipMemcpyHostToDevice), "order upload");
+	// the samples once in training order, so that no step chases the permutation
+	rc = s->samples.ensure(n_train * 16);
+	if (rc) return rc;
+	TG_CHECK_HIP(mlp::launch_gather_samples(s->xyz.as<const float>(), s->target.as<const float>(),
+		s->order.as<const uint32_t>(), s->samples.as<float4>(), n_train, s->stream), "samples launch");
 	const uint64_t total_steps = batches * epochs;
 	rc = s->partial.ensure(size_t(blocks) * mlp::kParams * 4);
 	if (!rc) rc = s->loss_partial.ensure(blocks * 4);
@@ -387,9 +389,7 @@ extern "C" int tg_surrogate_fit(tg_surrogate* s, const tg_program* exact, uint64
 	uint64_t* epoch = s->counters.as<uint64_t>();
 	mlp::TrainArgs ta{};
 	ta.net = surrogate_net(s);
-	ta.xyz = s->xyz.as<const float>();
-	ta.target = s->target.as<const float>();
-	ta.order = s->order.as<const uint32_t>();
+	ta.samples = s->samples.as<const float4>();
 	ta.batch = batch;
 	ta.groups_per_block = groups_per_block;
 	ta.partial = s->partial.as<float>();
