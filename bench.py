@@ -90,10 +90,12 @@ def roofline(flops: float, ms: float, kernel: str, **extra) -> dict:
     return out
 
 
-def block_kernel(st: dict, prune: bool) -> str:
+def block_kernel(st: dict, prune: bool, tuning: dict | None) -> str:
     """The grid-evaluation kernel an export's stats describe."""
     if not prune:
         return "k_eval_tiles"
+    if not st["block_workgroups"] and (tuning is None or tuning["workgroups_per_cu"]):
+        return f"k_eval_tile_programs ({st['points_per_lane']} points per lane)"
     if st["block_workgroups"]:
         return f"k_eval_batch<{st['points_per_lane']},true> (persistent block evaluation, one tree)"
     return f"k_eval_blocks<{st['points_per_lane']}>"
@@ -476,7 +478,7 @@ def main(argv=None) -> int:
     nverts, ntris = mesher.counts()
     prune = not args.no_prune
     launch_ms = res["block_ms"] if prune and res["block_ms"] > 0 else res["eval_ms"]
-    kernel = block_kernel(st, prune)
+    kernel = block_kernel(st, prune, tuning)
     traffic = MEASURED_TRAFFIC_BYTES.get(args.workload) if prune and not args.fast else None
     rl = roofline(st["flops"], launch_ms, kernel,
                   traffic=traffic,
@@ -519,7 +521,7 @@ def main(argv=None) -> int:
                                       f"{args.workload} fast")
         fms = fres["block_ms"] if prune and fres["block_ms"] > 0 else fres["eval_ms"]
         out["fast"] = {"ms_per_step": fres["ms_per_step"], "samples_per_s": samples / (fres["ms_per_step"] * 1e-3),
-                       "autotune": ftune, "roofline": roofline(fst["flops"], fms, block_kernel(fst, prune) + " (fast numerics)")}
+                       "autotune": ftune, "roofline": roofline(fst["flops"], fms, block_kernel(fst, prune, ftune) + " (fast numerics)")}
         # back to the exact export (and its launch shape) for the surrogate leg's comparison
         if tuning:
             mesher.set_tuning(tuning["points_per_lane"], tuning["waves"], tuning.get("min_prune_len", 0),
@@ -548,7 +550,7 @@ def main(argv=None) -> int:
         out["export512"] = {"workload": "256 random primitives (seed 1), 512^3 cells over [-6,6]^3",
                             "samples": n2, "ms_per_step": r2["ms_per_step"], "export_ms_device": r2["export_ms_device"],
                             "samples_per_s": n2 / (r2["ms_per_step"] * 1e-3), "autotune": t2,
-                            "roofline": roofline(st2["flops"], ms2, block_kernel(st2, prune),
+                            "roofline": roofline(st2["flops"], ms2, block_kernel(st2, prune, t2),
                                                  traffic=MEASURED_TRAFFIC_BYTES["export512"]
                                                  if prune and not args.fast else None)}
 

@@ -402,17 +402,20 @@ int prune_blocks(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t f
 	return prune_blocks_finish(m, p, g, flags);
 }
 
-// Grids whose tiles x program entries stay below this are pruned per 8^3
-// tile in grid-wide passes and evaluated a wave per tile, without blocks.  The
-// passes evaluate every entry at every tile's centre, so their cost grows with
-// this product; the block evaluators' per-block prologue, run by one wave,
-// costs a latency that few blocks cannot hide.
-constexpr uint64_t kTileEntryCells = 150ull << 20;
+// Grids of few tiles are pruned per 8^3 tile in grid-wide passes and evaluated a
+// wave per tile, without blocks.  The passes evaluate every entry at every tile's
+// centre and a tile has its own program to emit and read; the block evaluators'
+// per-block prologue, run by one wave, costs a latency that few blocks cannot hide.
+// (Export, tiles / blocks, ms: 64^3 of 256 primitives 0.21 / 3.7, 256^3 of 2048 1.14 /
+// 5.1, 320^3 of 2048 1.47 / 3.6, 400^3 of 32 0.34 / 0.42, of 256 0.65 / 0.93, of 2048 2.35 /
+// 3.05, 450^3 of 600 1.46 / 1.73, of 1000 1.85 / 1.70, 480^3 of 256 0.95 / 0.97, 512^3 of 256
+// 1.16 / 0.95, 700^3 of 100 1.85 / 1.33, 1024^3 of 32 3.6 / 2.6.)
+constexpr uint64_t kTileWork = 1310ull << 20, kTileEntries = 6144;
 
 bool tile_programs(const tg_program* p, const MeshArgs& ma)
 {
 	const uint64_t tiles = uint64_t(ma.tx) * ma.ty * ma.tz;
-	return tiles * p->decoded.entries.size() <= kTileEntryCells && treelet_prunable(p, tiles);
+	return tiles * (p->decoded.entries.size() + kTileEntries) <= kTileWork && treelet_prunable(p, tiles);
 }
 
 // The 8^3-sample tiles as cells (samples lie within 3.5 |d| of a tile's centre).
@@ -1543,19 +1546,19 @@ extern "C" int tg_mesher_copy_normals(const tg_mesher* m, float* normals)
 
 namespace {
 
-// Point grids whose tiles x program entries are within kTileEntryCells, and
-// whose cells x entries x (1 + refinement steps) reach this, go through one
-// program per 8^3 cells: below it the whole program at every cell is over before
+// Point grids whose cells x entries x (1 + refinement steps) reach this go
+// through one program per 8^3 cells (while the passes' scratch, a quarter byte an
+// entry and tile, stays within 150 MiB): below it the whole program at every cell is over before
 // the passes are.  (Whole call, whole program / tiles: 64 primitives unrefined
 // 32 Mi entry-cells 134 / 177 us, 121 Mi 225 / 190; 256 primitives unrefined 54 Mi
 // 250 / 245, two steps 16 Mi 937 / 1087, 54 Mi 935 / 733, 2 Gi 2404 / 388.)
-constexpr uint64_t kCloudEntryCells = 120ull << 20;
+constexpr uint64_t kCloudEntryCells = 120ull << 20, kCloudEntryTiles = 600ull << 20;
 
 bool cloud_tiles(const tg_program* p, const CloudArgs& a)
 {
 	const uint64_t t = kTile, entries = p->decoded.entries.size();
 	const uint64_t tiles = (a.ix + t - 1) / t * ((a.iy + t - 1) / t) * ((a.iz + t - 1) / t);
-	return a.cells * entries * (1 + uint64_t(a.iterations)) >= kCloudEntryCells && tiles * entries <= kTileEntryCells && treelet_prunable(p, tiles);
+	return a.cells * entries * (1 + uint64_t(a.iterations)) >= kCloudEntryCells && tiles * entries <= kCloudEntryTiles && treelet_prunable(p, tiles);
 }
 
 // The tiles' programs, valid within 4 cell diagonals of a tile's centre: its
