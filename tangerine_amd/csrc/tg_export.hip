@@ -62,6 +62,7 @@ struct tg_mesher
 	// launch shape of culled exports (tg_mesher_set_culled_tuning): their
 	// near-surface tiles run deeper programs, which want more spill room per
 	// wave than the plain export's tuning may leave
+	bool culled_by_blocks = false;  // a launch shape was set for culled exports
 	int culled_points_per_lane = 4, culled_waves = 4, culled_workgroups_per_cu = 6;
 	// tg_mesher_set_tuning / set_emission were called: exports then evaluate by
 	// blocks, whatever the grid (see tile_programs)
@@ -410,12 +411,15 @@ int prune_blocks(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t f
 // 5.1, 320^3 of 2048 1.47 / 3.6, 400^3 of 32 0.34 / 0.42, of 256 0.65 / 0.93, of 2048 2.35 /
 // 3.05, 450^3 of 600 1.46 / 1.73, of 1000 1.85 / 1.70, 480^3 of 256 0.95 / 0.97, 512^3 of 256
 // 1.16 / 0.95, 700^3 of 100 1.85 / 1.33, 1024^3 of 32 3.6 / 2.6.)
-constexpr uint64_t kTileWork = 1310ull << 20, kTileEntries = 6144;
+// Culled exports prune the tiles that they then skip too: 128^3 of 2048 primitives
+// 1.4 / 20, 320^3 of 16 0.33 / 0.42, of 2048 1.6 / 3.7, 400^3 of 16 0.47 / 0.42, 450^3 of 256
+// 0.96 / 0.84.
+constexpr uint64_t kTileWork = 1310ull << 20, kCulledTileWork = 700ull << 20, kTileEntries = 6144;
 
-bool tile_programs(const tg_program* p, const MeshArgs& ma)
+bool tile_programs(const tg_program* p, const MeshArgs& ma, bool culled = false)
 {
-	const uint64_t tiles = uint64_t(ma.tx) * ma.ty * ma.tz;
-	return tiles * (p->decoded.entries.size() + kTileEntries) <= kTileWork && treelet_prunable(p, tiles);
+	const uint64_t tiles = uint64_t(ma.tx) * ma.ty * ma.tz, limit = culled ? kCulledTileWork : kTileWork;
+	return tiles * (p->decoded.entries.size() + kTileEntries) <= limit && treelet_prunable(p, tiles);
 }
 
 // The 8^3-sample tiles as cells (samples lie within 3.5 |d| of a tile's centre).
@@ -651,13 +655,19 @@ int eval_blocks(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t fl
 
 // Evaluation of every tile from its own program (m->blocks pruned per tile).
 // Asynchronous, read as eval_blocks is.
-int eval_tile_programs(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t flags)
+int eval_tile_programs(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t flags, bool masked)
 {
 	int rc = m->counters.ensure(kWorkBytes);
 	if (rc) return rc;
 	unsigned long long* work = m->counters.as<unsigned long long>();
 	TG_CHECK_HIP(hipMemsetAsync(m->counters.ptr, 0, kWorkBytes, m->stream), "counter reset");
-	const TileEvalArgs ta = tile_args(m, p, g, work);
+	TileEvalArgs ta = tile_args(m, p, g, work);
+	if (masked)
+	{
+		ta.tile_mask = m->tile_mask.as<const uint64_t>();
+		ta.bx = (ta.tx + kBlockTiles - 1) / kBlockTiles;
+		ta.by = (ta.ty + kBlockTiles - 1) / kBlockTiles;
+	}
 	m->last_points_per_lane = int(ta.points);
 	m->last_waves = int(kTileEvalWaves);
 	m->last_workgroups = 0;
@@ -763,7 +773,7 @@ struct Selection
 };
 
 int select_tiles(tg_mesher* m, const tg_program* p, const tg_grid* g, const tg_surrogate* s, bool certify, bool tiles,
-	uint32_t flags, Selection& sel)
+	bool by_tiles, uint32_t flags, Selection& sel)
 {
 	MeshArgs& ma = m->args;
 	const uint32_t bx = (ma.tx + kBlockTiles - 1) / kBlockTiles, by = (ma.ty + kBlockTiles - 1) / kBlockTiles,
@@ -820,6 +830,12 @@ int select_tiles(tg_mesher* m, const tg_program* p, const tg_grid* g, const tg_s
 		ca.bx = bx; ca.by = by; ca.bz = bz;
 		ca.cbx = ma.cbx; ca.cby = ma.cby; ca.cbz = ma.cbz;
 		ca.radius = radius * (1.0f + 1.0e-5f) + rounding_slack(p->decoded, grid_reach(g));
+		if (by_tiles)
+		{
+			ca.words = m->blocks.pool.as<const uint32_t>();
+			ca.tile_desc = m->blocks.desc.as<const BlockDesc>();
+			ca.tx = ma.tx; ca.ty = ma.ty;
+		}
 		ca.flags = m->brick_flags.as<uint8_t>();
 		ca.counters = ctr;
 		ca.slots = std::max<uint32_t>(1, std::max(blocks ? m->blocks.max_stack : 0u, p->decoded.max_stack) - 1);
@@ -830,10 +846,11 @@ int select_tiles(tg_mesher* m, const tg_program* p, const tg_grid* g, const tg_s
 		m->brick_flags.as<const uint8_t>(), ma.cbx, ma.cby, ma.cbz, ma.tx, ma.ty, ma.tz, bx, by, bz,
 		m->tile_mask.as<unsigned long long>(), ctr);
 	TG_CHECK_HIP(hipGetLastError(), "tile selection launch");
-	if (tiles)
+	// (evaluation by tiles reads the mask)
+	if (tiles && !by_tiles)
 		hipLaunchKernelGGL(k_list_tiles, dim3(grid_for(ntiles)), dim3(256), 0, m->stream,
 			m->tile_mask.as<const unsigned long long>(), ma.tx, ma.ty, ma.tz, bx, by, m->tile_list.as<uint32_t>(), ctr + 1);
-	else
+	else if (!by_tiles)
 		hipLaunchKernelGGL(k_list_blocks, dim3(grid_for(nblocks)), dim3(256), 0, m->stream,
 			m->tile_mask.as<const unsigned long long>(), uint32_t(nblocks), m->block_list.as<uint32_t>(), ctr + 1);
 	TG_CHECK_HIP(hipGetLastError(), "list launch");
@@ -887,7 +904,7 @@ int run_export(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t fla
 	TG_CHECK_HIP(hipEventRecord(m->ev[0], m->stream), "event");
 	m->blocks.valid = false;
 	bool sorted = false;
-	const bool by_tiles = !culled && !m->by_blocks && !(flags & TG_FLAG_NO_PRUNE) && tile_programs(p, ma);
+	const bool by_tiles = !(culled ? m->culled_by_blocks : m->by_blocks) && !(flags & TG_FLAG_NO_PRUNE) && tile_programs(p, ma, culled);
 	if (by_tiles)
 	{
 		const BlockGrid t = tile_grid(m, g);
@@ -918,7 +935,7 @@ int run_export(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t fla
 	Selection sel;
 	if (culled)
 	{
-		rc = select_tiles(m, p, g, sur, certify, !blocks, flags, sel);
+		rc = select_tiles(m, p, g, sur, certify, !blocks, by_tiles, flags, sel);
 		if (rc) return rc;
 	}
 	TG_CHECK_HIP(hipEventRecord(m->ev[3], m->stream), "event");
@@ -926,7 +943,7 @@ int run_export(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t fla
 	double flops = 0.0;
 	if (by_tiles)
 	{
-		rc = eval_tile_programs(m, p, g, flags);
+		rc = eval_tile_programs(m, p, g, flags, culled);
 		if (rc) return rc;
 	}
 	else if (blocks)
@@ -959,7 +976,7 @@ int run_export(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t fla
 	{
 		rc = eval_blocks_read(m, &evals, &flops);
 		if (rc) return rc;
-		if (by_tiles) evals = uint64_t(ga.ntiles) * kTileSamples;
+		if (by_tiles && !culled) evals = uint64_t(ga.ntiles) * kTileSamples;
 	}
 	float t_pre = 0, t_eval = 0, t_mesh = 0, t_all = 0;
 	TG_CHECK_HIP(hipEventElapsedTime(&t_pre, m->ev[0], m->ev[3]), "timing");
@@ -1079,6 +1096,7 @@ extern "C" int tg_mesher_set_culled_tuning(tg_mesher* m, uint32_t points_per_lan
 		return fail(TG_ERR_INVALID,
 			"tg_mesher_set_culled_tuning: points per lane in {2,4,8}, waves in {1,2,4}, workgroups per CU 0..16");
 	if (int rc = refuse_batch_owned(m, "tg_mesher_set_culled_tuning")) return rc;
+	m->culled_by_blocks = true;
 	m->culled_points_per_lane = int(points_per_lane);
 	m->culled_waves = int(waves);
 	m->culled_workgroups_per_cu = int(workgroups_per_cu);

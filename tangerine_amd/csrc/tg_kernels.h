@@ -219,7 +219,9 @@ struct TileEvalArgs
 	float* out_pool;
 	uint8_t* signs;              // 64 bytes per tile id (see GridArgs)
 	uint32_t slots;              // LDS spill slots per wave, each P floats per lane
-	unsigned long long* work;    // slots (kWorkBytes): 1 cost units over the grid's samples
+	unsigned long long* work;    // slots (kWorkBytes): 0 samples evaluated (with a mask), 1 cost units over the grid's samples
+	const uint64_t* tile_mask;   // per block of 4^3 tiles: tiles to evaluate (null: all)
+	uint32_t bx, by;             // blocks per axis, of the mask
 };
 constexpr uint32_t kTileEvalWaves = 4;  // waves per workgroup
 
@@ -260,6 +262,10 @@ struct CertifyArgs
 	uint8_t* flags;
 	unsigned long long* counters;  // slots (kWorkBytes): 2 bricks newly flagged, 3 cost units executed
 	uint32_t slots;
+	// one program per tile instead (TileEvalArgs), or null
+	const uint32_t* words;
+	const BlockDesc* tile_desc;
+	uint32_t tx, ty;             // tiles per axis
 };
 
 // ---- sphere tracing -------------------------------------------------------------
