@@ -381,8 +381,8 @@ int tg_mesher_copy_normals(const tg_mesher* mesher, float* normals);
  * persistent workgroups per CU, which take blocks from a queue and keep the
  * tables and tile programs in global scratch (LDS: the spill region only).
  * One work parameter: the shortest block program still pruned per tile.
- * Until set or tuned, points per lane go by the grid and the program (4, or 8
- * on large grids).
+ * Until set or tuned, points per lane and workgroups per CU go by the grid and
+ * the program.
  * tg_mesher_autotune prunes `program` for `grid`, times every launch on the
  * device, then the threshold at the fastest launch, and keeps the best for
  * later exports on this mesher.  Every setting writes the same samples. */

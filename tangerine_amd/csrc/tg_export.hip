@@ -56,7 +56,7 @@ struct tg_mesher
 	bool have_grid = false;
 	tg_export_stats stats{};
 	int points_per_lane = 4;      // block kernel: points per lane (2, 4, 8; tg_mesher_autotune)
-	bool shape_set = false;       // by the caller or autotune; else block_points
+	bool shape_set = false;       // by the caller or autotune; else block_shape
 	int waves = 2;                // block kernel: waves per workgroup (1, 2, 4)
 	int workgroups_per_cu = 8;    // 0: a workgroup per block (LDS tables); else persistent, global tables
 	// launch shape of culled exports (tg_mesher_set_culled_tuning): their
@@ -540,14 +540,27 @@ int block_order(tg_mesher* m, const BlockDesc* desc, const uint32_t* list, uint3
 	return TG_OK;
 }
 
-// Points per lane of a plain export's blocks where the caller has not set them:
-// 8 share an entry's decode and transform among more samples, 4 leave more waves
-// per block.  (Whole export, 4 / 8 points: 1024^3 of 2048 primitives 12.05 / 11.6 ms, of
-// 512 9.95 / 9.52, of 16 3.45 / 3.06; 800^3 of 2048 8.03 / 8.26, of 256 3.11 / 2.86; 700^3 of
-// 256 2.74 / 2.57; 600^3 of 512 2.44 / 2.76.)
-int block_points(const tg_program* p, uint32_t nblocks)
+// Launch shape of a plain export's blocks where the caller has not set one: points
+// per lane and workgroups per CU, of two waves.  Eight points share an entry's
+// decode and transform among more samples, four leave more waves to each block; a
+// few thousand blocks feed twelve workgroups a CU, fewer leave long queue tails.
+// (Whole export, ms, shape 4/8, 8/8, 4/12: 450^3 of 2048 primitives 2.68, 4.27, 2.86;
+// 512^3 of 16 0.64, 0.58, 0.60, of 256 0.98, 0.98, 0.94, of 2048 2.56, 3.46, 2.61; 600^3 of 100
+// 1.01, 0.89, 0.91, of 512 1.58, 1.76, 1.51, of 2048 3.32, 4.48, 3.25; 700^3 of 256 1.58, 1.42,
+// 1.47; 800^3 of 2048 5.11, 5.28, 4.79; 1024^3 of 16 3.15, 2.74, 2.84, of 512 4.63, 4.17, 4.25, of
+// 2048 7.21, 6.68, 6.57.)
+struct BlockShape
 {
-	return nblocks >= 24576 || (nblocks >= 8192 && p->decoded.entries.size() <= 1024) ? 8 : 4;
+	int points, workgroups_per_cu;
+};
+
+BlockShape block_shape(const tg_program* p, uint32_t nblocks, uint32_t max_depth)
+{
+	const size_t entries = p->decoded.entries.size();
+	if (nblocks >= 4096 && entries <= (nblocks >= 8192 ? 1024u : 256u)) return { 8, 8 };
+	const bool many = nblocks >= (entries <= 1024 ? 4096u : 6000u);
+	// (deep stacks: where twelve workgroups leave the spill region no room)
+	return { 4, many && block_lds_bytes_global(block_spill_slots(max_depth, 4), 4, 2) <= kMaxLds / 12 ? 12 : 8 };
 }
 
 // Pruned evaluation (k_eval_blocks) of the listed blocks' masked tiles, or of
@@ -565,9 +578,11 @@ int eval_blocks(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t fl
 	BlockEvalArgs ba = block_args(m, p, g, tile_mask, block_list, n_listed, work);
 	// culled exports (a block list) have their own launch shape
 	const bool culled = block_list != nullptr;
-	int pts = culled ? m->culled_points_per_lane : m->shape_set ? m->points_per_lane : block_points(p, ba.nblocks);
+	const BlockShape own = m->shape_set ? BlockShape{ m->points_per_lane, m->workgroups_per_cu }
+	                                    : block_shape(p, ba.nblocks, ba.max_depth);
+	int pts = culled ? m->culled_points_per_lane : own.points;
 	const int shape_waves = culled ? m->culled_waves : m->waves;
-	const int shape_wgs = culled ? m->culled_workgroups_per_cu : m->workgroups_per_cu;
+	const int shape_wgs = culled ? m->culled_workgroups_per_cu : own.workgroups_per_cu;
 	ba.waves = shape_waves;
 	if (shape_wgs > 0)
 	{
