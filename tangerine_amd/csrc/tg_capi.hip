@@ -198,14 +198,43 @@ namespace {
 // 373 / 335).  The bound is for the pinned memory an idle workspace keeps.
 constexpr size_t kDirectBytes = size_t(16) << 20;
 
+// Copies n words between device memory and the staging, both 16-byte aligned, on
+// the stream itself: a copy engine's transfer between kernels costs two waits for
+// another queue (100k gradients of 256 primitives 371 us with them).  Bound by the
+// host link.
+__global__ void __launch_bounds__(256) k_copy_words(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst, uint32_t n)
+{
+	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, quads = n / 4;
+	if (i < quads)
+		reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
+	else if (const uint32_t k = 4 * quads + (i - quads); k < n)
+		dst[k] = src[k];
+}
+
+__global__ void __launch_bounds__(256) k_zero_words(uint32_t* dst, uint32_t n)
+{
+	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+	if (i < n) dst[i] = 0;
+}
+
+// (n: at most kDirectBytes of words)
+hipError_t copy_words(const void* src, void* dst, uint64_t n)
+{
+	hipLaunchKernelGGL(k_copy_words, dim3(unsigned((n / 4 + 4 + 255) / 256)), dim3(256), 0, nullptr,
+		static_cast<const uint32_t*>(src), static_cast<uint32_t*>(dst), uint32_t(n));
+	return hipGetLastError();
+}
+
 }  // namespace
 
-int WorkspaceLease::stage(const float* host_xyz, uint64_t count, uint32_t width, const float** xyz, float** out)
+int WorkspaceLease::stage(const float* host_xyz, uint64_t count, uint32_t width, bool gathered, const float** xyz, float** out)
 {
-	const uint64_t bytes = count * (12 + 4 * width);
+	const uint64_t bytes = count * (12 + 4 * width) + 16;
 	size_t room = 65536;
 	while (room < bytes && room < kDirectBytes) room *= 2;
-	direct_ = bytes <= kDirectBytes && pinned(room) == TG_OK;
+	const bool held = bytes <= kDirectBytes && pinned(room) == TG_OK;
+	direct_ = held && !gathered;
+	copied_ = held && gathered;
 	if (direct_)
 	{
 		std::memcpy(ws_->pinned, host_xyz, count * 12);
@@ -216,20 +245,33 @@ int WorkspaceLease::stage(const float* host_xyz, uint64_t count, uint32_t width,
 	int rc = ws_->in.ensure(count * 12);
 	if (!rc) rc = ws_->out.ensure(count * 4 * width);
 	if (rc) return rc;
-	const hipError_t e = hipMemcpy(ws_->in.ptr, host_xyz, count * 12, hipMemcpyHostToDevice);
-	if (e != hipSuccess) return hip_fail(e, "points upload");
 	*xyz = ws_->in.as<const float>();
 	*out = ws_->out.as<float>();
-	return TG_OK;
+	return gathered ? TG_OK : upload(host_xyz, count);
+}
+
+int WorkspaceLease::upload(const float* host_xyz, uint64_t count)
+{
+	hipError_t e;
+	if (copied_)
+	{
+		std::memcpy(ws_->pinned, host_xyz, count * 12);
+		e = copy_words(ws_->pinned, ws_->in.ptr, 3 * count);
+	}
+	else
+		e = hipMemcpy(ws_->in.ptr, host_xyz, count * 12, hipMemcpyHostToDevice);
+	return e == hipSuccess ? TG_OK : hip_fail(e, "points upload");
 }
 
 int WorkspaceLease::collect(float* host_out, uint64_t count, uint32_t width)
 {
 	hipError_t e;
-	if (direct_)
+	if (direct_ || copied_)
 	{
-		e = hipStreamSynchronize(nullptr);
-		if (e == hipSuccess) std::memcpy(host_out, static_cast<const float*>(ws_->pinned) + 3 * count, count * 4 * width);
+		float* results = static_cast<float*>(ws_->pinned) + (copied_ ? (3 * count + 3) / 4 * 4 : 3 * count);
+		e = copied_ ? copy_words(ws_->out.ptr, results, count * width) : hipSuccess;
+		if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+		if (e == hipSuccess) std::memcpy(host_out, results, count * 4 * width);
 	}
 	else
 		e = hipMemcpy(host_out, ws_->out.ptr, count * 4 * width, hipMemcpyDeviceToHost);
@@ -596,24 +638,6 @@ namespace {
 // 39 / 24; 24 primitives 16384 16 / 15, 131072 16 / 18.)
 uint64_t split_evaluations(const tg_program* p) { return p->decoded.entries.size() >= 96 ? 131072 : 32768; }
 
-}  // namespace
-
-int tg::launch_gradients(const tg_program* p, const GradArgs& a, uint32_t flags, hipStream_t stream)
-{
-	const bool fast = (flags & TG_FLAG_FAST) != 0;
-	SplitProgram sp;
-	hipError_t e;
-	// (four taps to a point and k_gradient a lane to a tap: half the evaluations;
-	// 256 primitives 16384 points 210 / 105 us, 65536 276 / 275, 512 primitives 437 / 579)
-	if (a.count <= split_evaluations(p) / 8 && split_program(p, sp))
-		e = fast ? fast::launch_gradient_split(a, sp, stream) : exact::launch_gradient_split(a, sp, stream);
-	else
-		e = fast ? fast::launch_gradient(a, stream) : exact::launch_gradient(a, stream);
-	return e == hipSuccess ? TG_OK : hip_fail(e, "gradient launch");
-}
-
-namespace {
-
 // Whether gathering n points by cell and pruning the program for the cells costs
 // less than the entries they save.  Whole program: 0.15 us an entry and 0.74 an
 // entry and million points; gathered: 100 us and 0.16 an entry for the passes, 60
@@ -626,18 +650,29 @@ bool sort_points(const tg_program* p, uint64_t n)
 	return n > split_evaluations(p) && m * (0.675 * e - 60.0) > 105.0 + 0.01 * e;
 }
 
+// The same for gradients, four evaluations a point (whole call, as k_gradient /
+// gathered, us: 256 primitives 50000 points 223 / 266, 100k 353 / 337, 200k 587 / 472,
+// 1M 2684 / 1743; 64 primitives 200k 325 / 403, 1M 1636 / 1600; 512 primitives 20000
+// 338 / 292, 100k 593 / 412; 2000 primitives 20000 1211 / 904, 100k 1847 / 1077).
+bool sort_gradients(const tg_program* p, uint64_t n)
+{
+	const double m = 1e-6 * double(n), e = double(p->decoded.entries.size());
+	return n > split_evaluations(p) / 8 && m * (2.3 * e - 160.0) > 130.0 - 0.07 * e;
+}
+
 constexpr uint32_t kSortCells = 24, kSortOuterCells = 8;  // per axis (fine cells, 2M points of 256 / 2048 primitives: 16 440 / 2473 us, 20 371 / 1833, 24 335 / 1467)
 constexpr uint64_t kSortPoints = 4u << 20;  // points sorted at a time (their buffers: 144 MiB)
 
 // The launches of sorted_points, with the workspace's buffers.
-int sorted_launches(const tg_program* p, SortedPointsArgs& sa, float edge, float reach, bool fast, hipStream_t s,
-	Workspace& ws, bool* sorted)
+int sorted_launches(const tg_program* p, SortedPointsArgs& sa, const GradArgs* grad, float edge, float reach, bool fast,
+	hipStream_t s, Workspace& ws, const PointsReady& ready, bool* sorted)
 {
 	const DecodedProgram& d = p->decoded;
 	const uint64_t entries = d.entries.size(), count = sa.p.count;
 	const float* xyz = sa.p.xyz;
 	float* out = sa.p.out;
 	sa.bins = sa.groups = 1;
+	sa.chunk_shift = grad ? 4 : 6;
 	CellGrid grids[2];
 	for (int L = 0; L < 2; ++L)
 	{
@@ -665,6 +700,7 @@ int sorted_launches(const tg_program* p, SortedPointsArgs& sa, float edge, float
 		}
 		// (points on a face of the cube's cells, the cells' centres: rounding)
 		g.radius = 0.5f * cell * 1.7320508f * (1.0f + 1.0e-3f) + 1.0e-6f * (reach + 4.0f * edge);
+		if (grad) g.radius += 1.7320508f * (1.0f + 1.0e-3f) * std::fabs(grad->h);
 		g.words = true;
 	}
 	const tg_program* progs[2] = { p, p };
@@ -676,6 +712,8 @@ int sorted_launches(const tg_program* p, SortedPointsArgs& sa, float edge, float
 		sa.words[L] = outs[L]->pool.as<const uint32_t>();
 		sa.desc[L] = outs[L]->desc.as<const BlockDesc>();
 	}
+	if (ready) rc = ready();
+	if (rc) return rc;
 	const uint64_t batch = std::min<uint64_t>(count, kSortPoints);
 	rc = ws.ctl.ensure((3 * size_t(sa.bins + 1) + (kGroupStride + 1) * size_t(sa.groups + 1)) * 4);
 	if (!rc) rc = ws.out.ensure(batch * 4);
@@ -692,25 +730,42 @@ int sorted_launches(const tg_program* p, SortedPointsArgs& sa, float edge, float
 	for (uint64_t at = 0; at < count; at += batch)
 	{
 		sa.p.xyz = xyz + 3 * at;
-		sa.p.out = out + at;
+		sa.p.out = grad ? nullptr : out + at;
 		sa.p.count = std::min<uint64_t>(batch, count - at);
-		TG_CHECK_HIP(hipMemsetAsync(sa.counts[0], 0, (kGroupStride * size_t(sa.groups) + sa.bins) * 4, s), "bin reset");
-		const hipError_t e = fast ? fast::launch_points_sorted(sa, s) : exact::launch_points_sorted(sa, s);
-		if (e != hipSuccess) return hip_fail(e, "eval points launch");
+		// (a kernel of our own: hipMemsetAsync launches two for this size, 8 us against 4)
+		const uint32_t words = kGroupStride * sa.groups + sa.bins;
+		hipLaunchKernelGGL(k_zero_words, dim3((words + 255) / 256), dim3(256), 0, s, sa.counts[0], words);
+		TG_CHECK_HIP(hipGetLastError(), "bin reset");
+		GradArgs ga{};
+		if (grad)
+		{
+			ga = *grad;
+			ga.out = grad->out + 3 * at;
+		}
+		const GradArgs* g = grad ? &ga : nullptr;
+		const hipError_t e = fast ? fast::launch_points_sorted(sa, g, s) : exact::launch_points_sorted(sa, g, s);
+		if (e != hipSuccess) return hip_fail(e, "sorted points launch");
 	}
 	*sorted = true;
 	return TG_OK;
 }
 
-// Evaluates `a` through cell programs where that pays, asynchronously on `s`.
-// Not while `s` is captured: the call allocates.
-int sorted_points(const tg_program* p, const PointArgs& a, bool fast, hipStream_t s, bool* sorted)
+// Whether `count` points (with `gradients`, the gradients there) go through cell programs.
+bool gathers(const tg_program* p, uint64_t count, bool gradients)
+{
+	const uint64_t ncells = uint64_t(kSortCells) * kSortCells * kSortCells;
+	return (gradients ? sort_gradients(p, count) : sort_points(p, count)) && p->decoded.scene_finite &&
+	       ncells * p->decoded.entries.size() <= (150ull << 20) && treelet_prunable(p, ncells);
+}
+
+// Evaluates `a` (with `grad`, the gradients there) through cell programs where
+// that pays, asynchronously on `s`.  Not while `s` is captured: the call allocates.
+// `ready` (if any) is called when the points are wanted, behind the pruning.
+int sorted_points(const tg_program* p, const PointArgs& a, const GradArgs* grad, bool fast, hipStream_t s,
+	const PointsReady& ready, bool* sorted)
 {
 	const DecodedProgram& d = p->decoded;
-	const uint64_t entries = d.entries.size();
-	if (!sort_points(p, a.count) || !d.scene_finite) return TG_OK;
-	const uint64_t ncells = uint64_t(kSortCells) * kSortCells * kSortCells;
-	if (ncells * entries > (150ull << 20) || !treelet_prunable(p, ncells)) return TG_OK;
+	if (!gathers(p, a.count, grad != nullptr)) return TG_OK;
 	if (s)
 	{
 		hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -732,6 +787,8 @@ int sorted_points(const tg_program* p, const PointArgs& a, bool fast, hipStream_
 	}
 	edge = edge * 1.01f + 1e-3f;
 	if (!(edge < 1e6f) || !(reach < 1e6f)) return TG_OK;
+	// taps that reach beyond a cell of half the size prune little
+	if (grad && !(std::fabs(grad->h) < 0.25f * edge / float(kSortCells))) return TG_OK;
 	// allocations here are no part of a capture that another thread may have begun
 	hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
 	TG_CHECK_HIP(hipThreadExchangeStreamCaptureMode(&mode), "capture mode");
@@ -739,28 +796,51 @@ int sorted_points(const tg_program* p, const PointArgs& a, bool fast, hipStream_
 	WorkspaceLease ws;
 	int rc = ws.take(s);
 	if (rc) return rc;
-	rc = sorted_launches(p, sa, edge, reach, fast, s, *ws.operator->(), sorted);
+	rc = sorted_launches(p, sa, grad, edge, reach, fast, s, *ws.operator->(), ready, sorted);
 	const int left = ws.leave_to(s);
 	return rc ? rc : left;
 }
 
 }  // namespace
 
-extern "C" int tg_eval_points_device(const tg_program* p, const float* xyz, uint64_t n, float* out, uint32_t flags,
-	void* stream)
+bool tg::gathers_gradients(const tg_program* p, uint64_t count) { return gathers(p, count, true); }
+
+int tg::launch_gradients(const tg_program* p, const GradArgs& a, uint32_t flags, hipStream_t stream, const PointsReady& ready)
 {
-	if (!p || (n && (!xyz || !out))) return fail(TG_ERR_INVALID, "tg_eval_points_device: null argument");
-	if (n == 0) return TG_OK;
+	const bool fast = (flags & TG_FLAG_FAST) != 0;
+	PointArgs pa{};
+	pa.prog = a.prog;
+	pa.xyz = a.xyz;
+	pa.count = a.count;
+	pa.slots = a.slots;
+	bool sorted = false;
+	int rc = sorted_points(p, pa, &a, fast, stream, ready, &sorted);
+	if (!rc && !sorted && ready) rc = ready();
+	if (rc || sorted) return rc;
+	SplitProgram sp;
+	hipError_t e;
+	// (four taps to a point and k_gradient a lane to a tap: half the evaluations;
+	// 256 primitives 16384 points 210 / 105 us, 65536 276 / 275, 512 primitives 437 / 579)
+	if (a.count <= split_evaluations(p) / 8 && split_program(p, sp))
+		e = fast ? fast::launch_gradient_split(a, sp, stream) : exact::launch_gradient_split(a, sp, stream);
+	else
+		e = fast ? fast::launch_gradient(a, stream) : exact::launch_gradient(a, stream);
+	return e == hipSuccess ? TG_OK : hip_fail(e, "gradient launch");
+}
+
+static int launch_eval_points(const tg_program* p, const float* xyz, uint64_t n, float* out, uint32_t flags, hipStream_t s,
+	const PointsReady& ready)
+{
 	PointArgs a{};
 	a.prog = static_cast<const Instr*>(p->device.ptr);
 	a.xyz = xyz;
 	a.out = out;
 	a.count = n;
 	a.slots = std::max<uint32_t>(1, p->decoded.max_stack - 1);
-	hipStream_t s = static_cast<hipStream_t>(stream);
 	const bool fast = (flags & TG_FLAG_FAST) != 0;
 	bool sorted = false;
-	const int rc = sorted_points(p, a, fast, s, &sorted);
+	int rc = sorted_points(p, a, nullptr, fast, s, ready, &sorted);
+	if (!rc && !sorted && ready) rc = ready();
 	if (rc || sorted) return rc;
 	SplitProgram sp;
 	hipError_t e;
@@ -770,6 +850,14 @@ extern "C" int tg_eval_points_device(const tg_program* p, const float* xyz, uint
 		e = fast ? fast::launch_points(a, s) : exact::launch_points(a, s);
 	if (e != hipSuccess) return hip_fail(e, "eval points launch");
 	return TG_OK;
+}
+
+extern "C" int tg_eval_points_device(const tg_program* p, const float* xyz, uint64_t n, float* out, uint32_t flags,
+	void* stream)
+{
+	if (!p || (n && (!xyz || !out))) return fail(TG_ERR_INVALID, "tg_eval_points_device: null argument");
+	if (n == 0) return TG_OK;
+	return launch_eval_points(p, xyz, n, out, flags, static_cast<hipStream_t>(stream), {});
 }
 
 extern "C" int tg_check_sqrt(uint32_t scramble, uint64_t* mismatches)
@@ -812,8 +900,12 @@ extern "C" int tg_eval_points(const tg_program* p, const float* xyz, uint64_t n,
 	const float* in = nullptr;
 	float* res = nullptr;
 	int rc = ws.take();
-	if (!rc) rc = ws.stage(xyz, n, 1, &in, &res);
-	if (!rc) rc = tg_eval_points_device(p, in, n, res, flags, nullptr);
+	const bool gathered = gathers(p, n, false);
+	if (!rc) rc = ws.stage(xyz, n, 1, gathered, &in, &res);
+	if (!rc)
+		rc = launch_eval_points(p, in, n, res, flags, nullptr,
+			gathered ? PointsReady([&] { return ws.upload(xyz, n); }) : PointsReady());
+	if (rc && gathered) (void)hipStreamSynchronize(nullptr);  // the upload may be under way
 	if (!rc) rc = ws.collect(out, n, 1);
 	return rc;
 }

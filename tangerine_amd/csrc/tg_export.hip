@@ -1321,7 +1321,7 @@ int gradients_at(tg_mesher* m, const tg_program* p, const float* dev_xyz, uint64
 	ga.h = 1.0e-4f;
 	ga.tetra = 1;
 	ga.slots = std::max<uint32_t>(1, p->decoded.max_stack - 1);
-	rc = launch_gradients(p, ga, flags, m->stream);
+	rc = launch_gradients(p, ga, flags, m->stream, {});
 	if (rc) return rc;
 	TG_CHECK_HIP(hipMemcpyAsync(out.data(), dout.ptr, n * 12, hipMemcpyDeviceToHost, m->stream), "normal download");
 	TG_CHECK_HIP(hipStreamSynchronize(m->stream), "normals");

@@ -42,8 +42,8 @@ struct PointArgs
 struct BlockDesc;
 
 // Many points: counted into the cells of two cubes (a fine one around the
-// scene, a coarse one of four times its size), gathered by cell and evaluated 64 of
-// a cell to a wave with the cell's program.  Bin 0: points in neither cube.
+// scene, a coarse one of four times its size), gathered by cell and evaluated a
+// chunk of a cell to a wave with the cell's program.  Bin 0: points in neither cube.
 struct SortedPointsArgs
 {
 	PointArgs p;               // at most 2^31 points
@@ -53,7 +53,8 @@ struct SortedPointsArgs
 	uint32_t groups;           // 1 + those of 4^3 cells (point_groups)
 	uint32_t* counts[2];       // per group (kGroupStride words apart) / per bin (zeroed): points
 	uint32_t* first[2];        // per group / per bin, and one more: points in those before it
-	uint32_t* chunk;           // per bin and one more: 64-point chunks in the bins before it
+	uint32_t* chunk;           // per bin and one more: chunks in the bins before it
+	uint32_t chunk_shift;      // points per chunk, a wave's: 2^6, for gradients 2^4
 	uint32_t* rank;            // per point: its place among its group's / its bin's
 	float4* sorted[2];         // per point, by group / by bin: x, y, z, the point's index as bits
 	const uint32_t* words[2];  // the cells' programs (PruneArgs::words)
@@ -466,7 +467,7 @@ hipError_t launch_trace_resume(const TraceArgs& a, hipStream_t s);
 hipError_t launch_march(const TraceArgs& a, hipStream_t s);
 hipError_t launch_march_far(const FarArgs& a, uint32_t max_rays, hipStream_t s);
 hipError_t launch_points_split(const PointArgs& a, const SplitProgram& p, hipStream_t s);
-hipError_t launch_points_sorted(const SortedPointsArgs& a, hipStream_t s);
+hipError_t launch_points_sorted(const SortedPointsArgs& a, const GradArgs* grad, hipStream_t s);
 hipError_t launch_gradient_split(const GradArgs& a, const SplitProgram& p, hipStream_t s);
 hipError_t launch_gradient(const GradArgs& a, hipStream_t s);
 // all 2^32 float inputs of the exact build's square root against sqrtf
@@ -506,7 +507,7 @@ hipError_t launch_trace_resume(const TraceArgs& a, hipStream_t s);
 hipError_t launch_march(const TraceArgs& a, hipStream_t s);
 hipError_t launch_march_far(const FarArgs& a, uint32_t max_rays, hipStream_t s);
 hipError_t launch_points_split(const PointArgs& a, const SplitProgram& p, hipStream_t s);
-hipError_t launch_points_sorted(const SortedPointsArgs& a, hipStream_t s);
+hipError_t launch_points_sorted(const SortedPointsArgs& a, const GradArgs* grad, hipStream_t s);
 hipError_t launch_gradient_split(const GradArgs& a, const SplitProgram& p, hipStream_t s);
 hipError_t launch_gradient(const GradArgs& a, hipStream_t s);
 }

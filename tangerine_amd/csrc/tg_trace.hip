@@ -650,14 +650,16 @@ extern "C" int tg_gradient_points(const tg_program* p, const float* xyz, uint64_
 	GradArgs ga{};
 	WorkspaceLease ws;
 	rc = ws.take();
-	if (!rc) rc = ws.stage(xyz, count, 3, &ga.xyz, &ga.out);
+	const bool gathered = gathers_gradients(p, count);
+	if (!rc) rc = ws.stage(xyz, count, 3, gathered, &ga.xyz, &ga.out);
 	if (rc) return rc;
 	ga.prog = static_cast<const Instr*>(p->device.ptr);
 	ga.count = count;
 	ga.h = h;
 	ga.tetra = mode == 0 ? 1 : 0;
 	ga.slots = std::max<uint32_t>(1, p->decoded.max_stack - 1);
-	rc = launch_gradients(p, ga, flags, nullptr);
+	rc = launch_gradients(p, ga, flags, nullptr, gathered ? PointsReady([&] { return ws.upload(xyz, count); }) : PointsReady());
+	if (rc && gathered) (void)hipStreamSynchronize(nullptr);  // the upload may be under way
 	if (!rc) rc = ws.collect(out, count, 3);
 	return rc;
 }
