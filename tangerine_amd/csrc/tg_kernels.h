@@ -291,6 +291,9 @@ struct TraceLevel
 	float inv;               // RN(1 / cell)
 };
 
+// Entries whose values a group of lanes keeps in LDS: of 16 lanes; of a wave.
+constexpr uint32_t kGroupEntries = 256, kMaxGroupEntries = 8000;
+
 struct TraceArgs
 {
 	const Instr* prog;
@@ -332,6 +335,9 @@ struct TraceArgs
 	TraceRay* q_out;
 	uint32_t* q_keys;
 	uint32_t* q_out_count;
+	const uint32_t* q_in_count;       // k_trace_groups: rays in q_in
+	uint32_t group_entries;           // ... longest program a group of lanes runs
+	uint32_t entry_budget;            // a wave queues its rays too once it has interpreted more entries
 };
 
 // A whole program split over a workgroup: the waves run its treelets, stage by
@@ -464,6 +470,7 @@ hipError_t launch_eval_blocks(const BlockEvalArgs& a, int p, hipStream_t s);
 hipError_t launch_trace(const TraceArgs& a, hipStream_t s);
 // resumed pass (a.q_in set): a wave per a.q_per_wave of the a.q_count rays
 hipError_t launch_trace_resume(const TraceArgs& a, hipStream_t s);
+hipError_t launch_trace_groups(const TraceArgs& a, hipStream_t s);
 hipError_t launch_march(const TraceArgs& a, hipStream_t s);
 hipError_t launch_march_far(const FarArgs& a, uint32_t max_rays, hipStream_t s);
 hipError_t launch_points_split(const PointArgs& a, const SplitProgram& p, hipStream_t s);
@@ -504,6 +511,7 @@ hipError_t launch_eval_blocks(const BlockEvalArgs& a, int p, hipStream_t s);
 hipError_t launch_trace(const TraceArgs& a, hipStream_t s);
 // resumed pass (a.q_in set): a wave per a.q_per_wave of the a.q_count rays
 hipError_t launch_trace_resume(const TraceArgs& a, hipStream_t s);
+hipError_t launch_trace_groups(const TraceArgs& a, hipStream_t s);
 hipError_t launch_march(const TraceArgs& a, hipStream_t s);
 hipError_t launch_march_far(const FarArgs& a, uint32_t max_rays, hipStream_t s);
 hipError_t launch_points_split(const PointArgs& a, const SplitProgram& p, hipStream_t s);

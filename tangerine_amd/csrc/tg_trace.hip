@@ -35,16 +35,25 @@ struct Transform8
 	float x, y, z, w, tx, ty, tz, s;
 };
 
-// Marching passes of a camera render.  The first pass marches every pixel's
-// ray at most kFirstBudget steps, 64 rays (an 8x8 tile) to a wave; nearly all
-// rays end there.  Each later pass takes the rays still marching, sorted by
-// the cell they are in, at most kPassBudget steps, packed so that about
-// kResumeWaves waves run them (at most 64 rays, at least one to a wave): the
-// long marches of a frame no longer share a wave, where each waited on the
-// others' cell programs.  (1920x1080, 256 primitives: 10.6 ms in one pass;
-// two passes, the rays left one to a wave, two cameras: 64 + 192 steps 9.0 /
-// 10.2 ms, 48 + 208 8.0 / 9.4, 40 7.6 / 8.6, 32 7.1 / 7.8, 24 7.2 / 8.7, 16 7.2 /
-// 8.2.  Earlier than 32 the waves of single rays are more than run at once.)
+// Marching passes of a camera render.  The first marches every pixel's ray, 64
+// rays (an 8x8 tile) to a wave, which is what most rays cost least in; but a wave
+// whose rays part pays for each one's cell program in turn, and the few waves that
+// do so longest would end the frame alone (1920x1080, 256 primitives: 2.3 waves a
+// SIMD on average over 5.7 ms).  So a wave stops at kFirstSteps steps or once it has
+// interpreted first_entries() entries, and its rays go on in k_trace_groups: 16
+// lanes to a ray, then a wave to each ray that meets a longer program than those
+// hold, then (k_trace_resume, from kMaxGroupEntries entries on) the rest.
+// Whole call, passes of 32 + 224 steps with a wave to each ray left / this, ms:
+// 1920x1080 of 256 primitives 7.28 / 4.75 and (another scene) 8.57 / 6.26, of 512
+// 16.2 / 10.5, of 16 1.38 / 1.31; 640x360 of 64 1.91 / 1.23, of 2048 40.2 / 20;
+// 320x180 of 256 5.16 / 2.25.
+//
+// A tracer whose passes were set keeps to those: the first of kFirstBudget steps,
+// each later one of kPassBudget takes the rays still marching, sorted by the cell
+// they are in, packed so that about kResumeWaves waves run them (at most 64 rays, at
+// least one to a wave).
+constexpr int kFirstSteps = 48;        // 1920x1080, 256 primitives: 20 5.4 ms, 32 5.0, 48 4.8, 64 4.75; 16 primitives 1.29, 1.32, 1.32, 1.31
+constexpr int kGroupsMinSteps = 17;    // frames of fewer steps have no long marches
 constexpr int kFirstBudget = 32;
 constexpr int kPassBudget = 224;
 constexpr uint32_t kResumeWaves = 65536;
@@ -59,6 +68,7 @@ struct tg_tracer
 	uint32_t* host_count = nullptr;                  // pinned
 	int first_budget = kFirstBudget, budget = kPassBudget;
 	uint32_t resume_waves = kResumeWaves;
+	bool tuned = false;           // set_passes was called
 	CellPrograms levels[kTraceLevels];
 	PruneLaunches launches;
 	float dom_lo[3] = { 0, 0, 0 };
@@ -161,6 +171,17 @@ int ensure_pass_buffers(tg_tracer* tr, uint64_t n)
 	return TG_OK;
 }
 
+// Entries a wave of the first pass interprets at most: a few steps of the whole
+// program's length, more where other waves keep the GPU busy meanwhile (1920x1080, 256
+// primitives: 1500 entries 5.0 ms, 3000 4.8, 4500 5.1, 12000 7.5; 320x180: 600
+// 2.2, 1500 2.7, 3000 3.0; 2048 primitives, 640x360: 4500 33, 8200 23, 12000 20;
+// 16 primitives, 1920x1080: 190 1.31, 3000 1.69).
+uint32_t first_entries(uint64_t rays, size_t entries)
+{
+	const double waves = double(rays) / 64.0;
+	return uint32_t(double(entries) * std::min(6.0, std::max(1.0, std::sqrt(waves) / 24.0)));
+}
+
 void base_args(TraceArgs& ta, const tg_program* p)
 {
 	ta = TraceArgs{};
@@ -261,6 +282,7 @@ extern "C" int tg_tracer_set_passes(tg_tracer* tr, int first_budget, int budget,
 	tr->first_budget = first_budget;
 	tr->budget = budget;
 	tr->resume_waves = resume_waves;
+	tr->tuned = true;
 	return TG_OK;
 }
 
@@ -281,8 +303,14 @@ extern "C" int tg_tracer_render(tg_tracer* tr, const tg_program* p, const tg_cam
 	const bool fast = (flags & TG_FLAG_FAST) != 0;
 	const uint64_t n = uint64_t(cam->width) * cam->height;
 	// passes: the first, then enough resumed ones to reach max_steps
-	const bool passes = tr->first_budget > 0 && tr->first_budget < max_steps;
-	const int npass = passes ? 1 + (max_steps - tr->first_budget + tr->budget - 1) / tr->budget : 1;
+	// untuned: the rays left go on in groups of lanes, in as many passes as the
+	// program's entries can need
+	const size_t entries = p->decoded.entries.size();
+	const bool groups = !tr->tuned && !(flags & TG_FLAG_NO_PRUNE) && max_steps >= kGroupsMinSteps;
+	const bool passes = groups || (tr->first_budget > 0 && tr->first_budget < max_steps);
+	const int npass = groups  ? (entries <= kGroupEntries ? 2 : entries <= kMaxGroupEntries ? 3 : 4)
+	                  : passes ? 1 + (max_steps - tr->first_budget + tr->budget - 1) / tr->budget
+	                           : 1;
 	int rc = tr->t.ensure(n * 4);
 	if (!rc) rc = tr->normals.ensure(n * 12);
 	if (!rc) rc = tr->steps.ensure(n * 4);
@@ -382,14 +410,25 @@ extern "C" int tg_tracer_render(tg_tracer* tr, const tg_program* p, const tg_cam
 	for (int k = 0; k < npass; ++k)
 	{
 		const int left = max_steps - taken;
-		ta.budget = passes ? std::min(left, k == 0 ? tr->first_budget : tr->budget) : max_steps;
-		const bool last = k + 1 == npass;
+		ta.budget = groups  ? (k == 0 ? std::min(max_steps, kFirstSteps) : max_steps)
+		            : passes ? std::min(left, k == 0 ? tr->first_budget : tr->budget)
+		                     : max_steps;
+		ta.entry_budget = groups && k == 0 ? first_entries(n, entries) : ~0u;
+		// (a group pass has a queue even where no program is too long for it)
+		const bool last = k + 1 == npass && !(groups && (k == 1 || k == 2));
 		ta.q_out = last ? nullptr : tr->queue[k & 1].as<TraceRay>();
 		ta.q_keys = last ? nullptr : tr->keys.as<uint32_t>();
 		ta.q_out_count = last ? nullptr : ctl + k;
 		hipError_t e;
 		if (k == 0)
 			e = fast ? fast::launch_trace(ta, tr->stream) : exact::launch_trace(ta, tr->stream);
+		else if (groups && k <= 2)
+		{
+			ta.q_in = tr->queue[(k - 1) & 1].as<const TraceRay>();
+			ta.q_in_count = ctl + k - 1;
+			ta.group_entries = k == 1 ? kGroupEntries : std::min(ta.n_whole, kMaxGroupEntries);
+			e = fast ? fast::launch_trace_groups(ta, tr->stream) : exact::launch_trace_groups(ta, tr->stream);
+		}
 		else
 		{
 			// the rays the previous pass left, in key order (one cell's rays together)
