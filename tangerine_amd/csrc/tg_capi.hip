@@ -526,13 +526,16 @@ int tg::upload_program(const DecodedProgram& d, tg_program** out)
 	p->uid = next_uid++;
 	p->decoded = d;
 	p->plan = prune_plan(d);
+	p->split_plan = prune_plan(d, kSplitUpperItems);
 	static_assert(sizeof(HostEntry) == 16 && sizeof(TreeletItem) == 16 && sizeof(Treelet) == 16, "one array of 16-byte words");
 	std::vector<HostEntry> blob(d.entries);
-	const size_t items = blob.size(), treelets = items + p->plan.items.size();
-	blob.resize(std::max<size_t>(treelets + p->plan.treelets.size(), 1));
-	if (!p->plan.items.empty()) std::memcpy(&blob[items], p->plan.items.data(), p->plan.items.size() * sizeof(TreeletItem));
-	if (!p->plan.treelets.empty())
-		std::memcpy(&blob[treelets], p->plan.treelets.data(), p->plan.treelets.size() * sizeof(Treelet));
+	for (const PrunePlan* plan : { &p->plan, &p->split_plan })
+	{
+		const size_t items = blob.size(), treelets = items + plan->items.size();
+		blob.resize(std::max<size_t>(treelets + plan->treelets.size(), 1));
+		if (!plan->items.empty()) std::memcpy(&blob[items], plan->items.data(), plan->items.size() * sizeof(TreeletItem));
+		if (!plan->treelets.empty()) std::memcpy(&blob[treelets], plan->treelets.data(), plan->treelets.size() * sizeof(Treelet));
+	}
 	rc = p->device.ensure(d.instrs.size() * sizeof(Instr));
 	if (!rc) rc = p->entries.ensure(blob.size() * sizeof(HostEntry));
 	if (rc)
@@ -613,15 +616,18 @@ extern "C" void tg_program_destroy(tg_program* p)
 bool tg::split_program(const tg_program* p, SplitProgram& out)
 {
 	const DecodedProgram& d = p->decoded;
-	const PrunePlan& plan = p->plan;
 	out = SplitProgram{};
 	out.slots = std::max<uint32_t>(1, d.max_stack - 1);
-	if (plan.stages() < 2 || plan.stages() > kSplitStages ||
-		split_lds_bytes(plan.slots, out.slots, kSplitWaves) > kSplitMaxLds)
-		return false;
+	auto fits = [&](const PrunePlan& plan) {
+		return plan.stages() >= 2 && plan.stages() <= kSplitStages &&
+		       split_lds_bytes(plan.slots, out.slots, kSplitWaves) <= kSplitMaxLds;
+	};
+	const bool narrow = fits(p->split_plan);
+	const PrunePlan& plan = narrow ? p->split_plan : p->plan;
+	if (!narrow && !fits(plan)) return false;
 	out.prog = static_cast<const Instr*>(p->device.ptr);
-	out.items = p->items();
-	out.treelets = p->treelets();
+	out.items = narrow ? p->split_items() : p->items();
+	out.treelets = narrow ? p->split_treelets() : p->treelets();
 	out.records = uint32_t(d.entries.size());
 	out.stages = plan.stages();
 	for (uint32_t s = 0; s <= out.stages; ++s) out.stage_first[s] = plan.stage_first[s];

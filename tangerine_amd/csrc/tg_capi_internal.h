@@ -35,13 +35,16 @@ struct tg_program
 	uint64_t uid = 0;    // unique per uploaded program (caches of derived device data key on it)
 	tg::DecodedProgram decoded;
 	tg::PrunePlan plan;  // its treelets
+	tg::PrunePlan split_plan;  // those of a program split over a workgroup
 	tg::DevBuf device;   // Instr records
-	tg::DevBuf entries;  // whole program as pruning entries, then the plan's items and treelets
+	tg::DevBuf entries;  // whole program as pruning entries, then each plan's items and treelets
 	const tg::TreeletItem* items() const
 	{
 		return reinterpret_cast<const tg::TreeletItem*>(entries.as<const tg::HostEntry>() + decoded.entries.size());
 	}
 	const tg::Treelet* treelets() const { return reinterpret_cast<const tg::Treelet*>(items() + plan.items.size()); }
+	const tg::TreeletItem* split_items() const { return reinterpret_cast<const tg::TreeletItem*>(treelets() + plan.treelets.size()); }
+	const tg::Treelet* split_treelets() const { return reinterpret_cast<const tg::Treelet*>(split_items() + split_plan.items.size()); }
 };
 
 namespace tg {

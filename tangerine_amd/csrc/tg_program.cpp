@@ -188,7 +188,7 @@ float rounding_slack(const DecodedProgram& d, float pmax)
 	return float(std::max(s, 2.0e-4));
 }
 
-PrunePlan prune_plan(const DecodedProgram& d)
+PrunePlan prune_plan(const DecodedProgram& d, uint32_t upper_items)
 {
 	PrunePlan plan;
 	const uint32_t n = uint32_t(d.entries.size());
@@ -206,14 +206,15 @@ PrunePlan prune_plan(const DecodedProgram& d)
 	// for each cut operand) would exceed a treelet cuts the larger operand, then
 	// the other.
 	std::vector<uint32_t> size(n, 1), stage(n, 0);
-	std::vector<uint8_t> cut(n, 0);
+	std::vector<uint8_t> cut(n, 0), upper(n, 0);  // upper: its treelet so far has a cut operand
 	for (uint32_t e = 0; e < n; ++e)
 	{
 		uint32_t c[2] = { 0, 0 };
 		const uint32_t k = operands(e, c);
 		uint32_t total = 1;
 		for (uint32_t i = 0; i < k; ++i) total += size[c[i]];
-		for (uint32_t i = 0; i < k && total > kTreeletItems; ++i)
+		for (uint32_t i = 0; i < k; ++i) upper[e] |= upper[c[i]] | cut[c[i]];
+		for (uint32_t i = 0; i < k && total > (upper[e] ? upper_items : kTreeletItems); ++i)
 		{
 			uint32_t which = 0;
 			if (k == 2 && (cut[c[0]] || (!cut[c[1]] && size[c[1]] > size[c[0]]))) which = 1;
@@ -221,6 +222,7 @@ PrunePlan prune_plan(const DecodedProgram& d)
 			total -= size[x] - 1;
 			cut[x] = 1;
 			size[x] = 1;
+			upper[e] = 1;
 		}
 		size[e] = total;
 		for (uint32_t i = 0; i < k; ++i) stage[e] = std::max(stage[e], stage[c[i]] + (cut[c[i]] ? 1u : 0u));

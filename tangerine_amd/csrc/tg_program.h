@@ -49,6 +49,13 @@ struct DecodedProgram
 // is an entry of the treelet, or stands for a smaller treelet's root (a cut).
 // Treelets are ordered by stage; a treelet's cuts belong to earlier stages.
 constexpr uint32_t kTreeletItems = 32;
+// Of a program split over a workgroup, treelets above others: where a cut subtree
+// occurs only this many.  The widest stage is the first; those above it leave waves
+// idle, so they are cut finer: a stage of 7 items costs less than one wave running
+// 31.  (One point / 50k rays, us, 32 items everywhere / 8 above: 256 primitives 32 /
+// 30, 4117 / 3707; 120, 36 / 28, 2859 / 2184; 300, 52 / 33, 5757 / 3777; 2000, 122 /
+// 115, 25460 / 24118; 4 and 16 within 2% of 8.)
+constexpr uint32_t kSplitUpperItems = 8;
 constexpr uint32_t kItemLoad = 33u << 24;  // op of a cut item: the root's value is loaded
 
 struct TreeletItem
@@ -75,7 +82,8 @@ struct PrunePlan
 	uint32_t stages() const { return stage_first.empty() ? 0u : uint32_t(stage_first.size()) - 1; }
 };
 
-PrunePlan prune_plan(const DecodedProgram& d);
+// upper_items: the most in a treelet with a cut.
+PrunePlan prune_plan(const DecodedProgram& d, uint32_t upper_items = kTreeletItems);
 
 // Validates stack discipline and opcodes the way SDFInterpreter::Eval would
 // (tangerine/sdf_evaluator.cpp:1397-1600) and re-encodes the program.
