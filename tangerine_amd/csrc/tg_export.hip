@@ -1303,7 +1303,21 @@ __global__ void __launch_bounds__(256) k_centroids(const float* v, const uint32_
 }
 
 // Normalised tetrahedral gradients (SDFNode::Gradient, h = 1e-4) of the
-// program at `n` device points; result copied to the host.
+// program at `n` device points, on the mesher's stream.
+int launch_normals(tg_mesher* m, const tg_program* p, const float* dev_xyz, uint64_t n, uint32_t flags, float* dev_out)
+{
+	GradArgs ga{};
+	ga.prog = static_cast<const Instr*>(p->device.ptr);
+	ga.xyz = dev_xyz;
+	ga.out = dev_out;
+	ga.count = n;
+	ga.h = 1.0e-4f;
+	ga.tetra = 1;
+	ga.slots = std::max<uint32_t>(1, p->decoded.max_stack - 1);
+	return launch_gradients(p, ga, flags, m->stream, {});
+}
+
+// The same, copied to the host.
 int gradients_at(tg_mesher* m, const tg_program* p, const float* dev_xyz, uint64_t n, uint32_t flags,
 	std::vector<float>& out)
 {
@@ -1312,16 +1326,7 @@ int gradients_at(tg_mesher* m, const tg_program* p, const float* dev_xyz, uint64
 	DevBuf dout;
 	struct Guard { DevBuf* b; ~Guard() { b->release(); } } guard{ &dout };
 	int rc = dout.ensure(n * 12);
-	if (rc) return rc;
-	GradArgs ga{};
-	ga.prog = static_cast<const Instr*>(p->device.ptr);
-	ga.xyz = dev_xyz;
-	ga.out = dout.as<float>();
-	ga.count = n;
-	ga.h = 1.0e-4f;
-	ga.tetra = 1;
-	ga.slots = std::max<uint32_t>(1, p->decoded.max_stack - 1);
-	rc = launch_gradients(p, ga, flags, m->stream, {});
+	if (!rc) rc = launch_normals(m, p, dev_xyz, n, flags, dout.as<float>());
 	if (rc) return rc;
 	TG_CHECK_HIP(hipMemcpyAsync(out.data(), dout.ptr, n * 12, hipMemcpyDeviceToHost, m->stream), "normal download");
 	TG_CHECK_HIP(hipStreamSynchronize(m->stream), "normals");
@@ -1535,13 +1540,15 @@ extern "C" int tg_mesher_export_sodapop(tg_mesher* m, const tg_program* p, const
 	rc = run_export(m, p, &g, flags, false, nullptr);
 	if (rc) return rc;
 	const uint64_t nv = m->nverts, ni = m->ntris * 3;
+	rc = m->normals.ensure(std::max<uint64_t>(nv, 1) * 12);
+	if (rc) return rc;
+	std::vector<uint32_t> ex;  // (read by the copy until the last wait)
 	if (shuffle && nv > 1)
 	{
-		std::vector<uint32_t> ex;
 		vertex_sequence(nv, ex);
 		rc = m->exchange.ensure(nv * 4);
-		if (!rc) rc = m->normals.ensure(nv * 12);  // staging for the permuted positions
 		if (rc) return rc;
+		// m->normals: staging for the permuted positions
 		TG_CHECK_HIP(hipMemcpyAsync(m->exchange.ptr, ex.data(), nv * 4, hipMemcpyHostToDevice, m->stream), "upload");
 		hipLaunchKernelGGL(k_permute_vertices, dim3(grid_for(nv)), dim3(256), 0, m->stream,
 			m->vertices.as<const float>(), m->normals.as<float>(), m->exchange.as<const uint32_t>(), nv);
@@ -1554,15 +1561,15 @@ extern "C" int tg_mesher_export_sodapop(tg_mesher* m, const tg_program* p, const
 				m->exchange.as<const uint32_t>(), ni);
 			TG_CHECK_HIP(hipGetLastError(), "remap launch");
 		}
-		TG_CHECK_HIP(hipStreamSynchronize(m->stream), "vertex sequence");
 	}
 	// normals: SDFOctree::Gradient at every (final) vertex (USE_GRADIENT_NORMALS)
-	std::vector<float> normals;
-	rc = gradients_at(m, p, m->vertices.as<const float>(), nv, flags, normals);
-	if (rc) return rc;
-	rc = m->normals.ensure(std::max<uint64_t>(nv, 1) * 12);
-	if (rc) return rc;
-	if (nv) TG_CHECK_HIP(hipMemcpy(m->normals.ptr, normals.data(), nv * 12, hipMemcpyHostToDevice), "normals");
+	if (nv)
+	{
+		rc = launch_normals(m, p, m->vertices.as<const float>(), nv, flags, m->normals.as<float>());
+		const hipError_t e = hipStreamSynchronize(m->stream);
+		if (rc) return rc;
+		TG_CHECK_HIP(e, "normals");
+	}
 	m->have_normals = true;
 	return TG_OK;
 }
