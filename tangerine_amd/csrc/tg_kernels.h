@@ -451,9 +451,9 @@ hipError_t launch_prune_treelets_multi(const TreeletArgs* jobs, const uint32_t* 
 hipError_t launch_prune_cells_multi(const PruneArgs* jobs, const uint32_t* block_base, uint32_t njobs, uint32_t blocks,
 	uint32_t max_slots, hipStream_t s);
 // the same a wave per cell (PruneArgs::columns): job k owns workgroups [block_base[k], ...) of `blocks`
-// (prune_column_blocks of each); max_entries: over the jobs that emit whole entries
+// (prune_column_blocks of each); max_lds: the largest column_lds_bytes of one
 hipError_t launch_prune_columns_multi(const PruneArgs* jobs, const uint32_t* block_base, uint32_t njobs, uint32_t blocks,
-	uint32_t max_waves, uint32_t max_entries, hipStream_t s);
+	uint32_t max_waves, size_t max_lds, hipStream_t s);
 hipError_t launch_eval_tile_programs(const TileEvalArgs& a, hipStream_t s);
 // many grids in one launch: job k owns workgroups [block_base[k], ...) of `blocks` (tile_eval_blocks of each)
 hipError_t launch_eval_tile_programs_multi(const TileEvalArgs* jobs, const uint32_t* block_base, uint32_t njobs,
@@ -492,9 +492,9 @@ hipError_t launch_prune_treelets_multi(const TreeletArgs* jobs, const uint32_t* 
 hipError_t launch_prune_cells_multi(const PruneArgs* jobs, const uint32_t* block_base, uint32_t njobs, uint32_t blocks,
 	uint32_t max_slots, hipStream_t s);
 // the same a wave per cell (PruneArgs::columns): job k owns workgroups [block_base[k], ...) of `blocks`
-// (prune_column_blocks of each); max_entries: over the jobs that emit whole entries
+// (prune_column_blocks of each); max_lds: the largest column_lds_bytes of one
 hipError_t launch_prune_columns_multi(const PruneArgs* jobs, const uint32_t* block_base, uint32_t njobs, uint32_t blocks,
-	uint32_t max_waves, uint32_t max_entries, hipStream_t s);
+	uint32_t max_waves, size_t max_lds, hipStream_t s);
 hipError_t launch_eval_tile_programs(const TileEvalArgs& a, hipStream_t s);
 // many grids in one launch: job k owns workgroups [block_base[k], ...) of `blocks` (tile_eval_blocks of each)
 hipError_t launch_eval_tile_programs_multi(const TileEvalArgs* jobs, const uint32_t* block_base, uint32_t njobs,
@@ -581,6 +581,14 @@ inline uint32_t prune_column_blocks(const PruneArgs& a)
 {
 	const uint32_t per = a.emit_waves * a.emit_cells;
 	return (a.nx * a.ny * a.nz + per - 1) / per;
+}
+// LDS of one wave of the column emission for a program of n entries (16-byte
+// multiples, so that every wave's 8-byte masks stay aligned), and of a job's
+// workgroup: at most 48 KiB.
+__host__ __device__ inline uint32_t column_lds_stride(uint32_t n) { return ((n + 63) / 64 * 12 + 15) & ~15u; }
+inline size_t column_lds_bytes(const PruneArgs& a)
+{
+	return size_t(column_lds_stride(a.words ? 0u : a.n_entries)) * a.emit_waves;
 }
 inline uint32_t tile_eval_blocks(const TileEvalArgs& a)
 {

@@ -354,7 +354,8 @@ int prune_cells_many(hipStream_t stream, const tg_program* const* progs, const C
 	// latter's workgroups
 	std::vector<PruneArgs> ejobs, cjobs;
 	std::vector<uint32_t> ebase, cbase;
-	uint32_t blocks = 0, max_slots = 1, cells = 0, max_entries = 0, max_waves = 1;
+	uint32_t blocks = 0, max_slots = 1, cells = 0, max_waves = 1;
+	size_t max_lds = 0;
 	for (uint32_t i = 0; i < n; ++i)
 	{
 		if (!ready[i]) continue;
@@ -365,7 +366,8 @@ int prune_cells_many(hipStream_t stream, const tg_program* const* progs, const C
 			cbase.push_back(cells);
 			cells += prune_column_blocks(pa);
 			max_waves = std::max(max_waves, pa.emit_waves);
-			if (!pa.words) max_entries = std::max(max_entries, pa.n_entries);
+			// (of one job: a long program takes few waves, and its table is not every job's)
+			max_lds = std::max(max_lds, column_lds_bytes(pa));
 			cjobs.push_back(pa);
 			continue;
 		}
@@ -423,8 +425,8 @@ int prune_cells_many(hipStream_t stream, const tg_program* const* progs, const C
 		const PruneArgs* jobs = reinterpret_cast<const PruneArgs*>(dev + cj);
 		const uint32_t* base = reinterpret_cast<const uint32_t*>(dev + cb);
 		const hipError_t e =
-			fast ? fast::launch_prune_columns_multi(jobs, base, uint32_t(cjobs.size()), cells, max_waves, max_entries, stream)
-			     : exact::launch_prune_columns_multi(jobs, base, uint32_t(cjobs.size()), cells, max_waves, max_entries, stream);
+			fast ? fast::launch_prune_columns_multi(jobs, base, uint32_t(cjobs.size()), cells, max_waves, max_lds, stream)
+			     : exact::launch_prune_columns_multi(jobs, base, uint32_t(cjobs.size()), cells, max_waves, max_lds, stream);
 		if (e != hipSuccess) return hip_fail(e, "cell pruning launch");
 	}
 	hipLaunchKernelGGL(k_prune_counts, dim3(nbuf), dim3(64), 0, stream, dev_buffers, PruneBuffers{});
