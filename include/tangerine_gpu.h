@@ -283,7 +283,7 @@ int tg_tracer_set_domain(tg_tracer* tracer, const float lo[3], float size);
  * marching (sorted by the cell they are in) at most `budget` more, packed so
  * that about resume_waves waves run them, until max_steps.  first_budget <= 0:
  * one pass.  Results do not depend on these.  Default: passes chosen by the
- * frame and the program (unpruned renders: 32, 224, 65536). */
+ * frame and the program (unpruned renders: 48, 208, 65536). */
 int tg_tracer_set_passes(tg_tracer* tracer, int first_budget, int budget, uint32_t resume_waves);
 /* Renders width*height rays on the device; hit normals by central differences
  * with step normal_h (<= 0: none).  Results stay on the device until copied. */

@@ -525,6 +525,7 @@ int tg::upload_program(const DecodedProgram& d, tg_program** out)
 	auto p = std::make_unique<tg_program>();
 	p->uid = next_uid++;
 	p->decoded = d;
+	p->kept = kept_share(d);
 	p->plan = prune_plan(d);
 	p->split_plan = prune_plan(d, kSplitUpperItems);
 	static_assert(sizeof(HostEntry) == 16 && sizeof(TreeletItem) == 16 && sizeof(Treelet) == 16, "one array of 16-byte words");

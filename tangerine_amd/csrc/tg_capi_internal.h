@@ -34,6 +34,7 @@ struct tg_program
 {
 	uint64_t uid = 0;    // unique per uploaded program (caches of derived device data key on it)
 	tg::DecodedProgram decoded;
+	float kept = 0.0f;   // kept_share
 	tg::PrunePlan plan;  // its treelets
 	tg::PrunePlan split_plan;  // those of a program split over a workgroup
 	tg::DevBuf device;   // Instr records

@@ -48,14 +48,17 @@ struct Transform8
 // 16.2 / 10.5, of 16 1.38 / 1.31; 640x360 of 64 1.91 / 1.23, of 2048 40.2 / 20;
 // 320x180 of 256 5.16 / 2.25.
 //
-// A tracer whose passes were set keeps to those: the first of kFirstBudget steps,
-// each later one of kPassBudget takes the rays still marching, sorted by the cell
-// they are in, packed so that about kResumeWaves waves run them (at most 64 rays, at
-// least one to a wave).
+// Groups of lanes pay about ten times a wave's instructions for a ray's step, so
+// they lose where cells drop little and many rays are left (frame_groups).  Then, on
+// renders without pruning, and on a tracer whose passes were set: the first of
+// kFirstBudget steps, each later one of kPassBudget takes the rays still marching,
+// sorted by the cell they are in, packed so that about kResumeWaves waves run them (at
+// most 64 rays, at least one to a wave).  (1920x1080 without pruning, passes of 48 + 208
+// steps / 32 + 224, ms: 64 primitives 12.4 / 14.4, 256 60.2 / 82.6.)
 constexpr int kFirstSteps = 48;        // 1920x1080, 256 primitives: 20 5.4 ms, 32 5.0, 48 4.8, 64 4.75; 16 primitives 1.29, 1.32, 1.32, 1.31
 constexpr int kGroupsMinSteps = 17;    // frames of fewer steps have no long marches
-constexpr int kFirstBudget = 32;
-constexpr int kPassBudget = 224;
+constexpr int kFirstBudget = 48;
+constexpr int kPassBudget = 208;
 constexpr uint32_t kResumeWaves = 65536;
 constexpr int kKeyBits = 27;  // trace_key: level above an 18-bit Morton code
 
@@ -182,6 +185,17 @@ uint32_t first_entries(uint64_t rays, size_t entries)
 	return uint32_t(double(entries) * std::min(6.0, std::max(1.0, std::sqrt(waves) / 24.0)));
 }
 
+// Whether the long marches of a frame go on in groups of lanes.  (Passes / groups, ms,
+// by the share of the entries that cells keep.  1 (an ellipsoid): 64 primitives 640x360
+// 8.7 / 7.9, 960x540 9.3 / 11.1, 1920x1080 12.8 / 21.3, 256 primitives 38.7 / 26.3, 41.3 / 48.3,
+// 60.1 / 125.  0.66 to 0.8 (blends of 2 units): 256 primitives 42.9 / 31.4, 47.3 / 56.8, 76.4 /
+// 141.  0.44 (1 unit): 1280x720 28.4 / 25.1, 1920x1080 33.4 / 39.2.  0.32 (0.5): 1920x1080 22.5 /
+// 18.9.  0.05: 9.2 / 6.5.)
+bool frame_groups(uint64_t rays, float kept)
+{
+	return double(rays) * std::pow(double(kept), 1.75) <= 240.0e3;
+}
+
 void base_args(TraceArgs& ta, const tg_program* p)
 {
 	ta = TraceArgs{};
@@ -306,7 +320,8 @@ extern "C" int tg_tracer_render(tg_tracer* tr, const tg_program* p, const tg_cam
 	// untuned: the rays left go on in groups of lanes, in as many passes as the
 	// program's entries can need
 	const size_t entries = p->decoded.entries.size();
-	const bool groups = !tr->tuned && !(flags & TG_FLAG_NO_PRUNE) && max_steps >= kGroupsMinSteps;
+	const bool groups = !tr->tuned && !(flags & TG_FLAG_NO_PRUNE) && max_steps >= kGroupsMinSteps &&
+	                    frame_groups(n, p->kept);
 	const bool passes = groups || (tr->first_budget > 0 && tr->first_budget < max_steps);
 	const int npass = groups  ? (entries <= kGroupEntries ? 2 : entries <= kMaxGroupEntries ? 3 : 4)
 	                  : passes ? 1 + (max_steps - tr->first_budget + tr->budget - 1) / tr->budget

@@ -1,0 +1,38 @@
+"""Routes of calls whose program no cell prunes, or hardly any: they go as they would
+without cells where cells only cost.  Without a device: what is launched tells."""
+
+import pytest
+
+from tests.fake_device import run
+
+TREES = """
+from tangerine_amd import trace
+def tree(kind, n):
+    "random tree; with an ellipsoid (never pruned); every operator a blend of `kind` units"
+    spec = scenes.random_csg_spec(1, n)
+    if kind == "ellipsoid":
+        spec[next(i for i, t in enumerate(spec) if t[0] in scenes.PRIMITIVES)] = ("ellipsoid", 0.5, 0.7, 0.9)
+    elif kind != "random":
+        spec = [("blend_union", float(kind)) if t[0] in scenes.SET_OPS else t for t in spec]
+    return scenes.build_sdf(spec).program()
+"""
+
+
+@pytest.mark.parametrize("kind,prims,groups", [
+    ("ellipsoid", 64, (True, False)), ("ellipsoid", 256, (True, False)), ("2", 64, (True, False)), ("2", 256, (True, False)),
+    ("8", 256, (True, False)), ("0.1", 256, (True, True)), ("random", 16, (True, True)), ("random", 64, (True, True)),
+    ("random", 256, (True, True)), ("random", 2048, (True, True))])
+def test_frames(kind, prims, groups):
+    """Small frames go on in groups of lanes whatever the program (their waves do not
+    fill the GPU), large ones only where cells prune; unpruned renders never."""
+    run(TREES + f"""
+p = tree({kind!r}, {prims})
+tr = trace.Tracer()
+for (w, h), want in zip([(320, 180), (1920, 1080)], {groups!r}):
+    cam = trace.look_at((9, 6, 5), width=w, height=h)
+    launches()
+    tr.render(p, cam)
+    assert ran("k_trace_groups", launches()) == want, (w, h)
+    tr.render(p, cam, prune=False)
+    assert not ran("k_trace_groups", launches())
+""")
