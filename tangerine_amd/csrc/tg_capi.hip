@@ -648,23 +648,31 @@ uint64_t split_evaluations(const tg_program* p) { return p->decoded.entries.size
 // Whether gathering n points by cell and pruning the program for the cells costs
 // less than the entries they save.  Whole program: 0.15 us an entry and 0.74 an
 // entry and million points; gathered: 100 us and 0.16 an entry for the passes, 60
-// us and 0.065 an entry a million points.  (Whole / gathered, us: 256 primitives
-// 262144 points 184 / 195, 1M 483 / 241, 2M 802 / 297, 6M 2047 / 599; 2048 primitives
-// 524288 2002 / 862, 2M 5679 / 1373; 64 primitives 2M 222 / 250.)
+// us and 1.3 an entry that the cells keep a million points, 0.65 an entry kept at any
+// count.  (Whole / gathered, us, random trees (0.05 of the entries kept): 256
+// primitives 262144 points 184 / 195, 1M 483 / 241, 2M 802 / 297, 6M 2047 / 599; 2048
+// primitives 524288 2002 / 862, 2M 5679 / 1373; 64 primitives 2M 222 / 250.  256
+// primitives, 0.32 kept: 600k 362 / 412, 2M 835 / 719; 0.44: 2M 845 / 945; 1: 600k 363 /
+// 617, 2M 816 / 1267.  1024 primitives, 0.22 kept: 300k 784 / 999, 600k 1382 / 1222, 2M
+// 3147 / 2368; 0.38: 2M 3128 / 3273.)
 bool sort_points(const tg_program* p, uint64_t n)
 {
-	const double m = 1e-6 * double(n), e = double(p->decoded.entries.size());
-	return n > split_evaluations(p) && m * (0.675 * e - 60.0) > 105.0 + 0.01 * e;
+	const double m = 1e-6 * double(n), e = double(p->decoded.entries.size()), kept = p->kept;
+	return n > split_evaluations(p) && m * ((0.74 - 1.3 * kept) * e - 60.0) > 100.0 + (0.01 + 0.65 * kept) * e;
 }
 
 // The same for gradients, four evaluations a point (whole call, as k_gradient /
 // gathered, us: 256 primitives 50000 points 223 / 266, 100k 353 / 337, 200k 587 / 472,
 // 1M 2684 / 1743; 64 primitives 200k 325 / 403, 1M 1636 / 1600; 512 primitives 20000
-// 338 / 292, 100k 593 / 412; 2000 primitives 20000 1211 / 904, 100k 1847 / 1077).
+// 338 / 292, 100k 593 / 412; 2000 primitives 20000 1211 / 904, 100k 1847 / 1077.  256
+// primitives, 0.32 of the entries kept: 200k 604 / 696, 400k 1057 / 1078, 1M 2792 / 2461;
+// 0.44: 1M 2823 / 2938; 1: 100k 359 / 576, 1M 2849 / 3584.  1024 primitives, 0.22 kept:
+// 100k 1057 / 1179, 200k 1747 / 1599; 0.38: 400k 3001 / 3250, 1M 7047 / 6773).
 bool sort_gradients(const tg_program* p, uint64_t n)
 {
-	const double m = 1e-6 * double(n), e = double(p->decoded.entries.size());
-	return n > split_evaluations(p) / 8 && m * (2.3 * e - 160.0) > 130.0 - 0.07 * e;
+	const double m = 1e-6 * double(n), e = double(p->decoded.entries.size()), kept = p->kept;
+	return n > split_evaluations(p) / 8 &&
+	       m * ((2.5 - 4.7 * kept) * e - 160.0) > 130.0 + (0.9 * kept - 0.11) * e;
 }
 
 constexpr uint32_t kSortCells = 24, kSortOuterCells = 8;  // per axis (fine cells, 2M points of 256 / 2048 primitives: 16 440 / 2473 us, 20 371 / 1833, 24 335 / 1467)

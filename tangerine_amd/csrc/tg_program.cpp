@@ -280,27 +280,34 @@ PrunePlan prune_plan(const DecodedProgram& d, uint32_t upper_items)
 
 namespace {
 
-// Distance of p from a brush, roughly: as a ball of its mean size (a torus: as a
-// shell) in its own frame.
-float rough_distance(const Instr& in, const float (&p)[3])
+constexpr int kSharePoints = 8;
+
+// Distances of points from a brush, roughly: as a ball of its mean size (a torus: as
+// a shell) in its own frame.
+void rough_distances(const Instr& in, const float (&p)[3][kSharePoints], float (&d)[kSharePoints])
 {
 	const float* m = reinterpret_cast<const float*>(in.w) + 1;
-	float q[3] = { p[0], p[1], p[2] };
 	const uint32_t kind = instr_kind(in), op = instr_op(in);
-	for (int r = 0; r < 3; ++r)
-		if (kind == XF_OFFSET)
-			q[r] += m[4 * r + 3];
-		else if (kind == XF_MATRIX)
-			q[r] = m[4 * r] * p[0] + m[4 * r + 1] * p[1] + m[4 * r + 2] * p[2] + m[4 * r + 3];
 	const float a = m[12], b = m[13], c = m[14];
-	if (op == OP_PLANE) return a * q[0] + b * q[1] + c * q[2];
-	const float l = std::sqrt(q[0] * q[0] + q[1] * q[1] + q[2] * q[2]);
+	float q[3][kSharePoints];
+	for (int r = 0; r < 3; ++r)
+		for (int s = 0; s < kSharePoints; ++s)
+			q[r][s] = kind == XF_MATRIX ? m[4 * r] * p[0][s] + m[4 * r + 1] * p[1][s] + m[4 * r + 2] * p[2][s] + m[4 * r + 3]
+			                            : p[r][s] + (kind == XF_OFFSET ? m[4 * r + 3] : 0.0f);
+	float shell = 0.0f, radius;
 	switch (op)
 	{
-	case OP_SPHERE: return l - a;
-	case OP_TORUS: return std::fabs(l - a) - b;
-	case OP_CYLINDER: case OP_CONE: return l - 0.5f * (a + b);
-	default: return l - (a + b + c) * (1.0f / 3.0f);
+	case OP_SPHERE: radius = a; break;
+	case OP_TORUS: shell = a; radius = b; break;
+	case OP_CYLINDER: case OP_CONE: radius = 0.5f * (a + b); break;
+	default: radius = (a + b + c) * (1.0f / 3.0f); break;
+	}
+	for (int s = 0; s < kSharePoints; ++s)
+	{
+		const float l = std::sqrt(q[0][s] * q[0][s] + q[1][s] * q[1][s] + q[2][s] * q[2][s]);
+		d[s] = op == OP_PLANE ? a * q[0][s] + b * q[1][s] + c * q[2][s]
+		       : op == OP_TORUS ? std::fabs(l - shell) - radius
+		                        : l - radius;
 	}
 }
 
@@ -311,60 +318,73 @@ float kept_share(const DecodedProgram& d)
 	const uint32_t n = uint32_t(d.entries.size());
 	if (!d.prunable() || n == 0 || n >= 65535) return 1.0f;
 	if (!d.scene_finite) return 0.0f;
-	const uint32_t points = std::min<uint32_t>(8, std::max<uint32_t>(2, 4096 / n));
 	float edge = 0.0f;
 	for (int i = 0; i < 3; ++i) edge = std::max(edge, d.scene_hi[i] - d.scene_lo[i]);
 	const float two = edge / 24.0f * 1.7320508f;  // twice a cell's radius
-	std::vector<float> value(n);
-	std::vector<uint8_t> drop(n), live(n);  // drop: 1 the left operand, 2 the right one
-	uint64_t kept = 0;
-	for (uint32_t s = 0; s < points; ++s)
-	{
-		// (an additive sequence of the plastic number's powers: evenly spread)
-		const double step[3] = { 0.8191725134, 0.6710436067, 0.5497004779 };
-		float p[3];
-		for (int i = 0; i < 3; ++i)
+	// (an additive sequence of the plastic number's powers: evenly spread)
+	const double step[3] = { 0.8191725134, 0.6710436067, 0.5497004779 };
+	float p[3][kSharePoints];
+	for (int i = 0; i < 3; ++i)
+		for (int s = 0; s < kSharePoints; ++s)
 		{
 			const double t = 0.5 + double(s + 1) * step[i];
-			p[i] = d.scene_lo[i] + float(t - std::floor(t)) * (d.scene_hi[i] - d.scene_lo[i]);
+			p[i][s] = d.scene_lo[i] + float(t - std::floor(t)) * (d.scene_hi[i] - d.scene_lo[i]);
 		}
-		for (uint32_t e = 0; e < n; ++e)
+	// bottom up the values and each operator's points that keep the left and the
+	// right operand, then top down the points where an entry is left
+	struct Value
+	{
+		float v[kSharePoints];
+	};
+	std::vector<Value> value(n);
+	std::vector<uint8_t> left(n, 0xff), right(n, 0xff), live(n);
+	const uint32_t mask = 0x3fffffu;  // an entry's record
+	for (uint32_t e = 0; e < n; ++e)
+	{
+		const HostEntry& x = d.entries[e];
+		const Instr& in = d.instrs[x.rec & mask];
+		const uint32_t op = instr_op(in);
+		float(&v)[kSharePoints] = value[e].v;
+		if (is_brush(op))
 		{
-			const HostEntry& x = d.entries[e];
-			const Instr& in = d.instrs[x.rec & 0x3fffffu];
-			const uint32_t op = instr_op(in);
-			if (is_brush(op))
-				value[e] = rough_distance(in, p);
-			else if (!is_binary(op))
-				value[e] = op == OP_FLATE ? value[x.l] - as_float(in.w[1]) : value[x.l] * as_float(in.w[1]);
-			else
-			{
-				const uint32_t base = is_blend(op) ? op - (OP_BLEND_UNION - OP_UNION) : op;
-				// union: the nearer operand; intersection, difference: the farther
-				const float l = base == OP_UNION ? -value[x.l] : value[x.l];
-				const float r = base == OP_INTER ? value[x.r] : -value[x.r];
-				const float t = two + (is_blend(op) ? std::max(as_float(in.w[3]), 0.0f) : 0.0f);
-				drop[e] = l - r >= t ? 2 : r - l >= t ? 1 : 0;
-				value[e] = base == OP_UNION ? -std::max(l, r) : std::max(l, r);
-			}
+			rough_distances(in, p, v);
+			continue;
 		}
-		live[n - 1] = 1;
-		for (uint32_t e = n; e-- > 0;)
+		const float(&vl)[kSharePoints] = value[x.l].v;
+		if (!is_binary(op))
 		{
-			const HostEntry& x = d.entries[e];
-			const uint32_t op = instr_op(d.instrs[x.rec & 0x3fffffu]);
-			if (is_binary(op))
-			{
-				live[x.l] = live[e] && drop[e] != 1;
-				live[x.r] = live[e] && drop[e] != 2;
-				kept += live[e] && drop[e] == 0;
-				continue;
-			}
-			if (!is_brush(op)) live[x.l] = live[e];
-			kept += live[e];
+			const float by = as_float(in.w[1]);
+			for (int s = 0; s < kSharePoints; ++s) v[s] = op == OP_FLATE ? vl[s] - by : vl[s] * by;
+			continue;
 		}
+		// every operator as a maximum: union -max(-l, -r), intersection max(l, r),
+		// difference max(l, -r)
+		const uint32_t base = is_blend(op) ? op - (OP_BLEND_UNION - OP_UNION) : op;
+		const float sl = base == OP_UNION ? -1.0f : 1.0f, sr = base == OP_INTER ? 1.0f : -1.0f;
+		const float t = two + (is_blend(op) ? std::max(as_float(in.w[3]), 0.0f) : 0.0f);
+		const float(&vr)[kSharePoints] = value[x.r].v;
+		uint32_t kl = 0, kr = 0;
+		for (int s = 0; s < kSharePoints; ++s)
+		{
+			const float l = sl * vl[s], r = sr * vr[s];
+			kl |= uint32_t(!(r - l >= t)) << s;
+			kr |= uint32_t(!(l - r >= t)) << s;
+			v[s] = sl * std::max(l, r);
+		}
+		left[e] = uint8_t(kl);
+		right[e] = uint8_t(kr);
 	}
-	return float(double(kept) / (double(points) * double(n)));
+	live[n - 1] = 0xff;
+	uint64_t kept = 0;
+	for (uint32_t e = n; e-- > 0;)
+	{
+		const HostEntry& x = d.entries[e];
+		const uint32_t op = instr_op(d.instrs[x.rec & mask]);
+		if (!is_brush(op)) live[x.l] = live[e] & left[e];
+		if (is_binary(op)) live[x.r] = live[e] & right[e];
+		kept += uint32_t(__builtin_popcount(live[e] & left[e] & right[e]));
+	}
+	return float(double(kept) / (double(kSharePoints) * double(n)));
 }
 
 bool decode_words(const uint32_t* w, size_t n, DecodedProgram& out, std::string& err)

@@ -36,3 +36,27 @@ for (w, h), want in zip([(320, 180), (1920, 1080)], {groups!r}):
     tr.render(p, cam, prune=False)
     assert not ran("k_trace_groups", launches())
 """)
+
+
+@pytest.mark.parametrize("kind,prims,points,gradients", [
+    ("random", 256, {300_000: False, 600_000: True, 2_000_000: True}, {50_000: False, 200_000: True}),
+    ("random", 64, {2_000_000: False}, {100_000: False, 1_000_000: True}),
+    ("2", 256, {600_000: False, 2_000_000: False}, {100_000: False, 1_000_000: False}),
+    ("8", 256, {600_000: False, 2_000_000: False}, {100_000: False, 1_000_000: False}),
+    ("8", 1024, {150_000: False, 2_000_000: False}, {50_000: False, 1_000_000: False}),
+    ("0.5", 256, {600_000: False, 2_000_000: True}, {100_000: False, 1_000_000: True})])
+def test_points_and_gradients(kind, prims, points, gradients):
+    run(TREES + f"""
+p = tree({kind!r}, {prims})
+for n, want in {points!r}.items():
+    x = np.zeros((n, 3), np.float32)
+    launches()
+    p.eval_points(x)
+    assert ran("k_eval_points_sorted", launches()) == want, n
+for n, want in {gradients!r}.items():
+    x = np.zeros((n, 3), np.float32)
+    for central in (False, True):
+        launches()
+        trace.gradient(p, x, central=central)
+        assert ran("k_gradient_sorted", launches()) == want, (n, central)
+""")
