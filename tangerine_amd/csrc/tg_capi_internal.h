@@ -117,6 +117,7 @@ struct CellGrid
 	float origin[3], cell[3], radius;
 	uint32_t counts[3];
 	bool words = false;
+	uint32_t room = 0;  // entries a cell in the pool's first guess (0: a quarter of the program, for words at most 64)
 };
 
 // Job tables of prune_cells_many (kept between calls: the upload reads `host`).

@@ -199,7 +199,7 @@ namespace {
 // upload of the entries by height.  *ready is false when the program is not
 // pruned here.
 int prune_prepare(hipStream_t stream, const tg_program* p, const float origin[3], const float cell[3],
-	float radius, const uint32_t counts[3], CellPrograms& out, bool words, bool* ready)
+	float radius, const uint32_t counts[3], CellPrograms& out, bool words, uint32_t room, bool* ready)
 {
 	const DecodedProgram& d = p->decoded;
 	*ready = false;
@@ -255,6 +255,7 @@ int prune_prepare(hipStream_t stream, const tg_program* p, const float origin[3]
 	// (tile programs are short: at most 64 entries each at first)
 	size_t per_cell = std::max<size_t>(d.entries.size() / 4, 16);
 	if (words) per_cell = std::min<size_t>(per_cell, 64);
+	if (room) per_cell = room;
 	ps.capacity = std::max<uint64_t>(out.pool.bytes / entry_bytes(ps),
 		std::min<uint64_t>(ncells * per_cell, (1ull << 30) / entry_bytes(ps)));
 	*ready = true;
@@ -275,7 +276,7 @@ int prune_cells_start(hipStream_t stream, const tg_program* p, const float origi
 	float radius, const uint32_t counts[3], bool fast, CellPrograms& out, bool words)
 {
 	bool ready = false;
-	int rc = prune_prepare(stream, p, origin, cell, radius, counts, out, words, &ready);
+	int rc = prune_prepare(stream, p, origin, cell, radius, counts, out, words, 0, &ready);
 	if (rc || !ready) return rc;
 	rc = prune_pass(stream, p, origin, cell, counts, fast, out, true);
 	if (rc) return rc;
@@ -294,7 +295,7 @@ int prune_cells_many(hipStream_t stream, const tg_program* const* progs, const C
 	{
 		bool r = false;
 		int rc = prune_prepare(stream, progs[i], grids[i].origin, grids[i].cell, grids[i].radius, grids[i].counts,
-			*outs[i], grids[i].words, &r);
+			*outs[i], grids[i].words, grids[i].room, &r);
 		if (rc) return rc;
 		if (!r && grids[i].words) return fail(TG_ERR_LIMIT, "tile programs need the treelet passes");
 		if (!r) continue;

@@ -94,8 +94,9 @@ struct CubeDomain
 // Levels coarse to fine: doms[L] split into ns[L]^3 cells.  Every level's
 // passes of a stage are one launch: the coarse levels' are shorter than a launch
 // is apart from the next (a frame of 256 primitives, four levels one after another 0.55 ms, so 0.39).
+// rooms (or null): CellGrid::room of each.
 int build_levels(hipStream_t stream, const tg_program* p, const CubeDomain* doms, const uint32_t* ns, int count,
-	bool fast, CellPrograms* levels, PruneLaunches& work, TraceArgs& ta)
+	bool fast, CellPrograms* levels, PruneLaunches& work, TraceArgs& ta, const uint32_t* rooms = nullptr)
 {
 	ta.nlevels = 0;
 	count = std::min(count, kTraceLevels);
@@ -113,6 +114,7 @@ int build_levels(hipStream_t stream, const tg_program* p, const CubeDomain* doms
 			g.counts[i] = ns[L];
 		}
 		g.radius = 0.5f * cell * 1.7320508f;
+		g.room = rooms ? rooms[L] : 0;
 		progs[L] = p;
 		outs[L] = &levels[L];
 	}
@@ -647,7 +649,12 @@ extern "C" int tg_raymarch(const tg_program* p, const float* starts, const float
 	TG_CHECK_HIP(hipMemsetAsync(ws->ctl.ptr, 0, 256, nullptr), "ray queue reset");
 	TraceArgs& ta = fa.t;
 	base_args(ta, p);
-	rc = build_levels(nullptr, p, doms, ns, cubes, fast, ws->levels, ws->launches, ta);
+	// The scene's cells are many and their programs short: a first guess by the share
+	// they keep, so that the workspace stays small enough to be kept between calls
+	// (kPoolBytes; a quarter of the program a cell is beyond it from 270 primitives on,
+	// and each call then allocates and frees some 300 MiB)
+	const uint32_t rooms[2] = { 0, 16 + uint32_t(1.5f * p->kept * float(p->decoded.entries.size())) };
+	rc = build_levels(nullptr, p, doms, ns, cubes, fast, ws->levels, ws->launches, ta, rooms);
 	if (rc) return rc;
 	ta.starts = ds;
 	ta.dirs = dd;
