@@ -529,19 +529,45 @@ int raymarch_staged(const tg_program* p, const float* starts, const float* dirs,
 	return TG_OK;
 }
 
-// Cubes whose cells get programs for a batch of array rays, and their cells per
-// axis: the cube holding the starts and, inside it, the scene's.  None (0)
-// where the whole program is run instead: programs of few entries, programs
-// that cannot be pruned, or whose treelets do not fit a workgroup.
+constexpr uint64_t kManyRays = 4096;  // casts of fewer do not pay for many cells
 // (below kRayEntries the whole program a wave is as fast: 49 primitives, 100k
 // rays 3.1 ms against 3.7 here; 64 primitives 3.9 against 3.0, and 3.2 against
 // 1.3 at 64 rays)
 constexpr size_t kRayEntries = 112;
 
-int ray_cubes(const tg_program* p, const float* starts, uint64_t count, CubeDomain* doms, uint32_t* ns)
+// Whether cells pay for a cast: ms that the whole program takes a wave (a chain of
+// entries and steps, or the GPU's throughput, rays by the million) against the
+// pruning and the marching in groups of lanes, which costs the more the more cells
+// keep and does not grow in step with the steps, as rays end on the way.
+// (Whole / cells, ms, 256 primitives, 0.05 kept: 50k rays 16.1 / 3.0, of at most 12 steps
+// 1.94 / 0.96, of 3 0.61 / 0.64, of 1 0.31 / 0.56; 1M rays 55.5 / 30.1; 64 rays 14.2 / 2.4, of 1
+// step 0.21 / 0.34.  64 primitives: 50k rays 3.5 / 1.95, 200k 4.9 / 4.6, 400k 7.2 / 8.0, 1M 15.3 /
+// 19.1; 50k rays of 12 steps 0.55 / 0.68.  96 primitives: 1M 22.3 / 19.6.  0.44 kept: 64
+// primitives 50k rays 4.2 / 3.6, 100k 4.1 / 4.7; 256 primitives 100k 21.2 / 9.8, 1M 47.5 / 48.5.
+// 0.92 kept, rays that end early: 256 primitives 4096 rays 2.6 / 2.5, 100k 2.9 / 4.4.  1 kept,
+// rays of one step: 64 rays 0.23 / 0.39, 50k 0.32 / 2.2.)
+bool ray_cells(const tg_program* p, uint64_t count, int max_steps)
+{
+	const bool many = count >= kManyRays;
+	const double n = 1e-6 * double(count), e = double(p->decoded.entries.size()), kept = p->kept;
+	if (kept >= 0.97 || (many && kept >= 0.9)) return false;
+	const double s = std::min(max_steps, 100), root = std::sqrt(e);
+	const double whole = std::hypot(0.00027 * e * s, 0.0011 * e * s * n);
+	const double cells = 0.15 + (many ? 0.0001 + 0.004 * kept : 0.0002) * e +
+	                     std::hypot(0.00095 * root * s * std::min(1.0 + 3.0 * kept, 2.4),
+	                         0.11 * root * std::pow(s, 0.55) * (1.0 + 2.5 * kept) * n);
+	return cells < whole;
+}
+
+// Cubes whose cells get programs for a batch of array rays, and their cells per
+// axis: the cube holding the starts and, inside it, the scene's.  None (0)
+// where the whole program is run instead: programs of few entries, programs
+// that cannot be pruned, or whose treelets do not fit a workgroup, and casts that
+// cells cost more than they save (ray_cells).
+int ray_cubes(const tg_program* p, const float* starts, uint64_t count, int max_steps, CubeDomain* doms, uint32_t* ns)
 {
 	const DecodedProgram& d = p->decoded;
-	if (d.entries.size() < kRayEntries || !treelet_prunable(p, 64 * 64 * 64)) return 0;
+	if (d.entries.size() < kRayEntries || !ray_cells(p, count, max_steps) || !treelet_prunable(p, 64 * 64 * 64)) return 0;
 	float reach = 1.0f, scene = 0.0f;
 	for (uint64_t i = 0; i < 3 * count; ++i)
 	{
@@ -568,13 +594,13 @@ int ray_cubes(const tg_program* p, const float* starts, uint64_t count, CubeDoma
 	int n = 0;
 	doms[n].size = 2.0f * reach;
 	for (int i = 0; i < 3; ++i) doms[n].lo[i] = -reach;
-	ns[n++] = count >= 4096 ? 16u : 8u;
+	ns[n++] = count >= kManyRays ? 16u : 8u;
 	if (d.scene_finite && inner.size < 1e6f)
 	{
 		doms[n] = inner;
 		// (50k rays, 256 primitives, pruning and marching: 32 cells 1.42 ms, 48
-		// 1.15, 64 1.25; a few rays do not pay for many cells)
-		ns[n++] = count >= 4096 ? 48u : 24u;
+		// 1.15, 64 1.25)
+		ns[n++] = count >= kManyRays ? 48u : 24u;
 	}
 	return n;
 }
@@ -636,7 +662,7 @@ extern "C" int tg_raymarch(const tg_program* p, const float* starts, const float
 	CubeDomain doms[2];
 	uint32_t ns[2];
 	FarArgs fa{};
-	const int cubes = max_steps > 0 && split_program(p, fa.split) ? ray_cubes(p, starts, count, doms, ns) : 0;
+	const int cubes = max_steps > 0 && split_program(p, fa.split) ? ray_cubes(p, starts, count, max_steps, doms, ns) : 0;
 	if (cubes == 0)
 		return raymarch_staged(p, starts, dirs, count, max_steps, eps, far_distance, flags, hit, travel, position, ds, dd,
 			dt, dp, dh);

@@ -60,3 +60,22 @@ for n, want in {gradients!r}.items():
         trace.gradient(p, x, central=central)
         assert ran("k_gradient_sorted", launches()) == want, (n, central)
 """)
+
+
+@pytest.mark.parametrize("kind,prims,casts", [
+    ("random", 256, {(64, 100): True, (50_000, 100): True, (1_000_000, 100): True, (50_000, 12): True, (50_000, 1): False,
+                     (64, 1): False, (400_000, 6): False}),
+    ("random", 64, {(64, 100): True, (100_000, 100): True, (50_000, 12): False, (1_000_000, 100): False}),
+    ("1", 64, {(4096, 100): True, (200_000, 100): False}),
+    ("8", 256, {(64, 100): False, (4096, 100): False, (50_000, 100): False}),
+    ("ellipsoid", 256, {(4096, 100): False})])
+def test_ray_casts(kind, prims, casts):
+    run(TREES + f"""
+p = tree({kind!r}, {prims})
+for (n, steps), want in {casts!r}.items():
+    s = np.full((n, 3), 9.0, np.float32)
+    launches()
+    trace.raymarch(p, s, -s, max_steps=steps)
+    calls = launches()
+    assert ran("k_march", calls) == want and ran("k_trace", calls) != want, (n, steps)
+""")
