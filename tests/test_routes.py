@@ -79,3 +79,20 @@ for (n, steps), want in {casts!r}.items():
     calls = launches()
     assert ran("k_march", calls) == want and ran("k_trace", calls) != want, (n, steps)
 """)
+
+
+@pytest.mark.parametrize("kind,prims,clouds", [
+    ("random", 256, {(32, 0): False, (120, 0): True, (120, 2): True}), ("random", 16, {(200, 0): True, (120, 2): True}),
+    ("0.5", 256, {(120, 0): True, (120, 2): False, (200, 2): True}), ("8", 64, {(120, 0): False, (120, 2): False}),
+    ("8", 256, {(120, 0): False, (200, 2): False}), ("ellipsoid", 256, {(120, 0): False})])
+def test_point_clouds(kind, prims, clouds):
+    run(TREES + f"""
+from tangerine_amd.export import Mesher
+p = tree({kind!r}, {prims})
+m = Mesher()
+for (n, steps), want in {clouds!r}.items():
+    launches()
+    m.export_points(p, (-6.0,) * 3, (6.0,) * 3, (float(np.float32(12.0 / n)),) * 3, refine_iterations=steps)
+    calls = launches()
+    assert ran("k_cloud_select_tiles", calls) == want and ran("k_prune", calls) == want, (n, steps)
+""")
