@@ -413,13 +413,18 @@ int prune_blocks(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t f
 // 1.16 / 0.95, 700^3 of 100 1.85 / 1.33, 1024^3 of 32 3.6 / 2.6.)
 // Culled exports prune the tiles that they then skip too: 128^3 of 2048 primitives
 // 1.4 / 20, 320^3 of 16 0.33 / 0.42, of 2048 1.6 / 3.7, 400^3 of 16 0.47 / 0.42, 450^3 of 256
-// 0.96 / 0.84.
+// 0.96 / 0.84.  Where the tiles keep nearly all of a program, blocks are skipped unpruned
+// (256 primitives, 300^3, blends of 8 units and no surface in the grid 2.06 / 0.46; of 2
+// units 3.6 / 18.4).
+constexpr float kCulledKept = 0.9f;
+constexpr size_t kCulledEntries = 16;  // (the shortest programs keep all of themselves)
 constexpr uint64_t kTileWork = 1310ull << 20, kCulledTileWork = 700ull << 20, kTileEntries = 6144;
 
 bool tile_programs(const tg_program* p, const MeshArgs& ma, bool culled = false)
 {
 	const uint64_t tiles = uint64_t(ma.tx) * ma.ty * ma.tz, limit = culled ? kCulledTileWork : kTileWork;
-	return tiles * (p->decoded.entries.size() + kTileEntries) <= limit && treelet_prunable(p, tiles);
+	return tiles * (p->decoded.entries.size() + kTileEntries) <= limit && !(culled && p->kept > kCulledKept && p->decoded.entries.size() >= kCulledEntries) &&
+	       treelet_prunable(p, tiles);
 }
 
 // The 8^3-sample tiles as cells (samples lie within 3.5 |d| of a tile's centre).

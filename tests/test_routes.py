@@ -96,3 +96,13 @@ for (n, steps), want in {clouds!r}.items():
     calls = launches()
     assert ran("k_cloud_select_tiles", calls) == want and ran("k_prune", calls) == want, (n, steps)
 """)
+
+
+@pytest.mark.parametrize("kind,tiles", [("random", True), ("2", True), ("8", False)])
+def test_culled_exports(kind, tiles):
+    run(TREES + f"""
+from tangerine_amd.export import Mesher
+m = Mesher()
+m.export_culled(tree({kind!r}, 256), None, *scenes.grid_for(-6.0, 6.0, 128))
+assert ran("k_certify_tiles", launches()) == {tiles}
+""")
