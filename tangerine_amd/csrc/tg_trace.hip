@@ -192,10 +192,13 @@ uint32_t first_entries(uint64_t rays, size_t entries)
 // 8.7 / 7.9, 960x540 9.3 / 11.1, 1920x1080 12.8 / 21.3, 256 primitives 38.7 / 26.3, 41.3 / 48.3,
 // 60.1 / 125.  0.66 to 0.8 (blends of 2 units): 256 primitives 42.9 / 31.4, 47.3 / 56.8, 76.4 /
 // 141.  0.44 (1 unit): 1280x720 28.4 / 25.1, 1920x1080 33.4 / 39.2.  0.32 (0.5): 1920x1080 22.5 /
-// 18.9.  0.05: 9.2 / 6.5.)
-bool frame_groups(uint64_t rays, float kept)
+// 18.9.  0.05: 9.2 / 6.5.  Short programs: 8 primitives 320x180 1.14 / 0.79, 1920x1080 1.20 /
+// 1.07, 4 primitives 0.82 / 0.66, 0.98 / 1.05, 3840x2160 1.40 / 1.78, 2 primitives 0.73 / 0.79,
+// 0.84 / 0.88, 1.01 / 1.29.)
+bool frame_groups(uint64_t rays, size_t entries, float kept)
 {
-	return double(rays) * std::pow(double(kept), 1.75) <= 240.0e3;
+	const double share = entries < 12 ? 1.0 : double(kept);
+	return entries >= 7 && double(rays) * std::pow(share, 1.75) <= 240.0e3;
 }
 
 void base_args(TraceArgs& ta, const tg_program* p)
@@ -323,7 +326,7 @@ extern "C" int tg_tracer_render(tg_tracer* tr, const tg_program* p, const tg_cam
 	// program's entries can need
 	const size_t entries = p->decoded.entries.size();
 	const bool groups = !tr->tuned && !(flags & TG_FLAG_NO_PRUNE) && max_steps >= kGroupsMinSteps &&
-	                    frame_groups(n, p->kept);
+	                    frame_groups(n, entries, p->kept);
 	const bool passes = groups || (tr->first_budget > 0 && tr->first_budget < max_steps);
 	const int npass = groups  ? (entries <= kGroupEntries ? 2 : entries <= kMaxGroupEntries ? 3 : 4)
 	                  : passes ? 1 + (max_steps - tr->first_budget + tr->budget - 1) / tr->budget
