@@ -229,6 +229,7 @@ hipError_t copy_words(const void* src, void* dst, uint64_t n)
 
 int WorkspaceLease::stage(const float* host_xyz, uint64_t count, uint32_t width, bool gathered, const float** xyz, float** out)
 {
+	queued();
 	const uint64_t bytes = count * (12 + 4 * width) + 16;
 	size_t room = 65536;
 	while (room < bytes && room < kDirectBytes) room *= 2;
@@ -275,13 +276,14 @@ int WorkspaceLease::collect(float* host_out, uint64_t count, uint32_t width)
 	}
 	else
 		e = hipMemcpy(host_out, ws_->out.ptr, count * 4 * width, hipMemcpyDeviceToHost);
+	if (e == hipSuccess) waited();
 	return e == hipSuccess ? TG_OK : hip_fail(e, "results download");
 }
 
 WorkspaceLease::~WorkspaceLease()
 {
 	if (!ws_) return;
-	// (a call that ends here has waited for its own work, or left an event)
+	if (queued_) (void)hipStreamSynchronize(nullptr);
 	if (ws_->bytes() <= kPoolBytes)
 	{
 		std::lock_guard<std::mutex> lock(g_pool_mutex);
@@ -920,7 +922,6 @@ extern "C" int tg_eval_points(const tg_program* p, const float* xyz, uint64_t n,
 	if (!rc)
 		rc = launch_eval_points(p, in, n, res, flags, nullptr,
 			gathered ? PointsReady([&] { return ws.upload(xyz, n); }) : PointsReady());
-	if (rc && gathered) (void)hipStreamSynchronize(nullptr);  // the upload may be under way
 	if (!rc) rc = ws.collect(out, n, 1);
 	return rc;
 }

@@ -175,6 +175,10 @@ public:
 	int take(hipStream_t stream = nullptr);
 	// The work on `stream` so far goes on reading the workspace after the lease.
 	int leave_to(hipStream_t stream);
+	// Work on the default stream uses the workspace: unless waited() says that it is
+	// over, the end of the lease waits for it (a call that fails half way).
+	void queued() { queued_ = true; }
+	void waited() { queued_ = false; }
 	int pinned(size_t bytes);         // its staging, at least this large
 	// `count` points for a kernel to read at `xyz` and `width` floats each for it
 	// to write at `out`: the pinned staging itself for few points, else device
@@ -189,6 +193,7 @@ public:
 
 private:
 	Workspace* ws_ = nullptr;
+	bool queued_ = false;
 	bool direct_ = false;             // staged in pinned memory
 	bool copied_ = false;             // through it, to device buffers and back
 };

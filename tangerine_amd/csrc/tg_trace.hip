@@ -673,6 +673,7 @@ extern "C" int tg_raymarch(const tg_program* p, const float* starts, const float
 	rc = ws->queue.ensure(count * sizeof(TraceRay));
 	if (!rc) rc = ws->ctl.ensure(256);
 	if (rc) return rc;
+	ws.queued();
 	TG_CHECK_HIP(hipMemcpyAsync(ds, starts, count * 12, hipMemcpyHostToDevice, nullptr), "ray upload");
 	TG_CHECK_HIP(hipMemcpyAsync(dd, dirs, count * 12, hipMemcpyHostToDevice, nullptr), "ray upload");
 	TG_CHECK_HIP(hipMemsetAsync(ws->ctl.ptr, 0, 256, nullptr), "ray queue reset");
@@ -703,6 +704,7 @@ extern "C" int tg_raymarch(const tg_program* p, const float* starts, const float
 	e = fast ? fast::launch_march_far(fa, uint32_t(count), nullptr) : exact::launch_march_far(fa, uint32_t(count), nullptr);
 	if (e != hipSuccess) return hip_fail(e, "raymarch launch");
 	TG_CHECK_HIP(hipMemcpy(travel, dt, count * 4, hipMemcpyDeviceToHost), "travel download");
+	ws.waited();
 	if (position) TG_CHECK_HIP(hipMemcpy(position, dp, count * 12, hipMemcpyDeviceToHost), "position download");
 	if (hit) TG_CHECK_HIP(hipMemcpy(hit, dh, count, hipMemcpyDeviceToHost), "hit download");
 	return TG_OK;
@@ -749,7 +751,6 @@ extern "C" int tg_gradient_points(const tg_program* p, const float* xyz, uint64_
 	ga.tetra = mode == 0 ? 1 : 0;
 	ga.slots = std::max<uint32_t>(1, p->decoded.max_stack - 1);
 	rc = launch_gradients(p, ga, flags, nullptr, gathered ? PointsReady([&] { return ws.upload(xyz, count); }) : PointsReady());
-	if (rc && gathered) (void)hipStreamSynchronize(nullptr);  // the upload may be under way
 	if (!rc) rc = ws.collect(out, count, 3);
 	return rc;
 }
