@@ -46,6 +46,11 @@ int DevBuf::ensure(size_t need)
 	bytes = 0;
 	size_t grow = std::max(need, size_t(256));
 	hipError_t e = hipMalloc(&ptr, grow);
+	if (e != hipSuccess && free_idle_workspaces())
+	{
+		hipGetLastError();
+		e = hipMalloc(&ptr, grow);
+	}
 	if (e != hipSuccess)
 	{
 		ptr = nullptr;
@@ -103,6 +108,7 @@ size_t Workspace::bytes() const
 
 void Workspace::release()
 {
+	if (in_flight) (void)hipEventSynchronize(busy);
 	for (DevBuf* b : { &in, &out, &queue, &ctl }) b->release();
 	for (CellPrograms& l : levels) l.release();
 	launches.dev.release();
@@ -112,6 +118,26 @@ void Workspace::release()
 	if (busy) (void)hipEventDestroy(busy);
 	busy = nullptr;
 	in_flight = false;
+}
+
+bool free_idle_workspaces()
+{
+	int dev = 0;
+	if (hipGetDevice(&dev) != hipSuccess) return false;
+	std::vector<Workspace*> out;
+	{
+		std::lock_guard<std::mutex> lock(g_pool_mutex);
+		std::vector<Workspace*>& idle = pool();
+		const auto mine = std::stable_partition(idle.begin(), idle.end(), [dev](const Workspace* w) { return w->device != dev; });
+		out.assign(mine, idle.end());
+		idle.erase(mine, idle.end());
+	}
+	for (Workspace* w : out)
+	{
+		w->release();
+		delete w;
+	}
+	return !out.empty();
 }
 
 int WorkspaceLease::take(hipStream_t stream)
@@ -720,9 +746,14 @@ int sorted_launches(const tg_program* p, SortedPointsArgs& sa, const GradArgs* g
 		if (grad) g.radius += 1.7320508f * (1.0f + 1.0e-3f) * std::fabs(grad->h);
 		g.words = true;
 	}
+	const uint64_t batch = std::min<uint64_t>(count, kSortPoints);
+	int rc = ws.ctl.ensure((3 * size_t(sa.bins + 1) + (kGroupStride + 1) * size_t(sa.groups + 1)) * 4);
+	if (!rc) rc = ws.out.ensure(batch * 4);
+	if (!rc) rc = ws.queue.ensure(batch * 32);
+	if (rc) return rc;
 	const tg_program* progs[2] = { p, p };
 	CellPrograms* outs[2] = { &ws.levels[0], &ws.levels[1] };
-	int rc = prune_cells_many(s, progs, grids, 2, fast, outs, ws.launches);
+	rc = prune_cells_many(s, progs, grids, 2, fast, outs, ws.launches);
 	if (rc) return rc;
 	for (int L = 0; L < 2; ++L)
 	{
@@ -730,11 +761,6 @@ int sorted_launches(const tg_program* p, SortedPointsArgs& sa, const GradArgs* g
 		sa.desc[L] = outs[L]->desc.as<const BlockDesc>();
 	}
 	if (ready) rc = ready();
-	if (rc) return rc;
-	const uint64_t batch = std::min<uint64_t>(count, kSortPoints);
-	rc = ws.ctl.ensure((3 * size_t(sa.bins + 1) + (kGroupStride + 1) * size_t(sa.groups + 1)) * 4);
-	if (!rc) rc = ws.out.ensure(batch * 4);
-	if (!rc) rc = ws.queue.ensure(batch * 32);
 	if (rc) return rc;
 	sa.counts[0] = ws.ctl.as<uint32_t>();
 	sa.counts[1] = sa.counts[0] + kGroupStride * sa.groups;
@@ -814,6 +840,13 @@ int sorted_points(const tg_program* p, const PointArgs& a, const GradArgs* grad,
 	int rc = ws.take(s);
 	if (rc) return rc;
 	rc = sorted_launches(p, sa, grad, edge, reach, fast, s, *ws.operator->(), ready, sorted);
+	if (rc == TG_ERR_NOMEM)
+	{
+		// no room for the cells' programs (nothing is launched before the last
+		// allocation): the whole program needs none
+		ws->release();
+		return TG_OK;
+	}
 	const int left = ws.leave_to(s);
 	return rc ? rc : left;
 }

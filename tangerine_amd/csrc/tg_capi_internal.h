@@ -147,7 +147,8 @@ namespace tg {
 // Buffers of one host query (tg_eval_points, tg_gradient_points, tg_raymarch),
 // kept between calls.  A call leases a workspace of its device for its whole
 // length, so calls of several threads never share one; the pool keeps at most
-// kPoolSpaces idle ones per device, and none larger than kPoolBytes.
+// kPoolSpaces idle ones per device, and none larger than kPoolBytes, and gives them
+// back where device memory runs out (DevBuf::ensure).
 struct Workspace
 {
 	int device = 0;
@@ -162,6 +163,9 @@ struct Workspace
 	size_t bytes() const;
 	void release();
 };
+
+// Frees the current device's idle workspaces; false if there were none.
+bool free_idle_workspaces();
 
 class WorkspaceLease
 {

@@ -67,3 +67,62 @@ for n in (1000, 700_000):
     p.eval_points(x)
     assert fake.fake_pending() == 0
 """)
+
+
+@pytest.mark.parametrize("device_pointers", [False, True])
+def test_point_queries_without_room_for_cells(device_pointers):
+    """Queries that would be gathered by cell but find no memory for that run the whole
+    program, which needs none beside the points and results of a host call."""
+    run(f"""
+p = program(256)
+n = 700_000
+x, out = np.zeros((n, 3), np.float32), np.zeros(n, np.float32)
+def query():
+    if {device_pointers}:
+        _lib.check(lib.tg_eval_points_device(p.handle, x.ctypes.data, n, out.ctypes.data, 0, None), "query")
+    else:
+        p.eval_points(x)
+room = 0 if {device_pointers} else 16 * n + 4096
+fake.fake_limit(fake.fake_used() + room)
+launches()
+query()
+calls = launches()
+assert ran("k_eval_points", calls) and not ran("sorted", calls) and not ran("k_prune", calls)
+fake.fake_limit(1 << 38)
+query()
+assert ran("k_eval_points_sorted", launches())
+""")
+
+
+def test_gradients_without_room_for_cells():
+    run("""
+from tangerine_amd import trace
+p = program(256)
+n = 300_000
+x = np.zeros((n, 3), np.float32)
+fake.fake_limit(fake.fake_used() + 24 * n + 4096)
+launches()
+trace.gradient(p, x)
+calls = launches()
+assert ran("k_gradient", calls) and not ran("sorted", calls)
+""")
+
+
+def test_idle_workspaces_are_given_back():
+    """What queries left allocated goes where an allocation would fail without it."""
+    run("""
+from tangerine_amd.export import Mesher
+base = fake.fake_used()
+p = program(256)
+p.eval_points(np.zeros((700_000, 3), np.float32))
+kept = fake.fake_used() - base
+assert kept > (1 << 20)
+fake.fake_peak()
+m = Mesher()
+m.export(p, *scenes.grid_for(-6.0, 6.0, 100))
+need = fake.fake_peak() - base - kept
+m.close()
+fake.fake_limit(base + need + kept // 2)
+m = Mesher()
+m.export(p, *scenes.grid_for(-6.0, 6.0, 100))
+""")
