@@ -67,6 +67,7 @@ struct tg_mesher
 	// tg_mesher_set_tuning / set_emission were called: exports then evaluate by
 	// blocks, whatever the grid (see tile_programs)
 	bool by_blocks = false;
+	bool last_by_tiles = false;   // how the last export went
 	int cus = 0;                  // compute units of the device
 	DevBuf persist_args, persist_head, persist_tables;  // the persistent launch's argument copy, queue head, tables
 	DevBuf order_keys, order_values, order, order_tmp;   // its queue: blocks by program cost
@@ -888,8 +889,9 @@ int select_tiles(tg_mesher* m, const tg_program* p, const tg_grid* g, const tg_s
 	return TG_OK;
 }
 
-int run_export(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t flags, bool culled,
-	const tg_surrogate* sur)
+// `tiles` false: by blocks whatever the grid.
+int export_by(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t flags, bool culled, const tg_surrogate* sur,
+	bool tiles)
 {
 	int rc = validate_grid(g);
 	if (rc) return rc;
@@ -924,7 +926,9 @@ int run_export(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t fla
 	TG_CHECK_HIP(hipEventRecord(m->ev[0], m->stream), "event");
 	m->blocks.valid = false;
 	bool sorted = false;
-	const bool by_tiles = !(culled ? m->culled_by_blocks : m->by_blocks) && !(flags & TG_FLAG_NO_PRUNE) && tile_programs(p, ma, culled);
+	const bool by_tiles = tiles && !(culled ? m->culled_by_blocks : m->by_blocks) && !(flags & TG_FLAG_NO_PRUNE) &&
+	                      tile_programs(p, ma, culled);
+	m->last_by_tiles = by_tiles;
 	if (by_tiles)
 	{
 		const BlockGrid t = tile_grid(m, g);
@@ -1030,6 +1034,18 @@ int run_export(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t fla
 	}
 	m->have_grid = !culled;
 	return TG_OK;
+}
+
+int run_export(tg_mesher* m, const tg_program* p, const tg_grid* g, uint32_t flags, bool culled,
+	const tg_surrogate* sur)
+{
+	m->last_by_tiles = false;
+	const int rc = export_by(m, p, g, flags, culled, sur, true);
+	if (rc != TG_ERR_NOMEM || !m->last_by_tiles) return rc;
+	// The passes over 8^3 tiles take up to about 0.7 GB beside the samples (a quarter byte
+	// an entry and tile, and their values), those over blocks a sixty-fourth.
+	m->blocks.release();
+	return export_by(m, p, g, flags, culled, sur, false);
 }
 
 }  // namespace
@@ -1697,7 +1713,10 @@ extern "C" int tg_mesher_export_points(tg_mesher* m, const tg_program* p, const 
 	if (cloud_tiles(p, a) && !(flags & TG_FLAG_NO_PRUNE))
 	{
 		rc = cloud_programs(m, p, a, fast);
-		if (rc) return rc;
+		if (rc == TG_ERR_NOMEM)  // the whole program needs none
+			m->blocks.release();
+		else if (rc)
+			return rc;
 	}
 	if (cells)
 	{
@@ -1713,6 +1732,12 @@ extern "C" int tg_mesher_export_points(tg_mesher* m, const tg_program* p, const 
 		np = uint64_t(tail[0]) + tail[1];
 	}
 	rc = m->vertices.ensure(std::max<uint64_t>(np, 1) * 12);
+	if (rc == TG_ERR_NOMEM && a.desc)
+	{
+		m->blocks.release();
+		a.desc = nullptr;
+		rc = m->vertices.ensure(std::max<uint64_t>(np, 1) * 12);
+	}
 	if (rc) return rc;
 	a.points = m->vertices.as<float>();
 	a.npoints = np;

@@ -670,9 +670,16 @@ extern "C" int tg_raymarch(const tg_program* p, const float* starts, const float
 		return raymarch_staged(p, starts, dirs, count, max_steps, eps, far_distance, flags, hit, travel, position, ds, dd,
 			dt, dp, dh);
 	const bool fast = (flags & TG_FLAG_FAST) != 0;
+	// (no room for cells: the whole program needs none)
+	const auto whole = [&]() {
+		for (CellPrograms& l : ws->levels) l.release();
+		ws->queue.release();
+		return raymarch_staged(p, starts, dirs, count, max_steps, eps, far_distance, flags, hit, travel, position, ds, dd,
+			dt, dp, dh);
+	};
 	rc = ws->queue.ensure(count * sizeof(TraceRay));
 	if (!rc) rc = ws->ctl.ensure(256);
-	if (rc) return rc;
+	if (rc) return rc == TG_ERR_NOMEM ? whole() : rc;
 	ws.queued();
 	TG_CHECK_HIP(hipMemcpyAsync(ds, starts, count * 12, hipMemcpyHostToDevice, nullptr), "ray upload");
 	TG_CHECK_HIP(hipMemcpyAsync(dd, dirs, count * 12, hipMemcpyHostToDevice, nullptr), "ray upload");
@@ -685,7 +692,7 @@ extern "C" int tg_raymarch(const tg_program* p, const float* starts, const float
 	// and each call then allocates and frees some 300 MiB)
 	const uint32_t rooms[2] = { 0, 16 + uint32_t(1.5f * p->kept * float(p->decoded.entries.size())) };
 	rc = build_levels(nullptr, p, doms, ns, cubes, fast, ws->levels, ws->launches, ta, rooms);
-	if (rc) return rc;
+	if (rc) return rc == TG_ERR_NOMEM ? whole() : rc;
 	ta.starts = ds;
 	ta.dirs = dd;
 	ta.nrays = uint32_t(count);

@@ -1,0 +1,81 @@
+"""Calls whose usual route needs more memory than there is take the one that needs
+little, without a device: each runs within what it needed by that route."""
+
+import pytest
+
+from tests.fake_device import run
+
+
+@pytest.mark.parametrize("culled", [False, True])
+@pytest.mark.parametrize("headroom", [0, 1 << 20, 1 << 22, 1 << 24])
+def test_exports_go_by_blocks(culled, headroom):
+    """Within the memory of an export by blocks, and a little more: the passes over
+    tiles find no room at their start, or the later stages none behind them."""
+    run(f"""
+from tangerine_amd.export import Mesher
+p = program(1500)
+g = scenes.grid_for(-6.0, 6.0, 200)
+def export(blocks):
+    m = Mesher()
+    if blocks:
+        m.set_tuning(4, 2, 8, 8)
+        m.set_culled_tuning(4, 4, 6)
+    fake.fake_peak()
+    launches()
+    st = m.export_culled(p, None, *g) if {culled} else m.export(p, *g)
+    return m, launches()
+base = fake.fake_used()
+m, calls = export(True)
+need = fake.fake_peak() - base
+m.close()
+m, calls = export(False)
+assert ran("k_eval_tile_programs", calls)
+more = fake.fake_peak() - base
+m.close()
+assert more > need + (1 << 24), (need, more)
+fake.fake_limit(base + need + {headroom})
+m, calls = export(False)
+assert not ran("k_eval_tile_programs", calls)
+fake.fake_limit(1 << 38)
+m.export(p, *g)
+assert ran("k_eval_tile_programs", launches())
+""")
+
+
+def test_point_clouds_take_the_whole_program():
+    run("""
+from tangerine_amd.export import Mesher
+p = program(256)
+def cloud(m):
+    fake.fake_peak()
+    launches()
+    m.export_points(p, (-6.0,) * 3, (6.0,) * 3, (0.1,) * 3, refine_iterations=2)
+    return launches()
+base = fake.fake_used()
+m = Mesher()
+assert ran("k_cloud_select_tiles", cloud(m))
+m.close()
+base = fake.fake_used()
+fake.fake_limit(base + 121 ** 3 * 8 + (1 << 20))  # flags and ranks
+m = Mesher()
+calls = cloud(m)
+assert ran("k_cloud_select", calls) and not ran("tiles", calls)
+""")
+
+
+@pytest.mark.parametrize("headroom", [0, 1 << 18, 1 << 23])
+def test_ray_casts_take_the_whole_program(headroom):
+    run(f"""
+from tangerine_amd import trace
+p = program(256)
+s = np.full((5000, 3), 9.0, np.float32)
+fake.fake_limit(fake.fake_used() + 5000 * 41 + 512 + {headroom})
+launches()
+trace.raymarch(p, s, -s)
+calls = launches()
+assert ran("k_trace", calls) and not ran("k_march", calls)
+assert fake.fake_pending() == 0
+fake.fake_limit(1 << 38)
+trace.raymarch(p, s, -s)
+assert ran("k_march", launches())
+""")
