@@ -2214,21 +2214,17 @@ extern "C" int tg_batch_set_tuning(tg_batch* b, uint32_t points_per_lane, uint32
 	return TG_OK;
 }
 
-extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, const tg_grid* grids, uint32_t count,
-	uint32_t flags)
+namespace {
+
+// Device memory that the trees of a batch which go by tile programs may take for
+// those, a seventeenth of the card's; the trees after that go by blocks, whose passes
+// need a sixty-fourth.
+constexpr uint64_t kBatchTileBytes = 16ull << 30;
+
+// `tiles` false: every tree by blocks.
+int export_batch(tg_batch* b, const tg_program* const* programs, const tg_grid* grids, uint32_t count, uint32_t flags,
+	bool tiles)
 {
-	if (!b || (count && (!programs || !grids))) return fail(TG_ERR_INVALID, "tg_batch_export: null argument");
-	if (count == 0 || count > 4096) return fail(TG_ERR_INVALID, "tg_batch_export: 1..4096 trees");
-	if (flags & TG_FLAG_NO_PRUNE) return fail(TG_ERR_INVALID, "tg_batch_export: the batch evaluates pruned blocks");
-	for (uint32_t i = 0; i < count; ++i)
-	{
-		if (!programs[i]) return fail(TG_ERR_INVALID, "tg_batch_export: null program");
-		if (!programs[i]->decoded.prunable())
-			return fail(TG_ERR_PROGRAM, "tg_batch_export: every tree must be prunable (1-Lipschitz, at most 128 "
-			                            "nested blend / flate / field-scale operators)");
-		int rc = validate_grid(&grids[i]);
-		if (rc) return rc;
-	}
 	drop_graph(b);
 	b->exported = false;
 	b->fast = (flags & TG_FLAG_FAST) != 0;
@@ -2262,6 +2258,7 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 	const bool fast = (flags & TG_FLAG_FAST) != 0;
 	std::vector<CellGrid> cgs(count);
 	std::vector<CellPrograms*> outs(count);
+	uint64_t tile_bytes = 0;
 	for (uint32_t i = 0; i < count; ++i)
 	{
 		tg_mesher* m = b->meshers[i];
@@ -2269,7 +2266,12 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 		m->nbricks = 0;
 		rc = layout(m, &grids[i]);
 		if (rc) return rc;
-		b->by_tiles[i] = !b->by_blocks && tile_programs(programs[i], m->args) ? 1 : 0;
+		if (tiles && !b->by_blocks && tile_programs(programs[i], m->args))
+		{
+			const uint64_t bytes = tile_program_bytes(programs[i], uint64_t(m->args.tx) * m->args.ty * m->args.tz);
+			b->by_tiles[i] = tile_bytes + bytes <= kBatchTileBytes ? 1 : 0;
+			if (b->by_tiles[i]) tile_bytes += bytes;
+		}
 		const BlockGrid bg = b->by_tiles[i] ? tile_grid(m, &grids[i]) : block_grid(m, &grids[i]);
 		CellGrid& cg = cgs[i];
 		cg.words = b->by_tiles[i] != 0;
@@ -2284,7 +2286,7 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 	}
 	std::vector<TileEvalArgs> tile_jobs;
 	std::vector<uint32_t> tile_base;
-	uint64_t tiles = 0;
+	uint64_t ntiles = 0;
 	b->tile_njobs = b->tile_blocks = 0;
 	b->tile_lds = 0;
 	rc = prune_cells_many(b->stream, programs, cgs.data(), count, fast, outs.data(), b->prune);
@@ -2303,7 +2305,7 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 			const TileEvalArgs ta = tile_args(m, programs[i], &grids[i], work);
 			tile_jobs.push_back(ta);
 			b->tile_lds = std::max(b->tile_lds, spill_bytes_per_wave(ta.slots, int(ta.points)));
-			tiles += ta.ntiles;
+			ntiles += ta.ntiles;
 			continue;
 		}
 		args[i] = block_args(m, programs[i], &grids[i], nullptr, nullptr, 0, work);
@@ -2453,7 +2455,7 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 	st.mesh_ms = mesh_ms;
 	st.total_ms = std::chrono::duration<double, std::milli>(t3 - t0).count();
 	st.trees = count;
-	st.blocks = b->args.total + tiles;
+	st.blocks = b->args.total + ntiles;
 	st.samples = samples;
 	st.exact_evals = evals;
 	st.flops = flops;
@@ -2467,6 +2469,32 @@ extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, c
 	st.max_binary = q.max_binary;
 	st.max_depth = q.max_depth;
 	return TG_OK;
+}
+
+}  // namespace
+
+extern "C" int tg_batch_export(tg_batch* b, const tg_program* const* programs, const tg_grid* grids, uint32_t count,
+	uint32_t flags)
+{
+	if (!b || (count && (!programs || !grids))) return fail(TG_ERR_INVALID, "tg_batch_export: null argument");
+	if (count == 0 || count > 4096) return fail(TG_ERR_INVALID, "tg_batch_export: 1..4096 trees");
+	if (flags & TG_FLAG_NO_PRUNE) return fail(TG_ERR_INVALID, "tg_batch_export: the batch evaluates pruned blocks");
+	for (uint32_t i = 0; i < count; ++i)
+	{
+		if (!programs[i]) return fail(TG_ERR_INVALID, "tg_batch_export: null program");
+		if (!programs[i]->decoded.prunable())
+			return fail(TG_ERR_PROGRAM, "tg_batch_export: every tree must be prunable (1-Lipschitz, at most 128 "
+			                            "nested blend / flate / field-scale operators)");
+		int rc = validate_grid(&grids[i]);
+		if (rc) return rc;
+	}
+	int rc = export_batch(b, programs, grids, count, flags, true);
+	if (rc != TG_ERR_NOMEM || std::find(b->by_tiles.begin(), b->by_tiles.end(), 1) == b->by_tiles.end()) return rc;
+	// without tile programs a batch needs little more than its samples
+	for (tg_mesher* m : b->meshers) m->blocks.release();
+	b->tile_jobs.release();
+	b->prune.dev.release();
+	return export_batch(b, programs, grids, count, flags, false);
 }
 
 extern "C" int tg_batch_replay(tg_batch* b, double* eval_ms)

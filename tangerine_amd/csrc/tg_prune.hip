@@ -272,6 +272,15 @@ bool treelet_prunable(const tg_program* p, uint64_t ncells)
 	return p->plan.stages() <= kMaxStages && uint64_t(p->plan.slots) * ((ncells + 15) / 16) * 256 <= kMaxValueBytes;
 }
 
+uint64_t tile_program_bytes(const tg_program* p, uint64_t ncells)
+{
+	const DecodedProgram& d = p->decoded;
+	const uint64_t waves = (ncells + 63) / 64, entries = d.entries.size();
+	const uint64_t scratch = waves * prune_scratch_words(d.binary_entries, uint32_t(entries)) * 8;
+	const uint64_t values = uint64_t(p->plan.slots) * waves * 256;
+	return scratch + values + waves * 256 + ncells * (sizeof(BlockDesc) + 4 * std::min<uint64_t>(std::max<uint64_t>(entries / 4, 16), 64));
+}
+
 int prune_cells_start(hipStream_t stream, const tg_program* p, const float origin[3], const float cell[3],
 	float radius, const uint32_t counts[3], bool fast, CellPrograms& out, bool words)
 {

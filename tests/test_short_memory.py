@@ -79,3 +79,57 @@ fake.fake_limit(1 << 38)
 trace.raymarch(p, s, -s)
 assert ran("k_march", launches())
 """)
+
+
+BATCH = """
+from tangerine_amd.batch import Batch
+def batch(trees, cells, p, blocks):
+    b = Batch()
+    if blocks:
+        b.set_tuning(4, 4, 4)  # (the shape of an untuned batch)
+    fake.fake_peak()
+    launches()
+    st = b.export([p] * trees, [scenes.grid_for(-6.0, 6.0, cells)] * trees)
+    return b, st, launches()
+def units(cells):
+    t = cells // 8 + 1
+    return t ** 3, (-(-t // 4)) ** 3
+"""
+
+
+@pytest.mark.parametrize("headroom", [0, 1 << 20, 1 << 24, 1 << 27])
+def test_batches_go_by_blocks(headroom):
+    run(BATCH + f"""
+tiles, blocks = units(150)
+p = program(1500)
+base = fake.fake_used()
+b, st, calls = batch(32, 150, p, True)
+need = fake.fake_peak() - base
+assert st["blocks"] == 32 * blocks
+b.close()
+b, st, calls = batch(32, 150, p, False)
+assert st["blocks"] == 32 * tiles and fake.fake_peak() - base > need + (1 << 27)
+b.close()
+fake.fake_limit(base + need + {headroom})
+b, st, calls = batch(32, 150, p, False)
+assert st["blocks"] == 32 * blocks and not ran("k_eval_tile_programs", calls)
+assert b.replay() > 0
+""")
+
+
+def test_tile_programs_of_a_large_batch_are_bounded():
+    """200 trees whose tile programs would take 21 GB: as many as 16 GiB hold go by
+    tiles, the others by blocks."""
+    run(BATCH + """
+tiles, blocks = units(330)
+p = program(2048)
+base = fake.fake_used()
+b, st, calls = batch(200, 330, p, True)
+need = fake.fake_peak() - base
+b.close()
+b, st, calls = batch(200, 330, p, False)
+by_tiles = (st["blocks"] - 200 * blocks) / (tiles - blocks)
+assert by_tiles == int(by_tiles) and 0 < by_tiles < 200, by_tiles
+assert fake.fake_peak() - base <= need + (17 << 30), (fake.fake_peak(), need)
+assert ran("k_eval_tile_programs_multi", calls) and ran("k_eval_batch", calls)
+""")
