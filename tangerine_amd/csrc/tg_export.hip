@@ -2517,6 +2517,7 @@ extern "C" int tg_batch_autotune(tg_batch* b, tg_batch_tune_result* out)
 	const int pts_c[3] = { 2, 4, 8 };
 	const int shape_c[6][2] = { { 4, 2 }, { 4, 3 }, { 4, 4 }, { 4, 6 }, { 2, 6 }, { 2, 8 } };
 	tg_batch_tune_result r{};
+	const int kept[3] = { b->points_per_lane, b->waves, b->workgroups_per_cu };
 	double best = 1e300;
 	uint32_t k = 0;
 	for (int pi = 0; pi < 3; ++pi)
@@ -2550,6 +2551,13 @@ extern "C" int tg_batch_autotune(tg_batch* b, tg_batch_tune_result* out)
 		}
 	r.candidates = k;
 	r.eval_ms = best;
+	if (b->args.total == 0)
+	{
+		// no tree went through the queue: its shape made no difference
+		r.points_per_lane = uint32_t(kept[0]);
+		r.waves = uint32_t(kept[1]);
+		r.workgroups_per_cu = uint32_t(kept[2]);
+	}
 	b->points_per_lane = int(r.points_per_lane);
 	b->waves = int(r.waves);
 	b->workgroups_per_cu = int(r.workgroups_per_cu);
