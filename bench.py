@@ -90,11 +90,11 @@ def roofline(flops: float, ms: float, kernel: str, **extra) -> dict:
     return out
 
 
-def block_kernel(st: dict, prune: bool, tuning: dict | None) -> str:
+def block_kernel(st: dict, prune: bool) -> str:
     """The grid-evaluation kernel an export's stats describe."""
     if not prune:
         return "k_eval_tiles"
-    if not st["block_workgroups"] and (tuning is None or tuning["workgroups_per_cu"]):
+    if not st["block_max_len"]:  # no block programs
         return f"k_eval_tile_programs ({st['points_per_lane']} points per lane)"
     if st["block_workgroups"]:
         return f"k_eval_batch<{st['points_per_lane']},true> (persistent block evaluation, one tree)"
@@ -338,7 +338,7 @@ def train_mfma(fit: dict) -> dict:
 def batch_leg(args) -> dict:
     """64 seeded trees exported together: a cold export (buffers allocated),
     warm exports (the whole pipeline again: pruning, evaluation, surface nets),
-    then the captured persistent evaluation replayed."""
+    then the captured evaluation replayed."""
     from tangerine_amd.batch import Batch
     specs = scenes.batch_specs(4, 64)
     progs = [scenes.build_sdf(spec).program() for spec, _ in specs]
@@ -348,8 +348,12 @@ def batch_leg(args) -> dict:
     t0 = time.perf_counter()
     b.export(progs, grids, fast=args.fast)
     cold_ms = 1000.0 * (time.perf_counter() - t0)
+    # trees that go by tile programs have no items in the queue of k_eval_batch
+    queue_only = sum((-(-(res // 8 + 1) // 4)) ** 3 for _, res in specs)
+    queue, tiles = b.stats()["max_len"] > 0, b.stats()["blocks"] != queue_only
+    kernel = " and ".join((["k_eval_batch"] if queue else []) + (["k_eval_tile_programs_multi"] if tiles else []))
     tune = None
-    if not args.no_autotune:
+    if not args.no_autotune and queue:
         tune = b.autotune()
         log(f"batch autotune: {tune['points_per_lane']} points/lane, {tune['waves']} waves, "
             f"{tune['workgroups_per_cu']} workgroups/CU, {tune['eval_ms']:.2f} ms")
@@ -372,7 +376,7 @@ def batch_leg(args) -> dict:
         "eval_ms_replay": replay_ms,
         "samples_per_s_replay": samples / (replay_ms * 1e-3),
         "samples_per_s_warm_export": samples / (float(np.mean(warm)) * 1e-3),
-        "roofline": roofline(st["flops"], replay_ms, "k_eval_batch (captured replay)"),
+        "roofline": roofline(st["flops"], replay_ms, f"{kernel} (captured replay)"),
         "launch": {"points_per_lane": st["points_per_lane"], "waves": st["waves"], "workgroups": st["workgroups"],
                    "lds_bytes": st["lds_bytes"], "max_len": st["max_len"]},
         "autotune": None if tune is None else {k: tune[k] for k in ("points_per_lane", "waves", "workgroups_per_cu",
@@ -478,7 +482,7 @@ def main(argv=None) -> int:
     nverts, ntris = mesher.counts()
     prune = not args.no_prune
     launch_ms = res["block_ms"] if prune and res["block_ms"] > 0 else res["eval_ms"]
-    kernel = block_kernel(st, prune, tuning)
+    kernel = block_kernel(st, prune)
     traffic = MEASURED_TRAFFIC_BYTES.get(args.workload) if prune and not args.fast else None
     rl = roofline(st["flops"], launch_ms, kernel,
                   traffic=traffic,
@@ -521,7 +525,7 @@ def main(argv=None) -> int:
                                       f"{args.workload} fast")
         fms = fres["block_ms"] if prune and fres["block_ms"] > 0 else fres["eval_ms"]
         out["fast"] = {"ms_per_step": fres["ms_per_step"], "samples_per_s": samples / (fres["ms_per_step"] * 1e-3),
-                       "autotune": ftune, "roofline": roofline(fst["flops"], fms, block_kernel(fst, prune, ftune) + " (fast numerics)")}
+                       "autotune": ftune, "roofline": roofline(fst["flops"], fms, block_kernel(fst, prune) + " (fast numerics)")}
         # back to the exact export (and its launch shape) for the surrogate leg's comparison
         if tuning:
             mesher.set_tuning(tuning["points_per_lane"], tuning["waves"], tuning.get("min_prune_len", 0),
@@ -550,7 +554,7 @@ def main(argv=None) -> int:
         out["export512"] = {"workload": "256 random primitives (seed 1), 512^3 cells over [-6,6]^3",
                             "samples": n2, "ms_per_step": r2["ms_per_step"], "export_ms_device": r2["export_ms_device"],
                             "samples_per_s": n2 / (r2["ms_per_step"] * 1e-3), "autotune": t2,
-                            "roofline": roofline(st2["flops"], ms2, block_kernel(st2, prune, t2),
+                            "roofline": roofline(st2["flops"], ms2, block_kernel(st2, prune),
                                                  traffic=MEASURED_TRAFFIC_BYTES["export512"]
                                                  if prune and not args.fast else None)}
 
