@@ -715,7 +715,7 @@ int sorted_launches(const tg_program* p, SortedPointsArgs& sa, const GradArgs* g
 	const float* xyz = sa.p.xyz;
 	float* out = sa.p.out;
 	sa.bins = sa.groups = 1;
-	sa.chunk_shift = grad ? 4 : 6;
+	sa.chunk_shift = !grad ? 6 : grad->tetra ? 4 : 5;
 	CellGrid grids[2];
 	for (int L = 0; L < 2; ++L)
 	{

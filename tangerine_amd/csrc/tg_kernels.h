@@ -54,7 +54,7 @@ struct SortedPointsArgs
 	uint32_t* counts[2];       // per group (kGroupStride words apart) / per bin (zeroed): points
 	uint32_t* first[2];        // per group / per bin, and one more: points in those before it
 	uint32_t* chunk;           // per bin and one more: chunks in the bins before it
-	uint32_t chunk_shift;      // points per chunk, a wave's: 2^6, for gradients 2^4
+	uint32_t chunk_shift;      // points per chunk, a wave's: 2^6, for gradients 2^4 or 2^5
 	uint32_t* rank;            // per point: its place among its group's / its bin's
 	float4* sorted[2];         // per point, by group / by bin: x, y, z, the point's index as bits
 	const uint32_t* words[2];  // the cells' programs (PruneArgs::words)
