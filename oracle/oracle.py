@@ -296,6 +296,12 @@ class Oracle(_Cpu):
         self.lib.tgo_mt19937_10000th.restype = C.c_uint32
         return int(self.lib.tgo_mt19937_10000th())
 
+    def training_order(self, seed: int, n: int) -> np.ndarray:
+        out = np.zeros(n, dtype=np.uint32)
+        self.lib.tgo_training_order.argtypes = [C.c_uint64, C.c_uint64, _u32p]
+        self.lib.tgo_training_order(int(seed), int(n), out.ctypes.data_as(_u32p))
+        return out
+
     def vertex_sequence(self, n: int) -> np.ndarray:
         out = np.zeros(n, dtype=np.uint32)
         self.lib.tgo_vertex_sequence.argtypes = [C.c_uint64, _u32p]

@@ -1391,4 +1391,13 @@ uint32_t tgo_mt19937_10000th(void)
 
 void tgo_vertex_sequence(uint64_t n, uint32_t* exchange) { vertex_sequence(n, exchange); }
 
+// The order in which a surrogate fit of this seed takes its n samples (no reference
+// counterpart; pinned by the fit's own losses).
+void tgo_training_order(uint64_t seed, uint64_t n, uint32_t* out)
+{
+	for (uint64_t i = 0; i < n; ++i) out[i] = uint32_t(i);
+	std::mt19937_64 rng(seed ^ 0x5eedull);
+	std::shuffle(out, out + n, rng);
+}
+
 }  // extern "C"
