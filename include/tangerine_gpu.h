@@ -121,16 +121,16 @@ typedef struct tg_export_stats
 	double flops;              /* algorithmic FP32 work (cost table) of the programs run at the grid's samples */
 	uint64_t bricks_total;     /* culled export: 8^3-cube bricks of the grid (0 otherwise) */
 	uint64_t bricks_flagged;   /* culled export: bricks the surrogate kept for exact evaluation */
-	double prune_ms;           /* block pruning, and for a culled export brick selection (HIP events; inside eval_ms) */
+	double prune_ms;           /* block or tile pruning, and for a culled export brick selection (HIP events; inside eval_ms) */
 	double cull_threshold;     /* culled export: bricks with |prediction at the centre| above this were skipped */
 	uint64_t bricks_certified; /* culled export: bricks the exact certificate kept that the surrogate skipped */
-	double block_ms;           /* the pruned block-evaluation kernel alone (HIP events; 0 if it did not run) */
+	double block_ms;           /* the pruned evaluation kernel alone (HIP events; 0 if it did not run) */
 	uint32_t points_per_lane;  /* its launch: points per lane and waves per workgroup */
 	uint32_t waves;
-	uint32_t block_max_len;    /* longest pruned block program (entries) and its binary entries */
+	uint32_t block_max_len;    /* longest pruned block program (entries) and its binary entries (both 0: from tile programs) */
 	uint32_t block_max_binary;
-	uint32_t block_lds_bytes;  /* LDS per workgroup of the block kernel */
-	uint32_t block_workgroups; /* persistent workgroups of that launch (0: a workgroup per block) */
+	uint32_t block_lds_bytes;  /* LDS per workgroup of that kernel */
+	uint32_t block_workgroups; /* persistent workgroups of that launch (0: a workgroup per block, or tile programs) */
 } tg_export_stats;
 
 typedef struct tg_surrogate_stats
@@ -216,7 +216,11 @@ void tg_program_destroy(tg_program* program);
 /* ---- point queries (EvalTree / SDFNode::Eval, batched) --------------------- */
 /* xyz: 3 floats per point; host buffers. */
 int tg_eval_points(const tg_program* program, const float* xyz, uint64_t count, float* out, uint32_t flags);
-/* Same with device buffers on `stream` (a hipStream_t, or NULL for the null stream). */
+/* Same with device buffers on `stream` (a hipStream_t, or NULL for the null stream).
+ * Many points may be gathered by cell and evaluated with pruned programs: the call
+ * then allocates up to a few hundred MB, which the library keeps for later calls and
+ * gives back when it needs the memory elsewhere.  It allocates nothing while `stream`
+ * is captured, and does without where memory is short. */
 int tg_eval_points_device(const tg_program* program, const float* xyz, uint64_t count, float* out,
                           uint32_t flags, void* stream);
 
@@ -386,7 +390,10 @@ int tg_mesher_copy_normals(const tg_mesher* mesher, float* normals);
  * the program.
  * tg_mesher_autotune prunes `program` for `grid`, times every launch on the
  * device, then the threshold at the fastest launch, and keeps the best for
- * later exports on this mesher.  Every setting writes the same samples. */
+ * later exports on this mesher that go by blocks: grids of few tiles and short
+ * programs are still evaluated from tile programs (see
+ * tg_mesher_set_emission), unless tg_mesher_set_tuning sets the result.  Every
+ * setting writes the same samples. */
 typedef struct tg_tune_result
 {
 	uint32_t points_per_lane;     /* chosen */
@@ -419,34 +426,38 @@ int tg_mesher_set_culled_tuning(tg_mesher* mesher, uint32_t points_per_lane, uin
  * walking the entries of 16 blocks at a time, 2 a wave per block.  Every
  * setting emits the same programs, so exports give the same samples and
  * mesh.  A mesher whose emission or tuning was set (to any value) evaluates
- * every grid by blocks; one left alone evaluates grids of few tiles and short
- * programs a wave per 8^3-sample tile, with the same samples. */
+ * every plain export by blocks; one left alone (or autotuned) evaluates grids of
+ * few tiles and short programs a wave per 8^3-sample tile, with the same
+ * samples.  Culled exports go by tg_mesher_set_culled_tuning alone. */
 int tg_mesher_set_emission(tg_mesher* mesher, uint32_t mode);
 
 /* ---- batched export (no reference counterpart; closest: one Sodapop
  * MeshingJob per model on Scheduler workers, sodapop.cpp:214-224,
  * scheduler.cpp:307-330) ------------------------------------------------------
- * Exports many trees, each on its own grid: every tree is pruned per block,
- * then all trees' blocks are evaluated by one persistent launch that takes
- * work items (one block of one tree) from a device queue, heaviest trees
- * first; the launch is captured in a hipGraph.  Each tree's samples and mesh
+ * Exports many trees, each on its own grid.  Grids of few tiles and short
+ * programs are pruned per 8^3-sample tile and evaluated a wave per tile, all
+ * trees' in one launch (up to 16 GiB of tile programs, and not once
+ * tg_batch_set_tuning was called); the other trees are pruned per block, and
+ * one persistent launch takes their work items (one block of one tree) from a
+ * device queue, the costliest first.  tg_batch_replay captures both launches in
+ * a hipGraph.  Each tree's samples and mesh
  * stay in its own mesher (tg_batch_mesher), so tg_mesher_counts /
  * tg_mesher_copy_mesh / tg_mesher_copy_grid read them.  Programs must be
  * 1-Lipschitz and stay alive while the batch is replayed. */
 typedef struct tg_batch_stats
 {
-	double prune_ms;           /* layout and per-tree block pruning (host clock) */
-	double eval_ms;            /* the persistent launch (graph replay, HIP events) */
+	double prune_ms;           /* layout and pruning of every tree (host clock) */
+	double eval_ms;            /* the evaluation launches (HIP events) */
 	double mesh_ms;            /* surface nets of every tree (host clock) */
 	double total_ms;
 	uint64_t trees;
-	uint64_t blocks;           /* queue items */
+	uint64_t blocks;           /* queue items, and the tiles of the trees that go by tile programs */
 	uint64_t samples;
 	uint64_t exact_evals;
 	double flops;
-	uint32_t points_per_lane, waves, workgroups;
-	uint32_t lds_bytes;        /* LDS per workgroup of the short-program launch (the long one if none) */
-	uint32_t max_len, max_binary, max_depth;  /* its layout: the largest over its queue */
+	uint32_t points_per_lane, waves, workgroups;  /* of the queue's launch */
+	uint32_t lds_bytes;        /* LDS per workgroup of that launch */
+	uint32_t max_len, max_binary, max_depth;  /* its layout: the largest over its queue (0: no items) */
 } tg_batch_stats;
 typedef struct tg_batch_tune_result
 {
@@ -462,11 +473,12 @@ int tg_batch_export(tg_batch* batch, const tg_program* const* programs, const tg
                     uint32_t flags);
 /* Replays the captured evaluation launch of the last export (same trees). */
 int tg_batch_replay(tg_batch* batch, double* eval_ms);
-/* Times points per lane {2,4,8} x waves {2,4} x persistent workgroups per CU
- * {1,2,4} for the short-program queue (blocks of at most 256 entries) on the
- * last exported batch, keeps the fastest, then picks the long-program queue's
- * shape among seven; eval_ms is the best whole-batch time seen. */
+/* Times points per lane {2,4,8} x six pairs of waves and persistent workgroups
+ * per CU on the last exported batch and keeps the fastest shape for the queue's
+ * launch (that of a batch without queue items makes no difference: it keeps the
+ * shape it had); eval_ms is the best whole-batch time seen. */
 int tg_batch_autotune(tg_batch* batch, tg_batch_tune_result* out);
+/* The queue's launch shape; later exports evaluate every tree through the queue. */
 int tg_batch_set_tuning(tg_batch* batch, uint32_t points_per_lane, uint32_t waves, uint32_t workgroups_per_cu);
 /* Tree `index`'s mesher, owned by the batch: read its results (counts, mesh,
  * grid, stats, bricks, STL/PLY writers); exports, tuning and destroy on it

@@ -1,4 +1,4 @@
-"""Batched export of many trees in one persistent launch (tg_batch_*)."""
+"""Batched export of many trees in shared launches (tg_batch_*)."""
 
 from __future__ import annotations
 

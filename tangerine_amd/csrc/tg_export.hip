@@ -2253,8 +2253,8 @@ int export_batch(tg_batch* b, const tg_program* const* programs, const tg_grid* 
 	std::vector<BlockEvalArgs> args(count);
 	BatchArgs ba{};
 	uint64_t samples = 0;
-	// every tree's pruning on the batch's stream: each height of every tree's
-	// level pass in one launch, every tree's emission in one launch, one wait
+	// every tree's pruning on the batch's stream: each stage of every tree's
+	// treelet passes in one launch, every tree's emission in one launch, one wait
 	const bool fast = (flags & TG_FLAG_FAST) != 0;
 	std::vector<CellGrid> cgs(count);
 	std::vector<CellPrograms*> outs(count);

@@ -195,8 +195,7 @@ int prune_pass(hipStream_t stream, const tg_program* p, const float origin[3], c
 
 namespace {
 
-// Everything of prune_cells_start before the passes: sizes, buffers and the
-// upload of the entries by height.  *ready is false when the program is not
+// Everything of prune_cells_start before the passes: sizes and buffers.  *ready is false when the program is not
 // pruned here.
 int prune_prepare(hipStream_t stream, const tg_program* p, const float origin[3], const float cell[3],
 	float radius, const uint32_t counts[3], CellPrograms& out, bool words, uint32_t room, bool* ready)

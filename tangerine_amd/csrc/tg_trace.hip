@@ -43,7 +43,8 @@ struct Transform8
 // interpreted first_entries() entries, and its rays go on in k_trace_groups: 16
 // lanes to a ray, then a wave to each ray that meets a longer program than those
 // hold, then (k_trace_resume, from kMaxGroupEntries entries on) the rest.
-// Whole call, passes of 32 + 224 steps with a wave to each ray left / this, ms:
+// Pruning and marching (the call without its read-back), passes of 32 + 224 steps with
+// a wave to each ray left / this, ms:
 // 1920x1080 of 256 primitives 7.28 / 4.75 and (another scene) 8.57 / 6.26, of 512
 // 16.2 / 10.5, of 16 1.38 / 1.31; 640x360 of 64 1.91 / 1.23, of 2048 40.2 / 20;
 // 320x180 of 256 5.16 / 2.25.

@@ -57,7 +57,7 @@ class Mesher:
 
     def autotune(self, program, origin, step, cells, fast: bool = False) -> dict:
         """Time every (points per lane, waves) configuration of the block
-        kernel on this grid and keep the fastest for later exports."""
+        kernel on this grid and keep the fastest for later exports by blocks."""
         g = _lib.grid_struct(origin, step, cells)
         r = _lib.TgTuneResult()
         check(self.lib.tg_mesher_autotune(self.h, program.handle, C.byref(g), _lib.TG_FLAG_FAST if fast else 0,
