@@ -21,8 +21,8 @@ of the same line (--legs picks them; default all):
   surrogate   surrogate fit, then culled exports (surrogate + certificate,
               certificate alone, surrogate alone) compared with the plain one
   batch64     64 seeded trees (8..2048 primitives, {64..384}^3 over [-6,6]^3):
-              cold and warm whole-batch exports, and the captured persistent
-              evaluation replayed
+              cold and warm whole-batch exports, and the captured evaluation
+              replayed
   trace1080p  sphere tracing of the 256-primitive tree (seed 1) at 1920x1080
               from a seeded eye on the sphere of radius 12: at most 256 steps,
               hit at d <= 1e-4, far 40, central-difference normals (h = 1e-3)

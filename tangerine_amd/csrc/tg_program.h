@@ -52,7 +52,8 @@ constexpr uint32_t kTreeletItems = 32;
 // Of a program split over a workgroup, treelets above others: where a cut subtree
 // occurs only this many.  The widest stage is the first; those above it leave waves
 // idle, so they are cut finer: a stage of 7 items costs less than one wave running
-// 31.  (One point / 50k rays, us, 32 items everywhere / 8 above: 256 primitives 32 /
+// 31.  (One point / 50k rays, us, one scene each, before a treelet's items were read in
+// one load, 32 items everywhere / 8 above: 256 primitives 32 /
 // 30, 4117 / 3707; 120, 36 / 28, 2859 / 2184; 300, 52 / 33, 5757 / 3777; 2000, 122 /
 // 115, 25460 / 24118; 4 and 16 within 2% of 8.)
 constexpr uint32_t kSplitUpperItems = 8;
