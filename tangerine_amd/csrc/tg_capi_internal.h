@@ -111,7 +111,7 @@ int launch_gradients(const tg_program* p, const GradArgs& a, uint32_t flags, hip
 // Whether `p` can be pruned over ncells cells by the treelet passes.
 bool treelet_prunable(const tg_program* p, uint64_t ncells);
 
-// Device memory of `p` pruned to a word an entry over ncells cells (a first pass).
+// Device memory of `p` pruned to a word an entry over ncells cells, about.
 uint64_t tile_program_bytes(const tg_program* p, uint64_t ncells);
 
 // A cell grid to prune a program over.

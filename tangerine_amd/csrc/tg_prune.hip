@@ -277,7 +277,9 @@ uint64_t tile_program_bytes(const tg_program* p, uint64_t ncells)
 	const uint64_t waves = (ncells + 63) / 64, entries = d.entries.size();
 	const uint64_t scratch = waves * prune_scratch_words(d.binary_entries, uint32_t(entries)) * 8;
 	const uint64_t values = uint64_t(p->plan.slots) * waves * 256;
-	return scratch + values + waves * 256 + ncells * (sizeof(BlockDesc) + 4 * std::min<uint64_t>(std::max<uint64_t>(entries / 4, 16), 64));
+	// the pool: its first guess, or what the tiles keep if that is more
+	const uint64_t kept = std::max(std::min<uint64_t>(std::max<uint64_t>(entries / 4, 16), 64), uint64_t(double(p->kept) * double(entries)));
+	return scratch + values + waves * 256 + ncells * (sizeof(BlockDesc) + 4 * kept);
 }
 
 int prune_cells_start(hipStream_t stream, const tg_program* p, const float origin[3], const float cell[3],

@@ -1,7 +1,9 @@
 """Runs a script against libtangerine_gpu.so with tests/fake_hip.cpp in the HIP
 runtime's place: the library's host code without a device."""
 
+import atexit
 import functools
+import shutil
 import subprocess
 import sys
 import tempfile
@@ -43,6 +45,7 @@ def program(prims, seed=1):
 def _fake_lib():
     from tangerine_amd.build import HIPCC
     out = Path(tempfile.mkdtemp(prefix="fake_hip_")) / "libfake_hip.so"
+    atexit.register(shutil.rmtree, out.parent, True)
     subprocess.run([HIPCC, "--offload-arch=gfx950", "-O1", "-std=c++17", "-shared", "-fPIC", "-o", str(out),
                     str(ROOT / "tests" / "fake_hip.cpp")], check=True, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)
     return out

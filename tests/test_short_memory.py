@@ -133,3 +133,15 @@ assert by_tiles == int(by_tiles) and 0 < by_tiles < 200, by_tiles
 assert fake.fake_peak() - base <= need + (17 << 30), (fake.fake_peak(), need)
 assert ran("k_eval_tile_programs_multi", calls) and ran("k_eval_batch", calls)
 """)
+
+
+def test_what_tiles_keep_counts_towards_the_bound():
+    """Tiles of wide blends keep the whole program: 250 such trees would take 40 GB."""
+    run(BATCH + """
+spec = [("blend_union", 8.0) if t[0] in scenes.SET_OPS else t for t in scenes.random_csg_spec(1, 600)]
+p = scenes.build_sdf(spec).program()
+tiles, blocks = units(250)
+b, st, calls = batch(250, 250, p, False)
+by_tiles = (st["blocks"] - 250 * blocks) / (tiles - blocks)
+assert 0 < by_tiles < 140, by_tiles
+""")
