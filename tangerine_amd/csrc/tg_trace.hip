@@ -188,18 +188,26 @@ uint32_t first_entries(uint64_t rays, size_t entries)
 	return uint32_t(double(entries) * std::min(6.0, std::max(1.0, std::sqrt(waves) / 24.0)));
 }
 
-// Whether the long marches of a frame go on in groups of lanes.  (Passes / groups, ms,
-// by the share of the entries that cells keep.  1 (an ellipsoid): 64 primitives 640x360
-// 8.7 / 7.9, 960x540 9.3 / 11.1, 1920x1080 12.8 / 21.3, 256 primitives 38.7 / 26.3, 41.3 / 48.3,
-// 60.1 / 125.  0.66 to 0.8 (blends of 2 units): 256 primitives 42.9 / 31.4, 47.3 / 56.8, 76.4 /
-// 141.  0.44 (1 unit): 1280x720 28.4 / 25.1, 1920x1080 33.4 / 39.2.  0.32 (0.5): 1920x1080 22.5 /
-// 18.9.  0.05: 9.2 / 6.5.  Short programs: 8 primitives 320x180 1.14 / 0.79, 1920x1080 1.20 /
-// 1.07, 4 primitives 0.82 / 0.66, 0.98 / 1.05, 3840x2160 1.40 / 1.78, 2 primitives 0.73 / 0.79,
-// 0.84 / 0.88, 1.01 / 1.29.)
+// Whether the long marches of a frame go on in groups of lanes, by the share of the
+// entries that cells keep.  A group's step costs the height of the cell's program where
+// a wave's costs its length, but the wave's serves up to 64 rays: groups win while rays
+// are few or the programs short, and where cells keep nearly all, scenes differ by more
+// than any line (1142 frames of 2 to 512 primitives, 64x36 to 3840x2160: random trees
+// at most 1.2 times the better way's time, 0.5 % on average; the passes are never slower
+// than those of 32 + 224 steps were, and the line gives the others to them).
+// (Passes / groups, ms.  1 (an ellipsoid): 64 primitives 320x180 8.76 / 5.55, 640x360
+// 8.77 / 7.90, 1280x720 9.83 / 14.2; 256 primitives 37.3 / 11.3, 38.4 / 28.2, 45.7 / 65.8.
+// 1 (blends of 4 to 8 units): 12 primitives 320x180 2.82 / 1.95, 640x360 2.76 / 3.42; 24
+// 400x225 0.60 / 1.16; 256 320x180 12.2 / 9.5, 640x360 12.0 / 27.9.  0.66 (2 units): 256
+// primitives 500x281 44.2 / 25.0, 960x540 47.8 / 57.8.  0.44 (1 unit): 960x540 24.7 / 22.8,
+// 1280x720 28.8 / 26.0, 1920x1080 33.4 / 40.1.  0.32 (0.5): 1280x720 20.7 / 14.4, 1920x1080
+// 22.3 / 18.9, 3840x2160 42.0 / 41.1.  0.05: 1920x1080 9.23 / 6.69.  Short programs: 8
+// primitives, 0.12, 200x112 0.93 / 0.46, 1920x1080 1.23 / 1.12, 3840x2160 1.64 / 1.87; 4,
+// 0.36, 400x225 0.86 / 0.72, 1920x1080 1.02 / 1.06; 3, 0.25, 640x360 0.67 / 0.50; 2, 0.33,
+// 200x112 0.60 / 0.42, 1920x1080 0.85 / 0.88; 1 from 400x225 on 0.48 / 0.50.)
 bool frame_groups(uint64_t rays, size_t entries, float kept)
 {
-	const double share = entries < 12 ? 1.0 : double(kept);
-	return entries >= 7 && double(rays) * std::pow(share, 1.75) <= 240.0e3;
+	return entries >= 3 && double(rays) * std::pow(double(kept), 2.4) <= 80.0e3;
 }
 
 void base_args(TraceArgs& ta, const tg_program* p)

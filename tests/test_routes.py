@@ -20,12 +20,13 @@ def tree(kind, n):
 
 @pytest.mark.parametrize("kind,prims,groups", [
     ("ellipsoid", 64, (True, False)), ("ellipsoid", 256, (True, False)), ("2", 64, (True, False)), ("2", 256, (True, False)),
-    ("8", 256, (True, False)), ("random", 2, (False, False)), ("random", 4, (True, False)), ("random", 8, (True, True)),
+    ("8", 256, (True, False)), ("random", 1, (False, False)), ("random", 2, (True, False)), ("random", 3, (True, False)), ("random", 4, (True, False)), ("random", 8, (True, True)),
     ("0.1", 256, (True, True)), ("random", 16, (True, True)), ("random", 64, (True, True)),
     ("random", 256, (True, True)), ("random", 2048, (True, True))])
 def test_frames(kind, prims, groups):
-    """Small frames go on in groups of lanes whatever the program (their waves do not
-    fill the GPU), large ones only where cells prune; unpruned renders never."""
+    """Small frames go on in groups of lanes whatever the program of 2 primitives or
+    more (their waves do not fill the GPU), large ones only where cells prune; unpruned
+    renders never."""
     run(TREES + f"""
 p = tree({kind!r}, {prims})
 tr = trace.Tracer()
