@@ -1615,12 +1615,16 @@ namespace {
 // 250 / 245, two steps 16 Mi 937 / 1087, 54 Mi 935 / 733, 2 Gi 2404 / 388.)
 //
 // That is where tiles keep a twentieth of the program.  Where they keep more, the
-// selection saves less, and a refinement step, a wave's latency either way, costs
-// more through a tile's program (fewer points to a wave) from a seventh on.  (No steps
-// / two, us, 120^3 cells, whole / tiles: 256 primitives, 0.23 kept 793 / 470, 1645 / 1632;
-// 0.32 775 / 479, 1637 / 1844; 0.66 779 / 807, 1505 / 2249; 64 primitives, 0.16 kept 261 / 226,
-// 424 / 483; 0.8 259 / 299, 424 / 633; 16 primitives, two steps, 0.07 kept 165 / 158, 0.19 172 / 182.
-// 200^3 cells of 256 primitives, 0.44 kept: 3110 / 1188, 4537 / 2372; 0.66 3115 / 2344, 4120 / 4787.)
+// selection saves less, the passes cost more, and a refinement step, a wave's latency
+// either way while the cells are few, costs more through a tile's program (fewer points
+// to a wave).  The line is fitted to 1408 calls of 8 to 512 primitives, 0.02 to 1 kept,
+// 60^3 to 256^3 cells, up to six steps: 22 of the 935 it sends through tiles were more than
+// 3 % faster whole (at most 1.27 times).  (Whole / tiles, us.  256 primitives, 120^3
+// cells, no steps and two: 0.23 kept 793 / 470, 1645 / 1632; 0.32 775 / 479, 1637 / 1844;
+// 0.66 779 / 807, 1505 / 2249; 200^3 cells, 0.44 kept 3110 / 1188, 4537 / 2372, 0.66 3115 /
+// 2344, 4120 / 4787.  64 primitives, 120^3: 0.16 kept 261 / 226, 424 / 483; 0.8 259 / 299,
+// 424 / 633.  28 primitives, 0.19 kept, six steps, 120^3 359 / 212, 160^3 461 / 346.  10
+// primitives, 0.12 to 0.2 kept, six steps, 160^3 241 / 196 to 254 / 182.)
 constexpr uint64_t kCloudEntryCells = 120ull << 20, kCloudEntryTiles = 600ull << 20;
 
 bool cloud_tiles(const tg_program* p, const CloudArgs& a)
@@ -1628,10 +1632,10 @@ bool cloud_tiles(const tg_program* p, const CloudArgs& a)
 	const uint64_t t = kTile, entries = p->decoded.entries.size();
 	const uint64_t tiles = (a.ix + t - 1) / t * ((a.iy + t - 1) / t) * ((a.iz + t - 1) / t);
 	if (a.cells * entries * (1 + uint64_t(a.iterations)) < kCloudEntryCells || tiles * entries > kCloudEntryTiles) return false;
-	const double e = double(entries), kept = p->kept;
-	const double selection = 0.84e-6 * double(a.cells) * e * (1.0 - 1.3 * kept);  // us saved
-	const double step = e * std::min(std::max(12.0 * (kept - 0.13), -0.42), 0.5);  // us lost
-	return selection - double(a.iterations) * step > 55.0 + 0.1 * e && treelet_prunable(p, tiles);
+	const double e = double(entries), kept = p->kept, cells = 1e-6 * double(a.cells);
+	const double selection = 0.6 * cells * e * (1.0 - 0.88 * kept);  // us saved
+	const double step = e * std::min(std::max(4.5 * (kept * std::sqrt(4.1 / cells) - 0.33), -0.48), 1.8);  // us lost
+	return selection - double(a.iterations) * step > 58.0 + (0.015 + 0.8 * kept) * e && treelet_prunable(p, tiles);
 }
 
 // The tiles' programs, valid within 4 cell diagonals of a tile's centre: its

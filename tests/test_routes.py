@@ -85,6 +85,7 @@ for (n, steps), want in {casts!r}.items():
 
 @pytest.mark.parametrize("kind,prims,clouds", [
     ("random", 256, {(32, 0): False, (120, 0): True, (120, 2): True}), ("random", 16, {(200, 0): True, (120, 2): True}),
+    ("random", 10, {(120, 0): False, (160, 6): True}), ("random", 28, {(120, 0): False, (120, 6): True}),
     ("0.5", 256, {(120, 0): True, (120, 2): False, (200, 2): True}), ("8", 64, {(120, 0): False, (120, 2): False}),
     ("8", 256, {(120, 0): False, (200, 2): False}), ("ellipsoid", 256, {(120, 0): False})])
 def test_point_clouds(kind, prims, clouds):
